@@ -233,6 +233,23 @@ int pp_spline_eval(const pp_spline* s, const double* pts, int64_t m, int32_t str
 /* Fused multi-step push: Pusher.track_batch step loop (pusher.py:966-990) /
    push_batch (pusher.py:699-801) when nsteps == 1. */
 int pp_push(const pp_push_args* args, pp_stream s);
+/* pp_push through fields that are sums of terms, E (or B) = sum_k weight_k term_k accumulated from zero in the
+   given order: CompositeField.__call__ (field.py:621-645) inside the step loop, so a track through an external
+   map plus a self-field map on another grid needs no field arrays.  terms: host array of 1..PP_MAX_SUM_TERMS
+   entries; the entries of each field keep their order.  A field that is not a sum is one entry flagged
+   PP_SUM_PLAIN (its value is taken as it is); a field without entries is zero.  PP_SUM_SAME_CELL: a MAP entry
+   on the same grid (nodes and periodicity) as the MAP entry before it, whose cell lookup it shares.  The args'
+   efield and bfield are not read; ARRAY terms and an alive mask are refused; the fast precisions take the
+   single-gather algorithms. */
+#define PP_MAX_SUM_TERMS 6
+enum pp_sum_flags { PP_SUM_TO_B = 1, PP_SUM_PLAIN = 2, PP_SUM_SAME_CELL = 4 };
+typedef struct pp_sum_term {
+    pp_field field;
+    double weight;           /* CompositeField.weights[k] */
+    int32_t flags;           /* enum pp_sum_flags */
+    int32_t _pad;
+} pp_sum_term;
+int pp_push_sum(const pp_push_args* args, const pp_sum_term* terms, int32_t nterms, pp_stream s);
 
 /* Per-step kernels with fields supplied per particle (the reference's Numba batch
    kernels).  v, E, B, r and outputs: device float64 (M, 3). */

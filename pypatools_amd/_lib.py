@@ -52,6 +52,10 @@ class PPPushArgs(ctypes.Structure):
     ]
 
 
+class PPSumTerm(ctypes.Structure):
+    _fields_ = [("field", PPField), ("weight", ctypes.c_double), ("flags", c_int32), ("_pad", c_int32)]
+
+
 class PPBunch(ctypes.Structure):
     _fields_ = [
         ("offset", c_int64), ("count", c_int64), ("algorithm", c_int32), ("nsteps", c_int32),
@@ -60,6 +64,8 @@ class PPBunch(ctypes.Structure):
     ]
 
 
+MAX_SUM_TERMS = 6                                # include/pypat_hip.h PP_MAX_SUM_TERMS
+SUM_TO_B, SUM_PLAIN, SUM_SAME_CELL = 1, 2, 4     # pp_sum_flags
 SPLINE_NEAREST_MODE, SPLINE_RGI = 1, 2          # pp_spline_flags
 TILES_ALL, TILES_SINGLE_GATHER, TILES_RK4 = 0, 1, 2   # pp_tile_class
 RK4_ALGS = ("rk4", "rk4_rel")
@@ -132,6 +138,7 @@ SIGNATURES = {
     "pp_field_eval": (c_int32, [ctypes.POINTER(PPField), c_int32, c_void_p, c_int64, ctypes.c_double, c_void_p,
                                 c_void_p]),
     "pp_push": (c_int32, [ctypes.POINTER(PPPushArgs), c_void_p]),
+    "pp_push_sum": (c_int32, [ctypes.POINTER(PPPushArgs), ctypes.POINTER(PPSumTerm), c_int32, c_void_p]),
     "pp_boris_push_batch": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, ctypes.c_double, ctypes.c_double,
                                       c_void_p, c_void_p]),
     "pp_vay_push_batch": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, ctypes.c_double, ctypes.c_double,

@@ -366,6 +366,33 @@ __global__ void __launch_bounds__(256) k_push_mixed(const PushParams p) {
     }
 }
 
+// Sums of field terms (SumFE64): every term is evaluated in FP32, weighted and accumulated in FP64, and the
+// sum is rounded to FP32 once, as when the terms come through (n, 3) float64 arrays.
+struct SumFE32 {
+    const PushParams& p;
+    const SumParams& t;
+    DEV void operator()(int64_t, double x, double y, double z, int64_t gs, int stage, f3& E, f3& B) const {
+        d3 e = mk3(0.0, 0.0, 0.0), b = e;
+        for (int k = 0; k < t.nterms; ++k) {
+            const FieldDev& f = t.f[k];
+            f3 raw = mkf(0.f, 0.f, 0.f);
+            if (f.kind == PP_FIELD_MAP) raw = map_components32(f, x, y, z);
+            const d3 v = tod(finish_term32(f, raw, f.rf != PP_RF_NONE ? (float)rf_factor(p, gs, stage, f.rf) : 1.f));
+            d3& total = (t.flags[k] & PP_SUM_TO_B) ? b : e;
+            total = (t.flags[k] & PP_SUM_PLAIN) ? v : SumFE64::add_weighted(total, t.weight[k], v);
+        }
+        E = tof(e);
+        B = tof(b);
+    }
+};
+
+template <int ALG>
+__global__ void __launch_bounds__(256) k_push_mixed_sum(const PushParams p, const SumParams t) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= p.n) return;
+    push_mixed_particle<ALG, false>(p, i, SumFE32{p, t});
+}
+
 __global__ void __launch_bounds__(256) k_field_eval32(const FieldDev f, const double* __restrict__ pts, int64_t m,
                                                        double rfv, double* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1185,6 +1212,29 @@ hipError_t launch_push(int alg, int prec, const PushParams& p, int block, hipStr
             PP_FAST_CASES(k_push_mixed, false, kFieldsGeneral)
         }
     }
+    return hipGetLastError();
+}
+
+// the single-gather algorithms (RK4 through summed fields keeps its FP64 stage kernels in the fast precisions)
+hipError_t launch_push_sum(int alg, int prec, const PushParams& p, const SumParams& t, int block, hipStream_t s) {
+    if (block <= 0) block = 256;
+    const dim3 g(grid_for(p.n, block)), b(block);
+#define PP_SUM_CASE(A)                                                                                  \
+    case A:                                                                                             \
+        if (prec == PP_PREC_FP64_FAST) hipLaunchKernelGGL(k_push64_sum<A>, g, b, 0, s, p, t);          \
+        else hipLaunchKernelGGL(k_push_mixed_sum<A>, g, b, 0, s, p, t);                                \
+        break;
+    switch (alg) {
+        PP_SUM_CASE(PP_ALG_LEAPFROG)
+        PP_SUM_CASE(PP_ALG_BORIS)
+        PP_SUM_CASE(PP_ALG_YOSHIDA)
+        PP_SUM_CASE(PP_ALG_VAY_REL)
+        PP_SUM_CASE(PP_ALG_YOSHIDA_REL)
+        PP_SUM_CASE(PP_ALG_BORIS_REL)
+        PP_SUM_CASE(PP_ALG_VAY)
+        default: return hipErrorInvalidValue;
+    }
+#undef PP_SUM_CASE
     return hipGetLastError();
 }
 

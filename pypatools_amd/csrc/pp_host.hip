@@ -590,7 +590,8 @@ int pp_field_eval(const pp_field* field, int32_t precision, const double* pts, i
     return PP_OK;
 }
 
-static int push_impl(const pp_push_args* a, const pp_mesh* mesh, pp_stream s) {
+// terms: the fields of pp_push_sum (efield and bfield of the args are then not read), or null
+static int push_impl(const pp_push_args* a, const pp_mesh* mesh, const pp_sum_term* terms, int32_t nterms, pp_stream s) {
     int rc = ensure_init();
     if (rc) return rc;
     if (!a) return fail(PP_ERR_INVALID, "null args");
@@ -624,9 +625,38 @@ static int push_impl(const pp_push_args* a, const pp_mesh* mesh, pp_stream s) {
                     (long long)a->n);
     PushParams p;
     memset(&p, 0, sizeof(p));
-    if ((rc = make_field(a->efield, a->precision, p.E))) return rc;
-    if ((rc = make_field(a->bfield, a->precision, p.B))) return rc;
-    const bool rf = p.E.rf != PP_RF_NONE || p.B.rf != PP_RF_NONE;
+    SumParams sum;
+    bool rf = false;
+    if (terms) {
+        memset(&sum, 0, sizeof(sum));
+        sum.nterms = nterms;
+        for (int32_t k = 0; k < nterms; ++k) {
+            if (terms[k].field.kind == PP_FIELD_ARRAY) return fail(PP_ERR_INVALID, "term %d is an array field", k);
+            if (terms[k].flags & ~(PP_SUM_TO_B | PP_SUM_PLAIN | PP_SUM_SAME_CELL))
+                return fail(PP_ERR_INVALID, "term %d: unknown flags", k);
+            if ((rc = make_field(terms[k].field, a->precision, sum.f[k]))) return rc;
+            sum.flags[k] = terms[k].flags;
+            sum.weight[k] = terms[k].weight;
+            rf = rf || sum.f[k].rf != PP_RF_NONE;
+            if (terms[k].flags & PP_SUM_SAME_CELL) {
+                // the shared cell lookup needs a map entry before this one with the same grid
+                const MapDesc* m = nullptr;
+                for (int32_t q = 0; q < k; ++q)
+                    if (sum.f[q].kind == PP_FIELD_MAP) m = &sum.f[q].map;
+                if (!m || sum.f[k].kind != PP_FIELD_MAP || memcmp(m->n, sum.f[k].map.n, sizeof(m->n)) ||
+                    memcmp(m->lo, sum.f[k].map.lo, sizeof(m->lo)) || memcmp(m->hi, sum.f[k].map.hi, sizeof(m->hi)) ||
+                    m->periodic != sum.f[k].map.periodic)
+                    return fail(PP_ERR_INVALID, "term %d does not share the grid of a map before it", k);
+            }
+        }
+        if (a->alive) return fail(PP_ERR_INVALID, "summed fields take no alive mask");
+        if (a->precision != PP_PREC_FP64 && (a->algorithm == PP_ALG_RK4 || a->algorithm == PP_ALG_RK4_REL))
+            return fail(PP_ERR_UNSUPPORTED, "RK4 through summed fields runs in PP_PREC_FP64");
+    } else {
+        if ((rc = make_field(a->efield, a->precision, p.E))) return rc;
+        if ((rc = make_field(a->bfield, a->precision, p.B))) return rc;
+        rf = p.E.rf != PP_RF_NONE || p.B.rf != PP_RF_NONE;
+    }
     if (rf) {
         if (!a->rf_table) return fail(PP_ERR_INVALID, "time-dependent field without an rf table");
         const int64_t last = a->step0 + (a->kick_only ? 0 : a->nsteps - 1);
@@ -635,10 +665,10 @@ static int push_impl(const pp_push_args* a, const pp_mesh* mesh, pp_stream s) {
                         (long long)a->rf_step0, (long long)(a->rf_step0 + a->rf_nsteps), (long long)a->step0,
                         (long long)last);
     }
-    const bool has_array = a->efield.kind == PP_FIELD_ARRAY || a->bfield.kind == PP_FIELD_ARRAY;
+    const bool has_array = !terms && (a->efield.kind == PP_FIELD_ARRAY || a->bfield.kind == PP_FIELD_ARRAY);
     if (has_array && (a->algorithm == PP_ALG_RK4 || a->algorithm == PP_ALG_RK4_REL || (a->nsteps != 1)))
         return fail(PP_ERR_INVALID, "array fields need a single-gather algorithm and nsteps == 1");
-    p.fused = (a->efield.kind == PP_FIELD_MAP && a->bfield.kind == PP_FIELD_MAP && a->efield.map == a->bfield.map) ? 1 : 0;
+    p.fused = (!terms && a->efield.kind == PP_FIELD_MAP && a->bfield.kind == PP_FIELD_MAP && a->efield.map == a->bfield.map) ? 1 : 0;
     p.n = a->n;
     p.x = a->x; p.y = a->y; p.z = a->z;
     p.vx = a->vx; p.vy = a->vy; p.vz = a->vz;
@@ -667,7 +697,11 @@ static int push_impl(const pp_push_args* a, const pp_mesh* mesh, pp_stream s) {
     if (mesh) p.mesh = pp_collide::device_view(mesh);   // null for an empty mesh: nothing to hit
     HotParams hp;
     hipError_t e;
-    if (hot_eligible(a, p, hp))
+    if (terms)
+        e = a->precision == PP_PREC_FP64
+                ? pp_strict::launch_push_sum(a->algorithm, p, sum, a->block_size, stream_of(s))
+                : pp_fast::launch_push_sum(a->algorithm, a->precision, p, sum, a->block_size, stream_of(s));
+    else if (hot_eligible(a, p, hp))
         e = pp_fast::launch_hot(a->algorithm, a->precision, p.E.map.periodic != 0, hp, a->block_size, stream_of(s));
     else if (a->precision == PP_PREC_FP64)
         e = pp_strict::launch_push(a->algorithm, p, a->block_size, stream_of(s));
@@ -677,11 +711,17 @@ static int push_impl(const pp_push_args* a, const pp_mesh* mesh, pp_stream s) {
     return PP_OK;
 }
 
-int pp_push(const pp_push_args* a, pp_stream s) { return push_impl(a, nullptr, s); }
+int pp_push(const pp_push_args* a, pp_stream s) { return push_impl(a, nullptr, nullptr, 0, s); }
+
+int pp_push_sum(const pp_push_args* a, const pp_sum_term* terms, int32_t nterms, pp_stream s) {
+    if (!terms || nterms < 1 || nterms > PP_MAX_SUM_TERMS)
+        return fail(PP_ERR_INVALID, "summed fields take 1 to %d terms", PP_MAX_SUM_TERMS);
+    return push_impl(a, nullptr, terms, nterms, s);
+}
 
 int pp_push_lossy(const pp_push_args* a, const pp_mesh* mesh, pp_stream s) {
     if (!mesh) return fail(PP_ERR_INVALID, "null mesh");
-    return push_impl(a, mesh, s);
+    return push_impl(a, mesh, nullptr, 0, s);
 }
 
 int pp_batch_tiles(const pp_bunch* bunches, int32_t nbunch, int32_t tile, int32_t* tile_bunch, int64_t* tile_start,

@@ -66,6 +66,15 @@ struct PushParams {
     double yc[3], yd[3];    // Yoshida coefficients, pusher.py:176-181
 };
 
+// Terms of summed fields (pp_push_sum), in evaluation order.
+struct SumParams {
+    int32_t nterms;
+    int32_t flags[PP_MAX_SUM_TERMS];    // pp_sum_flags
+    double weight[PP_MAX_SUM_TERMS];
+    FieldDev f[PP_MAX_SUM_TERMS];
+};
+static_assert(sizeof(PushParams) + sizeof(SumParams) <= 4096, "kernel arguments of the summed-field push");
+
 // Hot path: E and B from one uniform 3-D map (components 0..2 = E, 3..5 = B),
 // no RF / offset terms.  Compact, so the step loop keeps it in SGPRs.
 struct HotMap {
@@ -135,6 +144,7 @@ struct pp_map {
 
 namespace pp_strict {
 hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s);
+hipError_t launch_push_sum(int alg, const PushParams& p, const SumParams& t, int block, hipStream_t s);
 hipError_t launch_field_eval(const FieldDev& f, const double* pts, int64_t m, double rf, double* out,
                              hipStream_t s);
 struct BatchArgs {
@@ -157,6 +167,7 @@ hipError_t launch_build_coef(const MapDesc& d, double* c64, float* c32, hipStrea
 
 namespace pp_fast {
 hipError_t launch_push(int alg, int prec, const PushParams& p, int block, hipStream_t s);
+hipError_t launch_push_sum(int alg, int prec, const PushParams& p, const SumParams& t, int block, hipStream_t s);
 hipError_t launch_hot(int alg, int prec, bool periodic, const HotParams& p, int block, hipStream_t s);
 hipError_t launch_batched(int prec, bool periodic, int tile_class, const BatchParams& p, int block, hipStream_t s);
 hipError_t launch_field_eval(const FieldDev& f, int prec, const double* pts, int64_t m, double rf, double* out,

@@ -165,6 +165,24 @@ hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t launch_push_sum(int alg, const PushParams& p, const SumParams& t, int block, hipStream_t s) {
+    if (block <= 0) block = 256;
+    const dim3 g(grid_for(p.n, block)), b(block);
+    switch (alg) {
+        case PP_ALG_LEAPFROG: hipLaunchKernelGGL(k_push64_sum<PP_ALG_LEAPFROG>, g, b, 0, s, p, t); break;
+        case PP_ALG_BORIS: hipLaunchKernelGGL(k_push64_sum<PP_ALG_BORIS>, g, b, 0, s, p, t); break;
+        case PP_ALG_RK4: hipLaunchKernelGGL(k_push64_sum<PP_ALG_RK4>, g, b, 0, s, p, t); break;
+        case PP_ALG_YOSHIDA: hipLaunchKernelGGL(k_push64_sum<PP_ALG_YOSHIDA>, g, b, 0, s, p, t); break;
+        case PP_ALG_VAY_REL: hipLaunchKernelGGL(k_push64_sum<PP_ALG_VAY_REL>, g, b, 0, s, p, t); break;
+        case PP_ALG_RK4_REL: hipLaunchKernelGGL(k_push64_sum<PP_ALG_RK4_REL>, g, b, 0, s, p, t); break;
+        case PP_ALG_YOSHIDA_REL: hipLaunchKernelGGL(k_push64_sum<PP_ALG_YOSHIDA_REL>, g, b, 0, s, p, t); break;
+        case PP_ALG_BORIS_REL: hipLaunchKernelGGL(k_push64_sum<PP_ALG_BORIS_REL>, g, b, 0, s, p, t); break;
+        case PP_ALG_VAY: hipLaunchKernelGGL(k_push64_sum<PP_ALG_VAY>, g, b, 0, s, p, t); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_field_eval(const FieldDev& f, const double* pts, int64_t m, double rf, double* out, hipStream_t s) {
     hipLaunchKernelGGL(k_field_eval64, dim3(grid_for(m, 256)), dim3(256), 0, s, f, pts, m, rf, out);
     return hipGetLastError();

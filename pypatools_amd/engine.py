@@ -20,7 +20,8 @@ import numpy as np
 
 from . import _lib
 from .device import DeviceArray
-from .field import Field, RFField, ScaledField, compile_term, evaluate_on_device, is_time_dependent
+from .field import (CompositeField, Field, RFField, ScaledField, compile_sum, compile_term, evaluate_on_device,
+                    is_time_dependent, rf_source)
 from .interpolators import DeviceFieldMap
 
 REFERENCE_ALGORITHMS = ["leapfrog", "boris", "rk4", "yoshida", "vay_rel", "rk4_rel", "yoshida_rel"]
@@ -111,7 +112,7 @@ class ParticleState:
         a.x, a.y, a.z = self.x.ptr, self.y.ptr, self.z.ptr
         a.vx, a.vy, a.vz = self.vx.ptr, self.vy.ptr, self.vz.ptr
         if fp is not None:
-            a.efield, a.bfield = fp.tE, fp.tB
+            a.efield, a.bfield = fp.sort_terms()
         return a
 
     def sort(self, fp, refine_axis=2, refine_bits=0):
@@ -214,7 +215,27 @@ class FieldPair:
                 self.tE.comp0 = 0
                 self.tB.map = fm.handle
                 self.tB.comp0 = 3
+        # fields that are sums of direct terms: pp_push_sum evaluates them inside the step loop
+        self.sum = None if self.direct else compile_sum(efield, bfield)
 
+    def fused(self, algorithm, precision):
+        """True if the step loop runs inside the push kernels (sums: RK4 in the strict precision only)."""
+        return self.direct or (self.sum is not None and (precision == "fp64" or algorithm not in RK4_FAMILY))
+
+    def sort_terms(self):
+        """(efield, bfield) terms whose map the cell sort reads."""
+        if self.sum is None:
+            return self.tE, self.tB
+        return self.sum[2] or _lib.PPField(), _lib.PPField()
+
+    def rf_sources(self):
+        fields = [g for f in (self.efield, self.bfield)
+                  for g in (_sum_members(f) if self.sum is not None else [f])]
+        return {rf_source(g) for g in fields} - {None}
+
+
+def _sum_members(f):
+    return [h for g in f.fields for h in _sum_members(g)] if isinstance(f, CompositeField) else [f]
 
 
 def build_rf_table(field, t0, dt, n_rows):
@@ -232,12 +253,6 @@ def build_rf_table(field, t0, dt, n_rows):
             tab[n, s, 0] = np.cos(arg)
             tab[n, s, 1] = np.sin(arg)
     return tab
-
-
-def _rf_source(f):
-    while isinstance(f, ScaledField):
-        f = f.field
-    return f if isinstance(f, RFField) else None
 
 
 class Tracker:
@@ -273,8 +288,10 @@ class Tracker:
         a.q_over_m = self.qm
         a.nsteps = int(nsteps)
         a.step0 = int(step0)
-        a.efield = tE if tE is not None else fp.tE
-        a.bfield = tB if tB is not None else fp.tB
+        if tE is not None:
+            a.efield, a.bfield = tE, tB
+        elif fp.sum is None:
+            a.efield, a.bfield = fp.tE, fp.tB
         if rf is not None:
             a.rf_table, a.rf_step0, a.rf_nsteps = rf[0].ptr, rf[1], rf[2]
         if hist is not None:
@@ -283,14 +300,17 @@ class Tracker:
         a.block_size = self.block_size
         return a
 
-    def _launch(self, args, stream=None):
-        _lib.call("pp_push", args, stream)
+    def _launch(self, args, stream=None, fp=None):
+        if fp is not None and fp.sum is not None:
+            _lib.call("pp_push_sum", args, fp.sum[0], fp.sum[1], stream)
+        else:
+            _lib.call("pp_push", args, stream)
 
     def _rf(self, fp, t0, dt, nsteps):
         """Device rf table covering steps 0..nsteps (both fields share it: cos and sin columns)."""
         if not fp.time_dependent:
             return None
-        srcs = {_rf_source(fp.efield), _rf_source(fp.bfield)} - {None}
+        srcs = fp.rf_sources()
         omegas = {(s.omega, s.phase) for s in srcs}
         if len(omegas) != 1:
             raise NotImplementedError("E and B must share one (omega, phase) in a fused push")
@@ -327,22 +347,23 @@ class Tracker:
         rh.fill(fill)
         vh.fill(fill)
         hist = (rh, vh, rec, n_records)
-        rf = self._rf(fp, t0, dt, nsteps) if fp.direct else None
+        fused = fp.fused(alg, self.precision) if elec is None else fp.direct
+        rf = self._rf(fp, t0, dt, nsteps) if fused else None
         ustate = alg in U_STATE
         if ustate:
             st.v_to_u()
         if alg in STAGGERED:
-            self._kick(st, fp, -0.5 * dt, 0, rf, t0, dt)
+            self._kick(st, fp, fused, -0.5 * dt, 0, rf, t0, dt)
         # record 0
         st.positions_aos(_row(rh, 0, M))
         self._velocity_record(st, _row(vh, 0, M), ustate)
-        if fp.direct and elec is None:
+        if fused and elec is None:
             self._fused_loop(st, fp, nsteps, dt, 0, rf, hist, dtp, verbose)
             st.unsort()
         else:
             self._slow_loop(st, fp, nsteps, dt, t0, rf, hist, elec, active, dtp, verbose)
         if alg in STAGGERED:
-            self._kick(st, fp, 0.5 * dt, nsteps, rf, t0, dt)
+            self._kick(st, fp, fused, 0.5 * dt, nsteps, rf, t0, dt)
             vfin = DeviceArray((M, 3))
             self._velocity_record(st, vfin, ustate)
         r_hist = rh.to_host()
@@ -362,7 +383,7 @@ class Tracker:
         return r_hist, v_hist, active
 
     def _uses_sort(self, st, fp, dtp):
-        maps = fp.tE.kind == _lib.FIELD_MAP or fp.tB.kind == _lib.FIELD_MAP
+        maps = any(t.kind == _lib.FIELD_MAP for t in fp.sort_terms())
         return self.sort_every > 0 and maps and st.n >= SORT_MIN_PARTICLES and dtp is None
 
     def _fused_loop(self, st, fp, nsteps, dt, step0, rf, hist, dtp, verbose=False, steps_per_launch=None,
@@ -385,9 +406,9 @@ class Tracker:
                 _progress(step, end)
             args = self._args(st, fp, dt, k, step, rf=rf, hist=hist, dt_pp=dtp)
             if timer is not None:
-                timer(lambda: self._launch(args))
+                timer(lambda: self._launch(args, fp=fp))
             else:
-                self._launch(args)
+                self._launch(args, fp=fp)
             step += k
             if sort:
                 since += k
@@ -415,11 +436,11 @@ class Tracker:
         ustate = self.algorithm in U_STATE
         if ustate:
             st.v_to_u()
-        if self.algorithm in RK4_FAMILY and not fp.direct:
-            self._rk4_stage_loop(st, fp, 1, dt, t, None, dtp, False)
-        elif fp.direct:
+        if fp.fused(self.algorithm, self.precision):
             rf = self._rf(fp, t, dt, 1)
-            self._launch(self._args(st, fp, dt, 1, 0, rf=rf, dt_pp=dtp))
+            self._launch(self._args(st, fp, dt, 1, 0, rf=rf, dt_pp=dtp), fp=fp)
+        elif self.algorithm in RK4_FAMILY:
+            self._rk4_stage_loop(st, fp, 1, dt, t, None, dtp, False)
         else:
             tE, tB = self._array_terms(st, fp, t)
             self._launch(self._args(st, fp, dt, 1, 0, tE=tE, tB=tB, dt_pp=dtp))
@@ -437,9 +458,9 @@ class Tracker:
         _lib.call("pp_soa_to_aos", tmp[0].ptr, tmp[1].ptr, tmp[2].ptr, st.n, out_aos.ptr, None)
         return out_aos
 
-    def _kick(self, st, fp, dt_kick, step, rf, t0, dt):
-        if fp.direct:
-            self._launch(self._args(st, fp, dt_kick, 1, step, rf=rf, kick=True))
+    def _kick(self, st, fp, fused, dt_kick, step, rf, t0, dt):
+        if fused:
+            self._launch(self._args(st, fp, dt_kick, 1, step, rf=rf, kick=True), fp=fp)
             return
         t = t0 + step * dt
         tE, tB = self._array_terms(st, fp, t)

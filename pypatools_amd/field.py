@@ -421,6 +421,83 @@ def compile_term(f):
     return None
 
 
+def compile_sum(efield, bfield):
+    """(terms, count, primary) of a pair of fields of which at least one is a sum of direct terms (pp_push_sum:
+    the terms in evaluation order as an array, and the first map term, for the cell sort), or None.
+
+    CompositeField accumulates ``total += w * F`` from zero (field.py:621-645).  A sum whose first member is
+    itself a sum of weight 1 accumulates on (0 + 1 * s is s bit for bit: s = 0 + ... is never -0), so
+    ``E1 + E2 + E3`` is one list.
+    """
+    def entries(f):
+        if not isinstance(f, CompositeField):
+            return [(f, 1.0, True)]
+        if f.n_fields == 0 or len(f.fields) != len(f.weights):
+            return None
+        out = []
+        for k, (g, w) in enumerate(zip(f.fields, f.weights)):
+            if k == 0 and w == 1.0 and isinstance(g, CompositeField):
+                inner = entries(g)
+                if inner is None:
+                    return None
+                out += inner
+            else:
+                out.append((g, float(w), False))
+        return out
+
+    if not (isinstance(efield, CompositeField) or isinstance(bfield, CompositeField)):
+        return None
+    listed = []
+    for f, target in ((efield, 0), (bfield, _lib.SUM_TO_B)):
+        es = entries(f)
+        if es is None:
+            return None
+        for g, w, plain in es:
+            t = compile_term(g)
+            if t is None:
+                return None
+            listed.append((t, w, target | (_lib.SUM_PLAIN if plain else 0), g))
+    if len(listed) > _lib.MAX_SUM_TERMS:
+        return None
+    rf = {(s.omega, s.phase) for s in (rf_source(e[3]) for e in listed) if s is not None}
+    if len(rf) > 1:
+        return None
+
+    def grid(entry):
+        base = entry[3]
+        while isinstance(base, (ScaledField, RFField)):
+            base = base.field
+        return base._grid_source() if entry[0].kind == _lib.FIELD_MAP else None
+
+    def same(a, b):
+        return (a is not None and b is not None and a[2] == b[2] and len(a[0]) == len(b[0])
+                and all(np.array_equal(u, v) for u, v in zip(a[0], b[0])))
+
+    # B's first term follows the first E term on its grid: both then share one cell lookup
+    nb = sum(1 for e in listed if e[2] & _lib.SUM_TO_B)
+    es, bs = listed[:len(listed) - nb], listed[len(listed) - nb:]
+    g0 = grid(bs[0])
+    at = next((k for k, e in enumerate(es) if same(grid(e), g0)), None)
+    order = es + bs if at is None else es[:at + 1] + bs[:1] + es[at + 1:] + bs[1:]
+    terms = (_lib.PPSumTerm * len(order))()
+    last, primary = None, None
+    for t, e in zip(terms, order):
+        t.field, t.weight, t.flags = e[0], e[1], e[2]
+        g = grid(e)
+        if g is not None:
+            if same(g, last):
+                t.flags |= _lib.SUM_SAME_CELL
+            last = g
+            primary = primary or e[0]
+    return terms, len(order), primary
+
+
+def rf_source(f):
+    while isinstance(f, ScaledField):
+        f = f.field
+    return f if isinstance(f, RFField) else None
+
+
 def is_time_dependent(f):
     if isinstance(f, RFField):
         return True
