@@ -105,6 +105,31 @@ def test_aimed_segments_over_many_candidate_cells_match_brute_force():
     assert 0.2 < want.mean() < 0.9
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("length", [2.0, 300.0])
+def test_elongated_cells_match_brute_force(axis, length):
+    """Triangles much longer along one axis than across it give candidate cells of that shape (to the limit of
+    256 for the longer pipe, and one cell along a short axis): segments along and across the pipe, from far
+    inside to beyond its wall and its ends, are decided as by brute force."""
+    rng = np.random.default_rng(71)
+    base = TriangleElectrodes.cylinder(1.0, -length / 2, length / 2, n_phi=96, n_z=3)
+    order = np.roll([0, 1, 2], axis + 1)
+    m = TriangleElectrodes(np.ascontiguousarray(base.vertices[:, order]), base.triangles)
+    n = 9000
+    rad = rng.uniform(0.0, 1.05, n)
+    phi = rng.uniform(0, 2 * np.pi, n)
+    r0 = np.column_stack([rad * np.cos(phi), rad * np.sin(phi), rng.uniform(-0.52, 0.52, n) * length])
+    d = 0.05 * rng.standard_normal((n, 3))
+    d[: n // 3, 2] += 0.3 * rng.standard_normal(n // 3) * length / 3       # long steps along the pipe
+    d[n // 3: n // 2, :2] += rng.standard_normal((n // 2 - n // 3, 2))      # long steps across it
+    r1 = (r0 + d)[:, order]
+    r0 = np.ascontiguousarray(r0[:, order])
+    got = m.segment_intersects_surface(r0, r1)["hit_mask"]
+    want = segment_hits(m.vertices, m.triangles, r0, r1)
+    np.testing.assert_array_equal(got, want)
+    assert 0.02 < want.mean() < 0.9
+
+
 @pytest.mark.parametrize("kind", ["box", "cylinder", "soup"])
 def test_short_segments_near_surfaces_match_brute_force(kind):
     """Segments of 1e-7 .. 1e-2 of the mesh size around the surface (the occupancy grid decides most of
