@@ -91,6 +91,7 @@ struct HotMap {
     uint32_t zbias;         // nc2 * floor(2^30 / nc2): makes the z cell index non-negative before the wrap
     uint32_t zmask;         // nc2 - 1 when nc2 is a power of two, else 0
     double zinv;            // 1 / nc2 (exact when nc2 is a power of two)
+    uint64_t stage_exec;    // wavefronts with these lanes active stage cells in LDS: all lanes, or 0 (gather_direct)
 };
 
 // RF factors of the hot kernels: table [step - step0][stage][cos, sin]; e, b = pp_rf_mode of E and B
