@@ -340,18 +340,8 @@ int pp_map_create(const double* values, int32_t ncomp, int32_t nx, int32_t ny, i
     }
     if (periodic) d.inv_nz = 1.0 / (double)d.nc[2];
 
-    // raw table [comp][nx][ny][ngz] (periodic: node nz repeats node 0)
-    const int64_t ngz = d.ng[2];
-    const int64_t per_comp = (int64_t)nx * ny * ngz;
-    std::vector<double> raw((size_t)(per_comp * ncomp));
-    for (int c = 0; c < ncomp; ++c)
-        for (int64_t i = 0; i < nx; ++i)
-            for (int64_t j = 0; j < ny; ++j) {
-                const double* src = values + ((int64_t)c * nx * ny + i * ny + j) * nz;
-                double* dst = raw.data() + c * per_comp + (i * ny + j) * ngz;
-                memcpy(dst, src, sizeof(double) * nz);
-                if (periodic) dst[nz] = src[0];
-            }
+    // the values go up as they are; a kernel lays them out node by node (and repeats node 0 of a periodic axis)
+    const int64_t nodes = (int64_t)nx * ny * d.ng[2];
     void* p;
     hipStream_t s = g_stream;
     for (int a = 0; a < 3; ++a) {
@@ -362,12 +352,17 @@ int pp_map_create(const double* values, int32_t ncomp, int32_t nx, int32_t ny, i
             return fail(PP_ERR_HIP, "map upload failed");
         }
     }
-    if ((rc = map_alloc(m, sizeof(double) * raw.size(), &p))) { pp_map_destroy(m); return rc; }
+    if ((rc = map_alloc(m, sizeof(double) * nodes * ncomp, &p))) { pp_map_destroy(m); return rc; }
     d.raw = static_cast<const double*>(p);
-    if (hipMemcpyAsync(p, raw.data(), sizeof(double) * raw.size(), hipMemcpyHostToDevice, s) != hipSuccess) {
-        pp_map_destroy(m);
-        return fail(PP_ERR_HIP, "map upload failed");
-    }
+    const size_t src_bytes = sizeof(double) * (size_t)nx * ny * nz * ncomp;
+    void* src = nullptr;
+    hipError_t ue = hipMalloc(&src, src_bytes);
+    if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "hipMalloc (field map)"); }
+    ue = hipMemcpyAsync(src, values, src_bytes, hipMemcpyHostToDevice, s);
+    if (ue == hipSuccess) ue = pp_strict::launch_interleave(static_cast<const double*>(src), d, static_cast<double*>(p), s);
+    if (ue == hipSuccess) ue = hipStreamSynchronize(s);
+    (void)hipFree(src);
+    if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "map upload"); }
     const int64_t ncell = (int64_t)d.nc[0] * d.nc[1] * d.nc[2];
     double* c64 = nullptr;
     float* c32 = nullptr;

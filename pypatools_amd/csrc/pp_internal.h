@@ -23,7 +23,7 @@ struct MapDesc {
     double fill;        // value outside the grid
     double inv_nz;      // 1 / nc[2] (periodic maps)
     const double* g[3];
-    const double* raw;      // [comp][nx][ny][ng_z] float64
+    const double* raw;      // [nx][ny][ng_z][comp] float64: a node's components side by side
     const double* coef64;   // [cell][comp][8] float64, cell = (i*nc1 + j)*nc2 + k
     const float* coef32;    // same layout, float32
 };
@@ -163,6 +163,7 @@ hipError_t launch_util(int which, double* a, double* b, double* c, double* aos, 
                        hipStream_t s);
 hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s);
 hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s);
+hipError_t launch_interleave(const double* src, const MapDesc& d, double* raw, hipStream_t s);
 hipError_t launch_build_coef(const MapDesc& d, double* c64, float* c32, hipStream_t s);
 }  // namespace pp_strict
 

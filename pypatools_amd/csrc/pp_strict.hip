@@ -95,6 +95,19 @@ __global__ void __launch_bounds__(256) k_fill(double* p, double v, int64_t n) {
     if (i < n) p[i] = v;
 }
 
+// Node table [node][ncomp] from the components' grids src[comp][nx][ny][nz] (a periodic z axis gets node 0 again
+// as its last).  Writes are contiguous; reads run along ncomp streams.
+__global__ void __launch_bounds__(256) k_interleave(const double* __restrict__ src, const MapDesc d,
+                                                    double* __restrict__ raw) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t ngz = d.ng[2], nodes = (int64_t)d.ng[0] * d.ng[1] * ngz;
+    if (t >= nodes * d.ncomp) return;
+    const int64_t node = t / d.ncomp, comp = t - node * d.ncomp;
+    const int64_t col = node / ngz, k = node - col * ngz;
+    const int64_t nz = d.n[2];
+    raw[t] = src[(comp * d.n[0] * d.n[1] + col) * nz + (k < nz ? k : 0)];
+}
+
 // Per-cell trilinear coefficients of every component from the raw node table.
 __global__ void __launch_bounds__(256) k_build_coef(const MapDesc d, double* __restrict__ c64, float* __restrict__ c32) {
     const int64_t ncell = (int64_t)d.nc[0] * d.nc[1] * d.nc[2];
@@ -109,8 +122,8 @@ __global__ void __launch_bounds__(256) k_build_coef(const MapDesc d, double* __r
     const int i1 = d.n[0] > 1 ? i + 1 : i;
     const int j1 = d.n[1] > 1 ? j + 1 : j;
     const int k1 = d.n[2] > 1 ? k + 1 : k;   // periodic maps carry the wrap node at k = nz
-    const double* v = d.raw + (int64_t)comp * d.ng[0] * ngy * ngz;
-    auto at = [&](int a, int b, int c) { return v[((int64_t)a * ngy + b) * ngz + c]; };
+    const double* v = d.raw + comp;
+    auto at = [&](int a, int b, int c) { return v[(((int64_t)a * ngy + b) * ngz + c) * d.ncomp]; };
     const double c000 = at(i, j, k), c100 = at(i1, j, k), c010 = at(i, j1, k), c110 = at(i1, j1, k);
     const double c001 = at(i, j, k1), c101 = at(i1, j, k1), c011 = at(i, j1, k1), c111 = at(i1, j1, k1);
     double q[8];
@@ -151,7 +164,7 @@ DEV double row_bcast(double v) {
 // What one lane of a row interpolates: its component of the map and that component's chain of factors.
 struct RowFE64 {
     const PushParams& p;
-    const double* __restrict__ values;      // node table of this lane's component
+    const double* __restrict__ values;      // this lane's component of node 0
     double scale1, scale2, offset;
     int32_t has_offset, rf;
     bool second;                            // lanes 8..15: the second position
@@ -162,13 +175,22 @@ struct RowFE64 {
         const bool b = c >= 3;
         const int comp = b ? q.B.comp0 + (c - 3) : q.E.comp0 + c;
         const MapDesc& m = q.E.map;
-        values = m.raw + (int64_t)comp * ((int64_t)m.ng[0] * m.ng[1] * m.ng[2]);
+        values = m.raw + comp;
         scale1 = b ? q.B.scale1 : q.E.scale1;
         const int has2 = b ? q.B.has_scale2 : q.E.has_scale2;
         scale2 = has2 ? (b ? q.B.scale2 : q.E.scale2) : 1.0;        // a product with 1 changes no bit
         has_offset = b ? q.B.has_offset : q.E.has_offset;
         offset = b ? q.B.offset : q.E.offset;
         rf = b ? q.B.rf : q.E.rf;
+    }
+
+    // the corners of cell `base` in lerp8 order: x fastest, then y, then z
+    DEV void corners(int64_t base, double f[8]) const {
+        const MapDesc& m = p.E.map;
+        const double* v = values + 6 * base;
+        const int64_t sz = 6, sy = 6 * (int64_t)m.ng[2], sx = sy * m.ng[1];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) f[k] = v[(k & 1 ? sx : 0) + (k & 2 ? sy : 0) + (k & 4 ? sz : 0)];
     }
 
     // this lane's component at (x, y, z)
@@ -178,25 +200,20 @@ struct RowFE64 {
         if (m.periodic) z = wrap_periodic(z, m.lo[2], m.L, m.inv_d[2] * m.inv_nz);
         const AxisGuess qx = guess_axis(m, 0, x), qy = guess_axis(m, 1, y), qz = guess_axis(m, 2, z);
         StrictCell c;
-        c.sz = 1;
-        c.sy = m.ng[2];
-        c.sx = (int64_t)m.ng[1] * m.ng[2];
         c.base = ((int64_t)qx.i * m.ng[1] + qy.i) * m.ng[2] + qz.i;
-        const double* v = values + c.base;
-        const node_pair a = load_pair(v), b = load_pair(v + c.sy), e = load_pair(v + c.sx), d = load_pair(v + c.sx + c.sy);
-        double raw;
+        double f[8];
+        corners(c.base, f);
         if (guess_is_off(m, 0, qx, x) || guess_is_off(m, 1, qy, y) || guess_is_off(m, 2, qz, z)) {
-
             c = strict_locate_wrapped(m, x, y, z);
-            raw = strict_interp_3d(values + c.base, c);
+            corners(c.base, f);
         } else {
             const double wx = (x - qx.g0) / (qx.g1 - qx.g0), wy = (y - qy.g0) / (qy.g1 - qy.g0),
                          wz = (z - qz.g0) / (qz.g1 - qz.g0);
             c.tx = dmax(0.0, dmin(wx, 1.0));
             c.ty = dmax(0.0, dmin(wy, 1.0));
             c.tz = dmax(0.0, dmin(wz, 1.0));
-            raw = lerp8(a.x, e.x, b.x, d.x, a.y, e.y, b.y, d.y, c);
         }
+        double raw = lerp8(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7], c);
         const bool out = x < m.lo[0] || x > m.hi[0] || y < m.lo[1] || y > m.hi[1] || z < m.lo[2] || z > m.hi[2];
         raw = out ? m.fill : raw;
         double r = scale1 * raw;
@@ -303,16 +320,16 @@ __global__ void __launch_bounds__(64) k_push64_row(const PushParams p) {
 }
 
 // Launches k_push64_row takes: one 3-D six-component map of evenly spaced axes, no alive mask, and few enough
-// particles that the rows' redundant arithmetic costs less than the chain it shortens.  A SIMD holds 8 (RK4) or 2
+// particles that the rows' redundant arithmetic costs less than the chain it shortens.  A SIMD holds 3 (RK4) or 1
 // wavefronts of rows there.  100 steps through a 97 x 81 x 113 map, rows / a lane per particle in ms:
-//   rk4    1: 0.17 / 0.83   4096: 0.20 / 1.30   16384: 0.53 / 1.28   32768: 1.01 / 1.27   65536: 1.93 / 1.33
-//   vay    1: 0.15 / 0.29   4096: 0.17 / 0.43    8192: 0.28 / 0.43   16384: 0.52 / 0.42
-//   boris  1: 0.10 / 0.24   4096: 0.12 / 0.38    8192: 0.16 / 0.37   16384: 0.29 / 0.37
+//   rk4    1: 0.17 / 0.46   4096: 0.19 / 0.60   8192: 0.28 / 0.60   16384: 0.53 / 0.56   32768: 1.01 / 0.58
+//   vay    1: 0.15 / 0.20   4096: 0.17 / 0.24   8192: 0.28 / 0.24   16384: 0.52 / 0.24
+//   boris  1: 0.10 / 0.14   4096: 0.12 / 0.19   8192: 0.17 / 0.19   16384: 0.30 / 0.18
 // (1000 RK4 steps of 7 particles with a record per step: 9.6 -> 1.75 ms of device time.)
-constexpr int64_t kRowMaxRk4 = 32768, kRowMaxSingle = 8192;
+constexpr int64_t kRowMaxRk4 = 12288, kRowMaxSingle = 4096;
 
 static bool row_route(int alg, const PushParams& p) {
-    if (p.mesh || p.alive || !p.fused || !p.E.map.uniform || !stage_corners_ok(p.E.map)) return false;
+    if (p.mesh || p.alive || !p.fused || !p.E.map.uniform || !fused_3d(p)) return false;
     return p.n <= (alg == PP_ALG_RK4 || alg == PP_ALG_RK4_REL ? kRowMaxRk4 : kRowMaxSingle);
 }
 
@@ -364,6 +381,8 @@ hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s) {
         else PP_STRICT_CASES(true, kFieldsGeneral)
     } else if (fields == kFieldsUniform) {
         PP_STRICT_CASES(false, kFieldsUniform)
+    } else if (fields == kFieldsMap3d) {
+        PP_STRICT_CASES(false, kFieldsMap3d)
     } else if (fields == kFieldsFusedStatic) {
         PP_STRICT_CASES(false, kFieldsFusedStatic)
     } else if (fields == kFieldsFusedRF) {
@@ -414,6 +433,12 @@ hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s) {
 
 hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s) {
     hipLaunchKernelGGL(k_add_i64, dim3(1), dim3(64), 0, s, p, v);
+    return hipGetLastError();
+}
+
+hipError_t launch_interleave(const double* src, const MapDesc& d, double* raw, hipStream_t s) {
+    const int64_t work = (int64_t)d.ng[0] * d.ng[1] * d.ng[2] * d.ncomp;
+    hipLaunchKernelGGL(k_interleave, dim3(grid_for(work, 256)), dim3(256), 0, s, src, d, raw);
     return hipGetLastError();
 }
 

@@ -8,7 +8,7 @@ import pytest
 import pypatools_amd as pa
 
 pytestmark = pytest.mark.gpu
-LIMIT = {"rk4": 32768, "rk4_rel": 32768}        # others: 8192
+LIMIT = {"rk4": 12288, "rk4_rel": 12288}        # others: 4096
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -39,7 +39,7 @@ def _setup(n, periodic, jitter, seed=23):
 @pytest.mark.parametrize("periodic", [False, True])
 @pytest.mark.parametrize("algorithm", ["boris", "vay", "rk4", "rk4_rel", "yoshida"])
 def test_rows_and_lanes_agree(algorithm, periodic, jitter, rf):
-    limit = LIMIT.get(algorithm, 8192)
+    limit = LIMIT.get(algorithm, 4096)
     e, b, r0, v0 = _setup(limit + 1, periodic, jitter)
     e = 0.7 * e
     if rf:
@@ -57,7 +57,7 @@ def test_non_finite_particles_stay_alone(periodic):
     e, b, r0, v0 = _setup(9, periodic, False)
     r0[3, 2], v0[5, 0] = np.nan, np.inf
     push = pa.Pusher(pa.IonSpecies("proton"), "rk4")
-    rl, vl, _ = push.track_batch(np.tile(r0, (3700, 1)), np.tile(v0, (3700, 1)), e, b, 5, 2e-11, 1)
+    rl, vl, _ = push.track_batch(np.tile(r0, (1400, 1)), np.tile(v0, (1400, 1)), e, b, 5, 2e-11, 1)
     rs, vs, _ = push.track_batch(r0, v0, e, b, 5, 2e-11, 1)
     np.testing.assert_array_equal(rs, rl[:, :9])
     np.testing.assert_array_equal(vs, vl[:, :9])
