@@ -154,6 +154,11 @@ int pp_malloc(void** dptr, size_t bytes);
 int pp_free(void* dptr);
 int pp_memcpy_h2d(void* dst, const void* src, size_t bytes, pp_stream s);
 int pp_memcpy_d2h(void* dst, const void* src, size_t bytes, pp_stream s);
+/* Two device buffers to the host in one blocking call (their copies share the staging threads). */
+int pp_memcpy_d2h_pair(void* dst0, const void* src0, size_t bytes0, void* dst1, const void* src1, size_t bytes1,
+                       pp_stream s);
+/* Frees the pinned staging buffers (at most 48 MiB) that large copies keep. */
+int pp_release_staging(void);
 int pp_memcpy_d2d(void* dst, const void* src, size_t bytes, pp_stream s);
 int pp_fill_f64(double* dptr, double value, int64_t count, pp_stream s);   /* kernel fill, graph-safe */
 int pp_stream_create(pp_stream* s);
@@ -373,6 +378,14 @@ int pp_iota_i32(int32_t* ids, int64_t n, pp_stream s);
 int pp_aos_to_soa(const double* aos, int64_t m, double* a, double* b, double* c, pp_stream s);
 int pp_soa_to_aos(const double* a, const double* b, const double* c, int64_t m, double* aos, pp_stream s);
 int pp_v_to_u(double* vx, double* vy, double* vz, int64_t m, pp_stream s);   /* u = gamma(v) v, pusher.py:74-96 clamp */
+/* Velocities of n state slots as rows of aos (n, 3), u as v where ustate is set or, with bunches (device table) and
+   group (bunch of each slot), where the slot's bunch runs a u-state algorithm.  alive (optional): rows of dead slots
+   stay as they are. */
+int pp_velocity_rows(const double* vx, const double* vy, const double* vz, const uint8_t* alive, int32_t ustate,
+                     const pp_bunch* bunches, const int32_t* group, int64_t n, double* aos, pp_stream s);
+/* v -> u in the slots whose bunch runs a u-state algorithm. */
+int pp_bunch_v_to_u(double* vx, double* vy, double* vz, const pp_bunch* bunches, const int32_t* group, int64_t n,
+                    pp_stream s);
 int pp_u_to_v(double* ux, double* uy, double* uz, int64_t m, pp_stream s);   /* v = u / sqrt(1 + u^2/c^2) */
 
 /* Beam moments of a device-resident state (ParticleDistribution, particles.py:693-843).

@@ -3,6 +3,7 @@
 The library is built in-tree (``python -m pypatools_amd.build``).  Loading fails
 loudly when it is missing: there is no CPU fallback for the push or the gather.
 """
+import atexit
 import ctypes
 import os
 import threading
@@ -128,6 +129,9 @@ SIGNATURES = {
     "pp_host_alloc": (c_int32, [ctypes.POINTER(c_void_p), ctypes.c_size_t]),
     "pp_host_free": (c_int32, [c_void_p]),
     "pp_memcpy_h2d_async": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
+    "pp_memcpy_d2h_pair": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, c_void_p, c_void_p, ctypes.c_size_t,
+                                     c_void_p]),
+    "pp_release_staging": (c_int32, []),
     "pp_memcpy_d2h_async": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
     "pp_event_query": (c_int32, [c_void_p, ctypes.POINTER(c_int32)]),
     "pp_event_sync": (c_int32, [c_void_p]),
@@ -200,6 +204,9 @@ SIGNATURES = {
     "pp_beam_noalloc_scratch_bytes": (c_int32, [ctypes.POINTER(ctypes.c_size_t)]),
     "pp_soa_to_aos": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     "pp_v_to_u": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    "pp_velocity_rows": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int64,
+                                   c_void_p, c_void_p]),
+    "pp_bunch_v_to_u": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "pp_u_to_v": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
 }
 
@@ -219,6 +226,7 @@ def lib():
                 fn = getattr(h, name)
                 fn.restype = res
                 fn.argtypes = args
+            atexit.register(h.pp_release_staging)
             _lib = h
     return _lib
 

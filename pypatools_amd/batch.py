@@ -24,7 +24,7 @@ import time
 import numpy as np
 
 from . import _lib
-from .device import DeviceArray, Stream, synchronize
+from .device import DeviceArray, Stream, synchronize, to_host_pair
 from .engine import DEFAULT_REFINE_BITS, STAGGERED, U_STATE, _fused_map, motion_axis
 from .interpolators import DeviceFieldMap
 
@@ -137,13 +137,11 @@ class BatchedTracker:
         v = np.concatenate([b.v0 for b in self.bunches]) if self.bunches else np.zeros((0, 3))
         from .engine import ParticleState
         self.state = ParticleState.from_host(r, v)
-        for k, b in enumerate(self.bunches):
-            if b.algorithm in U_STATE and b.n:
-                o = int(offsets[k])
-                _lib.call("pp_v_to_u", self.state.vx.view_ptr(o), self.state.vy.view_ptr(o),
-                          self.state.vz.view_ptr(o), b.n, None)
         group = np.repeat(np.arange(len(self.bunches), dtype=np.int32), counts)
         self.group = DeviceArray.from_host(group if self.n else np.zeros(1, np.int32))
+        if any(b.algorithm in U_STATE for b in self.bunches):
+            _lib.call("pp_bunch_v_to_u", self.state.vx.ptr, self.state.vy.ptr, self.state.vz.ptr, self.table.ptr,
+                      self.group.ptr, self.n, None)
         m0 = self.maps[0]
         ncell = int(np.prod([max(s - 1, 1) for s in m0.shape[:2]]) * (m0.shape[2] if m0.periodic_z
                                                                       else max(m0.shape[2] - 1, 1)))
@@ -271,15 +269,10 @@ class BatchedTracker:
         """Per-bunch (r, v) host arrays in original particle order (v = velocity for every algorithm)."""
         st = self.state
         st.unsort()
-        for k, b in enumerate(self.bunches):
-            if b.algorithm in U_STATE and b.n:
-                o = int(self.offsets[k])
-                _lib.call("pp_u_to_v", st.vx.view_ptr(o), st.vy.view_ptr(o), st.vz.view_ptr(o), b.n, None)
-        r, v = st.to_host()
-        for k, b in enumerate(self.bunches):
-            if b.algorithm in U_STATE and b.n:
-                o = int(self.offsets[k])
-                _lib.call("pp_v_to_u", st.vx.view_ptr(o), st.vy.view_ptr(o), st.vz.view_ptr(o), b.n, None)
+        vel = DeviceArray((st.n, 3))
+        _lib.call("pp_velocity_rows", st.vx.ptr, st.vy.ptr, st.vz.ptr, None, 0, self.table.ptr, self.group.ptr, st.n,
+                  vel.ptr, None)
+        r, v = to_host_pair(st.positions_aos(), vel)
         out = []
         for k, b in enumerate(self.bunches):
             o, c = int(self.offsets[k]), int(self.counts[k])

@@ -20,7 +20,7 @@ BUILD_DIR = os.path.join(PKG, "_build")
 
 ARCH = os.environ.get("PYPAT_OFFLOAD_ARCH", "gfx950")
 SOURCES = ["pp_host.hip", "pp_strict.hip", "pp_fast.hip", "pp_sort.hip", "pp_moments.hip", "pp_collide.hip",
-           "pp_poisson.hip", "pp_spline.hip"]
+           "pp_poisson.hip", "pp_spline.hip", "pp_copy.hip"]
 COMMON = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",
     "-I", INCLUDE, "-I", CSRC,

@@ -139,15 +139,28 @@ int pp_free(void* dptr) {
 
 int pp_memcpy_h2d(void* dst, const void* src, size_t bytes, pp_stream s) {
     if (!bytes) return PP_OK;
-    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream_of(s)), "hipMemcpy H2D");
-    HIP_TRY(hipStreamSynchronize(stream_of(s)), "hipStreamSynchronize");
+    const pp_copy::Region r = {const_cast<void*>(src), dst, bytes};
+    HIP_TRY(pp_copy::transfer(&r, 1, false, g_device, stream_of(s)), "hipMemcpy H2D");
     return PP_OK;
 }
 
 int pp_memcpy_d2h(void* dst, const void* src, size_t bytes, pp_stream s) {
     if (!bytes) return PP_OK;
-    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream_of(s)), "hipMemcpy D2H");
-    HIP_TRY(hipStreamSynchronize(stream_of(s)), "hipStreamSynchronize");
+    const pp_copy::Region r = {dst, const_cast<void*>(src), bytes};
+    HIP_TRY(pp_copy::transfer(&r, 1, true, g_device, stream_of(s)), "hipMemcpy D2H");
+    return PP_OK;
+}
+
+int pp_memcpy_d2h_pair(void* dst0, const void* src0, size_t bytes0, void* dst1, const void* src1, size_t bytes1,
+                       pp_stream s) {
+    if ((bytes0 && (!dst0 || !src0)) || (bytes1 && (!dst1 || !src1))) return fail(PP_ERR_INVALID, "null pointer");
+    const pp_copy::Region r[2] = {{dst0, const_cast<void*>(src0), bytes0}, {dst1, const_cast<void*>(src1), bytes1}};
+    HIP_TRY(pp_copy::transfer(r, 2, true, g_device, stream_of(s)), "hipMemcpy D2H");
+    return PP_OK;
+}
+
+int pp_release_staging(void) {
+    pp_copy::release();
     return PP_OK;
 }
 
@@ -358,7 +371,8 @@ int pp_map_create(const double* values, int32_t ncomp, int32_t nx, int32_t ny, i
     void* src = nullptr;
     hipError_t ue = hipMalloc(&src, src_bytes);
     if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "hipMalloc (field map)"); }
-    ue = hipMemcpyAsync(src, values, src_bytes, hipMemcpyHostToDevice, s);
+    const pp_copy::Region up = {const_cast<double*>(values), src, src_bytes};
+    ue = pp_copy::transfer(&up, 1, false, g_device, s);
     if (ue == hipSuccess) ue = pp_strict::launch_interleave(static_cast<const double*>(src), d, static_cast<double*>(p), s);
     if (ue == hipSuccess) ue = hipStreamSynchronize(s);
     (void)hipFree(src);
@@ -1332,6 +1346,30 @@ int pp_soa_to_aos(const double* a, const double* b, const double* c, int64_t m, 
 
 int pp_v_to_u(double* vx, double* vy, double* vz, int64_t m, pp_stream s) {
     return util_common(PP_UT_V2U, vx, vy, vz, nullptr, m, s);
+}
+
+int pp_velocity_rows(const double* vx, const double* vy, const double* vz, const uint8_t* alive, int32_t ustate,
+                     const pp_bunch* bunches, const int32_t* group, int64_t n, double* aos, pp_stream s) {
+    int rc = ensure_init();
+    if (rc) return rc;
+    if (n < 0) return fail(PP_ERR_INVALID, "negative size");
+    if (n == 0) return PP_OK;
+    if (!vx || !vy || !vz || !aos || (bunches && !group)) return fail(PP_ERR_INVALID, "null device pointer");
+    HIP_TRY(pp_strict::launch_velocity_rows(vx, vy, vz, alive, ustate != 0, bunches, group, n, kClight * kClight, aos,
+                                            stream_of(s)), "velocity rows");
+    return PP_OK;
+}
+
+int pp_bunch_v_to_u(double* vx, double* vy, double* vz, const pp_bunch* bunches, const int32_t* group, int64_t n,
+                    pp_stream s) {
+    int rc = ensure_init();
+    if (rc) return rc;
+    if (n < 0) return fail(PP_ERR_INVALID, "negative size");
+    if (n == 0) return PP_OK;
+    if (!vx || !vy || !vz || !bunches || !group) return fail(PP_ERR_INVALID, "null device pointer");
+    HIP_TRY(pp_strict::launch_velocity_convert(vx, vy, vz, bunches, group, n, kClight * kClight, stream_of(s)),
+            "velocity conversion");
+    return PP_OK;
 }
 
 int pp_u_to_v(double* ux, double* uy, double* uz, int64_t m, pp_stream s) {

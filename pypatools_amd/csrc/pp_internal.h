@@ -161,11 +161,29 @@ struct BatchArgs {
 hipError_t launch_batch_kernel(const BatchArgs& args, hipStream_t s);
 hipError_t launch_util(int which, double* a, double* b, double* c, double* aos, int64_t m, double c2,
                        hipStream_t s);
+// velocities of a state (u-state slots as v) as rows of an (n, 3) array, or v -> u in place (velocity_convert).
+// ustate: every slot holds u; else, with bunches, the slots of a bunch with a u-state algorithm.  alive: other rows stay.
+hipError_t launch_velocity_rows(const double* vx, const double* vy, const double* vz, const uint8_t* alive, bool ustate,
+                                const pp_bunch* bunches, const int32_t* group, int64_t n, double c2, double* aos,
+                                hipStream_t s);
+hipError_t launch_velocity_convert(double* vx, double* vy, double* vz, const pp_bunch* bunches, const int32_t* group,
+                                   int64_t n, double c2, hipStream_t s);
 hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s);
 hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s);
 hipError_t launch_interleave(const double* src, const MapDesc& d, double* raw, hipStream_t s);
 hipError_t launch_build_coef(const MapDesc& d, double* c64, float* c32, hipStream_t s);
 }  // namespace pp_strict
+
+// blocking copies of ordinary host memory (pp_copy.hip): every region of a call, all to the host or all to the device
+namespace pp_copy {
+struct Region {
+    void* host;
+    void* dev;
+    size_t bytes;
+};
+hipError_t transfer(const Region* r, int n, bool to_host, int device, hipStream_t s);
+void release();     // frees the pinned buffers that no transfer uses
+}  // namespace pp_copy
 
 namespace pp_fast {
 hipError_t launch_push(int alg, int prec, const PushParams& p, int block, hipStream_t s);

@@ -86,6 +86,34 @@ __global__ void __launch_bounds__(256) k_util(int which, double* a, double* b, d
     }
 }
 
+DEV bool holds_u(const pp_bunch& b) { return b.algorithm == PP_ALG_BORIS_REL || b.algorithm == PP_ALG_VAY; }
+
+__global__ void __launch_bounds__(256) k_velocity_rows(const double* __restrict__ vx, const double* __restrict__ vy,
+                                                       const double* __restrict__ vz, const uint8_t* __restrict__ alive,
+                                                       int ustate, const pp_bunch* __restrict__ bunches,
+                                                       const int32_t* __restrict__ group, int64_t n, double c2,
+                                                       double* __restrict__ aos) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n || (alive && !alive[i])) return;
+    d3 v = mk3(vx[i], vy[i], vz[i]);
+    if (ustate || (bunches && holds_u(bunches[group[i]]))) v = v_from_u(v, c2);
+    aos[3 * i] = v.x;
+    aos[3 * i + 1] = v.y;
+    aos[3 * i + 2] = v.z;
+}
+
+__global__ void __launch_bounds__(256) k_velocity_convert(double* vx, double* vy, double* vz,
+                                                          const pp_bunch* __restrict__ bunches,
+                                                          const int32_t* __restrict__ group, int64_t n, double c2) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n || !holds_u(bunches[group[i]])) return;
+    const d3 v = mk3(vx[i], vy[i], vz[i]);
+    const d3 u = rgamma(v, c2) * v;
+    vx[i] = u.x;
+    vy[i] = u.y;
+    vz[i] = u.z;
+}
+
 __global__ void k_add_i64(int64_t* p, int64_t v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *p += v;
 }
@@ -423,6 +451,20 @@ hipError_t launch_batch_kernel(const BatchArgs& args, hipStream_t s) {
 
 hipError_t launch_util(int which, double* a, double* b, double* c, double* aos, int64_t m, double c2, hipStream_t s) {
     hipLaunchKernelGGL(k_util, dim3(grid_for(m, 256)), dim3(256), 0, s, which, a, b, c, aos, m, c2);
+    return hipGetLastError();
+}
+
+hipError_t launch_velocity_rows(const double* vx, const double* vy, const double* vz, const uint8_t* alive, bool ustate,
+                                const pp_bunch* bunches, const int32_t* group, int64_t n, double c2, double* aos,
+                                hipStream_t s) {
+    hipLaunchKernelGGL(k_velocity_rows, dim3(grid_for(n, 256)), dim3(256), 0, s, vx, vy, vz, alive, ustate ? 1 : 0,
+                       bunches, group, n, c2, aos);
+    return hipGetLastError();
+}
+
+hipError_t launch_velocity_convert(double* vx, double* vy, double* vz, const pp_bunch* bunches, const int32_t* group,
+                                   int64_t n, double c2, hipStream_t s) {
+    hipLaunchKernelGGL(k_velocity_convert, dim3(grid_for(n, 256)), dim3(256), 0, s, vx, vy, vz, bunches, group, n, c2);
     return hipGetLastError();
 }
 

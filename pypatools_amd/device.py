@@ -95,6 +95,13 @@ class DeviceArray:
         self.free()
 
 
+def to_host_pair(a, b):
+    """Host arrays of two device arrays, in one transfer."""
+    out = np.empty(a.shape, a.dtype), np.empty(b.shape, b.dtype)
+    _lib.call("pp_memcpy_d2h_pair", out[0].ctypes.data, a.ptr, a.nbytes, out[1].ctypes.data, b.ptr, b.nbytes, None)
+    return out
+
+
 class PinnedArray:
     """Page-locked host memory (pp_host_alloc) with a NumPy view, for asynchronous copies."""
 

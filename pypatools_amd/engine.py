@@ -19,7 +19,7 @@ import ctypes
 import numpy as np
 
 from . import _lib
-from .device import DeviceArray
+from .device import DeviceArray, to_host_pair
 from .field import (CompositeField, Field, RFField, ScaledField, compile_sum, compile_term, evaluate_on_device,
                     is_time_dependent, rf_source)
 from .interpolators import DeviceFieldMap
@@ -43,9 +43,9 @@ DEFAULT_REFINE_BITS = 3
 
 
 def motion_axis(v):
-    """Axis of the largest mean |velocity| component of an (M, 3) array."""
+    """Axis of the largest mean |velocity| component of an (M, 3) array (of at most 4096 rows, evenly spaced)."""
     v = np.asarray(v, dtype=np.float64).reshape(-1, 3)
-    return int(np.argmax(np.abs(v[: min(len(v), 100000)]).mean(axis=0))) if len(v) else 2
+    return int(np.argmax(np.abs(v[::-(-len(v) // 4096)]).mean(axis=0))) if len(v) else 2
 
 
 class ParticleState:
@@ -82,7 +82,7 @@ class ParticleState:
         return out
 
     def to_host(self):
-        return self.positions_aos().to_host(), self.velocities_aos().to_host()
+        return to_host_pair(self.positions_aos(), self.velocities_aos())
 
     def load_aos(self, r_dev=None, v_dev=None):
         if r_dev is not None:
@@ -241,18 +241,12 @@ def _sum_members(f):
 def build_rf_table(field, t0, dt, n_rows):
     """Host table [n_rows][4 stages][cos, sin] for RFField ``field`` at t_n + c dt, c = (0, 1/2, 1/2, 1).
 
-    Evaluated element by element with the same expressions the pusher uses for a
-    time-aware field (t_n = t0 + n*dt, stage time t_n + c*dt, ``omega*t + phase``).
+    The expressions are the ones the pusher uses for a time-aware field (t_n = t0 + n*dt,
+    stage time t_n + c*dt, ``omega*t + phase``), rounded in the same order.
     """
-    tab = np.empty((n_rows, 4, 2))
-    for n in range(n_rows):
-        t_n = t0 + n * dt
-        for s, c in enumerate((0.0, 0.5, 0.5, 1.0)):
-            ts = t_n + c * dt
-            arg = field.omega * ts + field.phase
-            tab[n, s, 0] = np.cos(arg)
-            tab[n, s, 1] = np.sin(arg)
-    return tab
+    t_n = t0 + np.arange(n_rows, dtype=np.float64) * dt
+    arg = field.omega * (t_n[:, None] + np.array([0.0, 0.5, 0.5, 1.0]) * dt) + field.phase
+    return np.stack([np.cos(arg), np.sin(arg)], axis=-1)
 
 
 class Tracker:
@@ -364,16 +358,11 @@ class Tracker:
             self._slow_loop(st, fp, nsteps, dt, t0, rf, hist, elec, active, dtp, verbose)
         if alg in STAGGERED:
             self._kick(st, fp, fused, 0.5 * dt, nsteps, rf, t0, dt)
-            vfin = DeviceArray((M, 3))
-            self._velocity_record(st, vfin, ustate)
-        r_hist = rh.to_host()
-        v_hist = vh.to_host()
-        if alg in STAGGERED:
-            vf = vfin.to_host()
-            if batch:
-                v_hist[-1][active] = vf[active]
-            else:
-                v_hist[-1] = vf
+            # resynchronised velocities into the last record; particles that were lost keep theirs
+            self._velocity_record(st, _row(vh, n_records - 1, M), ustate, live_only=True)
+        r_hist, v_hist = to_host_pair(rh, vh)
+        if elec is not None:
+            active[:] = st.alive.to_host().astype(bool)
         if verbose:
             print(f"Tracking complete: {nsteps} steps, {M} particles")
         if return_state:
@@ -448,14 +437,10 @@ class Tracker:
             st.u_to_v()
         return st.to_host()
 
-    def _velocity_record(self, st, out_aos, ustate):
-        if not ustate:
-            return st.velocities_aos(out_aos)
-        tmp = [DeviceArray((st.n,)) for _ in range(3)]
-        for d, s in zip(tmp, (st.vx, st.vy, st.vz)):
-            d.copy_from(s)
-        _lib.call("pp_u_to_v", tmp[0].ptr, tmp[1].ptr, tmp[2].ptr, st.n, None)
-        _lib.call("pp_soa_to_aos", tmp[0].ptr, tmp[1].ptr, tmp[2].ptr, st.n, out_aos.ptr, None)
+    def _velocity_record(self, st, out_aos, ustate, live_only=False):
+        alive = st.alive.ptr if live_only and st.alive is not None else None
+        _lib.call("pp_velocity_rows", st.vx.ptr, st.vy.ptr, st.vz.ptr, alive, 1 if ustate else 0, None, None, st.n,
+                  out_aos.ptr, None)
         return out_aos
 
     def _kick(self, st, fp, fused, dt_kick, step, rf, t0, dt):
@@ -539,7 +524,6 @@ class Tracker:
             _lib.call("pp_push_lossy", a, elec.handle, None)
             step += k
         st.unsort()
-        active[:] = st.alive.to_host().astype(bool)
 
     def _rk4_stage_loop(self, st, fp, nsteps, dt, t0, hist, dtp, verbose):
         """_rk4_step_batch (pusher.py:803-892) with fields evaluated between device stage kernels."""
