@@ -112,7 +112,23 @@ struct Gemm {
     const double* A; const double* B; double* C;
     int64_t M, N, K, lda, ldb, ldc, sa, sb, sc;
     double alpha;
+    // what becomes of an entry after the scaling by alpha (entries are nodes of the box there, sc = 0):
+    const int32_t* type;            // node types, or null: 0 on conductor nodes (type 2)
+    const double *lx, *ly, *lz;     // lx not null: times scale / (lx[row] + ly[column / nz] + lz[column % nz])
+    int nz;
+    double scale;
 };
+
+__device__ __forceinline__ void gemm_put(const Gemm& g, int64_t b, int64_t gm, int64_t gn, double v) {
+    if (gm >= g.M || gn >= g.N) return;
+    const int64_t e = b * g.sc + gm * g.ldc + gn;
+    v = g.alpha * v;
+    if (g.lx) {
+        const uint32_t y = (uint32_t)gn / (uint32_t)g.nz;
+        v = v * g.scale / ((g.lx[gm] + g.ly[y]) + g.lz[(uint32_t)gn - y * (uint32_t)g.nz]);
+    }
+    g.C[e] = g.type && g.type[e] == 2 ? 0.0 : v;
+}
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
@@ -128,7 +144,6 @@ __global__ void __launch_bounds__(256) k_gemm_mfma(const Gemm g) {
     const int64_t b = blockIdx.z;
     const double* A = g.A + b * g.sa;
     const double* B = g.B + b * g.sb;
-    double* C = g.C + b * g.sc;
     const int64_t m0 = (int64_t)blockIdx.y * kBM, n0 = (int64_t)blockIdx.x * kBN;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = (wave >> 1) * (kBM / 2), wn = (wave & 1) * (kBN / 2);   // this wavefront's quarter of the tile
@@ -194,22 +209,8 @@ __global__ void __launch_bounds__(256) k_gemm_mfma(const Gemm g) {
         for (int v = 0; v < kTV; ++v)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t gm = m0 + wm + 16 * u + lk + 4 * r, gn = n0 + wn + 16 * v + li;
-                if (gm < g.M && gn < g.N) C[gm * g.ldc + gn] = g.alpha * acc[u][v][r];
+                gemm_put(g, b, m0 + wm + 16 * u + lk + 4 * r, n0 + wn + 16 * v + li, acc[u][v][r]);
             }
-}
-
-// bhat / (lambda_x[i] + lambda_y[j] + lambda_z[k]) * scale, with b = rho / eps0 folded into scale
-__global__ void __launch_bounds__(256) k_divide(double* __restrict__ v, const double* __restrict__ lx,
-                                                const double* __restrict__ ly, const double* __restrict__ lz, int nx,
-                                                int ny, int nz, double scale) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)nx * ny * nz) return;
-    const int k = (int)(t % nz);
-    const int64_t r = t / nz;
-    const int j = (int)(r % ny);
-    const int i = (int)(r / ny);
-    v[t] = v[t] * scale / ((lx[i] + ly[j]) + lz[k]);
 }
 
 // E = -grad(phi) by central differences on interior nodes, 0 on the outer layer (poisson_amg.py:98-130)
@@ -239,113 +240,179 @@ __global__ void __launch_bounds__(256) k_gradient(const PoissonDesc d, const dou
 
 // Operator rows: coef[0] = diagonal, coef[1 + d] = neighbour d (+x, -x, +y, -y, +z, -z); 0 where there is no
 // entry (outside the box or a conductor).  Conductor rows hold only the box diagonal (phi = 0 there).
+// Rows without a conductor beside them are the box operator's: `regular` marks them and their coefficients come with
+// the launch (seven tables of doubles were two thirds of what an application read).
 struct SwOperator {
     const double* coef[7];
+    const uint8_t* regular;
+    double box[4];                  // diagonal, x, y, z neighbours of a regular row
     int nx, ny, nz;
 };
 
-__global__ void __launch_bounds__(256) k_sw_apply(const SwOperator A, const double* __restrict__ x,
-                                                  double* __restrict__ y) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n = (int64_t)A.nx * A.ny * A.nz;
-    if (t >= n) return;
+__device__ __forceinline__ double sw_row(const SwOperator& A, const double* __restrict__ x, int64_t t) {
     const int k = (int)(t % A.nz);
     const int64_t r = t / A.nz;
     const int j = (int)(r % A.ny);
     const int i = (int)(r / A.ny);
     const int64_t sx = (int64_t)A.ny * A.nz, sy = A.nz;
-    double acc = A.coef[0][t] * x[t];
-    if (i + 1 < A.nx) acc += A.coef[1][t] * x[t + sx];
-    if (i > 0) acc += A.coef[2][t] * x[t - sx];
-    if (j + 1 < A.ny) acc += A.coef[3][t] * x[t + sy];
-    if (j > 0) acc += A.coef[4][t] * x[t - sy];
-    if (k + 1 < A.nz) acc += A.coef[5][t] * x[t + 1];
-    if (k > 0) acc += A.coef[6][t] * x[t - 1];
-    y[t] = acc;
+    double c[7];
+    if (A.regular[t]) {
+#pragma unroll
+        for (int q = 0; q < 7; ++q) c[q] = A.box[(q + 1) / 2];
+    } else {
+#pragma unroll
+        for (int q = 0; q < 7; ++q) c[q] = A.coef[q][t];
+    }
+    double acc = c[0] * x[t];
+    if (i + 1 < A.nx) acc += c[1] * x[t + sx];
+    if (i > 0) acc += c[2] * x[t - sx];
+    if (j + 1 < A.ny) acc += c[3] * x[t + sy];
+    if (j > 0) acc += c[4] * x[t - sy];
+    if (k + 1 < A.nz) acc += c[5] * x[t + 1];
+    if (k > 0) acc += c[6] * x[t - 1];
+    return acc;
 }
 
-constexpr int kDotBlocks = 512;
+// BiCGSTAB scalars in device memory (no host round trip inside an iteration).  kDone: the residual is at the
+// tolerance (or not a number), and the updates of iterations enqueued beyond that do nothing.
+enum { kRho = 0, kRhoOld, kAlpha, kOmega, kBeta, kBNorm, kRes, kDone, kIter, kScalars = 16 };
 
-// partial sums of up to three dot products: part[block][q] = sum over the block's slice of a_q . b_q
-struct Dots {
-    const double* a[3];
-    const double* b[3];
-    int nq;
-};
+constexpr int kDotBlocks = 1024;
 
-__global__ void __launch_bounds__(256) k_dots(const Dots D, int64_t n, double* __restrict__ part) {
-    __shared__ double red[4][3];
-    double s[3] = {0.0, 0.0, 0.0};
-    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256)
-        for (int q = 0; q < D.nq; ++q) s[q] += D.a[q][t] * D.b[q][t];
-    for (int q = 0; q < 3; ++q)
-        for (int off = 32; off > 0; off >>= 1) s[q] += __shfl_xor(s[q], off, 64);
-    if ((threadIdx.x & 63) == 0)
-        for (int q = 0; q < 3; ++q) red[threadIdx.x >> 6][q] = s[q];
+// partial sums of the block's two dot products into part[block][2]
+__device__ __forceinline__ void put_partials(double s0, double s1, double* __restrict__ part) {
+    __shared__ double red[4][2];
+    for (int off = 32; off > 0; off >>= 1) {
+        s0 += __shfl_xor(s0, off, 64);
+        s1 += __shfl_xor(s1, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6][0] = s0;
+        red[threadIdx.x >> 6][1] = s1;
+    }
     __syncthreads();
-    if (threadIdx.x < 3) part[(size_t)blockIdx.x * 3 + threadIdx.x] =
+    if (threadIdx.x < 2) part[(size_t)blockIdx.x * 2 + threadIdx.x] =
         ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
 }
 
-// out[slot + q] = sum of the kDotBlocks partials of dot q, in a fixed order
-__global__ void __launch_bounds__(256) k_dots_finish(const double* __restrict__ part, int nq, double* __restrict__ sc,
-                                                     int slot) {
-    __shared__ double sh[256];
-    for (int q = 0; q < nq; ++q) {
-        double v = 0.0;
-        for (int b = threadIdx.x; b < kDotBlocks; b += 256) v += part[(size_t)b * 3 + q];
-        sh[threadIdx.x] = v;
-        __syncthreads();
-        for (int w = 128; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
+// y = A x with the partials of (y, w) and (y, y)
+__global__ void __launch_bounds__(256) k_sw_apply(const SwOperator A, const double* __restrict__ x,
+                                                  double* __restrict__ y, const double* __restrict__ w,
+                                                  double* __restrict__ part) {
+    const int64_t n = (int64_t)A.nx * A.ny * A.nz;
+    double s0 = 0.0, s1 = 0.0;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+        const double v = sw_row(A, x, t);
+        y[t] = v;
+        s0 += v * w[t];
+        s1 += v * v;
+    }
+    put_partials(s0, s1, part);
+}
+
+// start: r = b - A x into r, r0 and p; partials of (b, b) and (r, r)
+__global__ void __launch_bounds__(256) k_sw_start(const SwOperator A, const double* __restrict__ x,
+                                                  const double* __restrict__ b, double* __restrict__ r,
+                                                  double* __restrict__ r0, double* __restrict__ p,
+                                                  double* __restrict__ part) {
+    const int64_t n = (int64_t)A.nx * A.ny * A.nz;
+    double s0 = 0.0, s1 = 0.0;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+        const double bt = b[t], v = bt - sw_row(A, x, t);
+        r[t] = v;
+        r0[t] = v;
+        p[t] = v;
+        s0 += bt * bt;
+        s1 += v * v;
+    }
+    put_partials(s0, s1, part);
+}
+
+// The sums of the partials in a fixed order, then the scalars they give:
+// stage 0 (start) |b|, the first residual, rho; 1 alpha = rho / (r0, v); 2 omega = (t, s) / (t, t);
+// 3 residual, the next rho and beta.  host: residual, done flag and iteration count in mapped host memory.
+__global__ void __launch_bounds__(256) k_scalars(const double* __restrict__ part, int nblocks, int stage, double rtol,
+                                                 double* __restrict__ sc, double* __restrict__ host) {
+    __shared__ double sh[2][256];
+    double v0 = 0.0, v1 = 0.0;
+    for (int b = threadIdx.x; b < nblocks; b += 256) {
+        v0 += part[(size_t)b * 2];
+        v1 += part[(size_t)b * 2 + 1];
+    }
+    sh[0][threadIdx.x] = v0;
+    sh[1][threadIdx.x] = v1;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) {
+            sh[0][threadIdx.x] += sh[0][threadIdx.x + w];
+            sh[1][threadIdx.x] += sh[1][threadIdx.x + w];
         }
-        if (threadIdx.x == 0) sc[slot + q] = sh[0];
         __syncthreads();
     }
-}
-
-// BiCGSTAB scalars in device memory (no host round trip inside an iteration)
-// (b, b) and (r, r) are adjacent, as are (t, s) and (t, t): one two-dot reduction fills each pair
-enum { kRho = 0, kRhoOld, kAlpha, kOmega, kBeta, kR0V, kTS, kTT, kBB, kRR, kScalars = 16 };
-
-__global__ void k_scalars(double* sc, int stage) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (stage == 0) {          // start: rho_old = alpha = omega = 1
-        sc[kRhoOld] = 1.0;
-        sc[kAlpha] = 1.0;
+    if (threadIdx.x != 0) return;
+    const double q0 = sh[0][0], q1 = sh[1][0];
+    if (stage == 0) {
+        sc[kBNorm] = sqrt(q0);
+        sc[kRes] = q0 > 0.0 ? sqrt(q1) / sqrt(q0) : 0.0;
+        sc[kDone] = sc[kRes] > rtol ? 0.0 : 1.0;
+        sc[kIter] = 0.0;
+        sc[kRho] = q1;              // (r0, r) with r0 = r
+        sc[kBeta] = 0.0;            // p = r
         sc[kOmega] = 1.0;
-    } else if (stage == 1) {   // beta from the new rho
-        sc[kBeta] = (sc[kRho] / sc[kRhoOld]) * (sc[kAlpha] / sc[kOmega]);
-    } else if (stage == 2) {   // alpha = rho / (r0, v)
-        sc[kAlpha] = sc[kRho] / sc[kR0V];
-    } else if (stage == 3) {   // omega = (t, s) / (t, t); rho_old = rho
-        sc[kOmega] = sc[kTT] != 0.0 ? sc[kTS] / sc[kTT] : 0.0;
-        sc[kRhoOld] = sc[kRho];
+    } else if (sc[kDone] == 0.0) {
+        if (stage == 1) {
+            sc[kAlpha] = sc[kRho] / q0;
+        } else if (stage == 2) {
+            sc[kOmega] = q1 != 0.0 ? q0 / q1 : 0.0;
+        } else {
+            const double rho = q0;
+            sc[kBeta] = (rho / sc[kRho]) * (sc[kAlpha] / sc[kOmega]);
+            sc[kRho] = rho;
+            sc[kRes] = sqrt(q1) / sc[kBNorm];
+            sc[kIter] += 1.0;
+            sc[kDone] = sc[kRes] > rtol ? 0.0 : 1.0;
+        }
+    }
+    if (host) {
+        host[0] = sc[kRes];
+        host[1] = sc[kDone];
+        host[2] = sc[kIter];
     }
 }
 
-// which: 0 p = r + beta (p - omega v); 1 s = r - alpha v; 2 x += alpha ph + omega sh, r = s - omega t;
-// 3 r = b - r (residual from A x in r); 4 u0 = w0; 5 u0 = 0
-__global__ void __launch_bounds__(256) k_bicg_update(int which, int64_t n, const double* __restrict__ sc, double* u0,
-                                                     double* u1, const double* w0, const double* w1, const double* w2,
-                                                     const double* w3) {
+// p = r + beta (p - omega v)
+__global__ void __launch_bounds__(256) k_bicg_p(int64_t n, const double* __restrict__ sc, double* __restrict__ p,
+                                                const double* __restrict__ r, const double* __restrict__ v) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    if (which == 0) {
-        u0[t] = w0[t] + sc[kBeta] * (u0[t] - sc[kOmega] * w1[t]);                  // p
-    } else if (which == 1) {
-        u0[t] = w0[t] - sc[kAlpha] * w1[t];                                        // s
-    } else if (which == 2) {
-        u0[t] = u0[t] + sc[kAlpha] * w0[t] + sc[kOmega] * w1[t];                   // x
-        u1[t] = w2[t] - sc[kOmega] * w3[t];                                        // r
-    } else if (which == 3) {
-        u0[t] = w0[t] - u0[t];
-    } else if (which == 4) {
-        u0[t] = w0[t];
-    } else {
-        u0[t] = 0.0;
+    if (t >= n || sc[kDone] != 0.0) return;
+    p[t] = r[t] + sc[kBeta] * (p[t] - sc[kOmega] * v[t]);
+}
+
+// s = r - alpha v
+__global__ void __launch_bounds__(256) k_bicg_s(int64_t n, const double* __restrict__ sc, double* __restrict__ s,
+                                                const double* __restrict__ r, const double* __restrict__ v) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n || sc[kDone] != 0.0) return;
+    s[t] = r[t] - sc[kAlpha] * v[t];
+}
+
+// x += alpha ph + omega sh, r = s - omega t, with the partials of (r0, r) and (r, r)
+__global__ void __launch_bounds__(256) k_bicg_x(int64_t n, const double* __restrict__ sc, double* __restrict__ x,
+                                                double* __restrict__ r, const double* __restrict__ ph,
+                                                const double* __restrict__ sh, const double* __restrict__ s,
+                                                const double* __restrict__ tv, const double* __restrict__ r0,
+                                                double* __restrict__ part) {
+    if (sc[kDone] != 0.0) return;
+    const double alpha = sc[kAlpha], omega = sc[kOmega];
+    double s0 = 0.0, s1 = 0.0;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+        x[t] = x[t] + alpha * ph[t] + omega * sh[t];
+        const double v = s[t] - omega * tv[t];
+        r[t] = v;
+        s0 += r0[t] * v;
+        s1 += v * v;
     }
+    put_partials(s0, s1, part);
 }
 
 // b = rho / eps0 on non-conductor nodes, 0 on conductors; and phi = 0 on conductors (which == 1)
@@ -375,6 +442,9 @@ struct pp_poisson {
     double* vec;                         // BiCGSTAB vectors: x r r0 p v s t ph sh (9 N)
     double* part;                        // dot partials
     double* sc;                          // scalars
+    uint8_t* regular;                    // 1: the row is the box operator's (no conductor beside the node)
+    double box[4];                       // its diagonal and x, y, z coefficients
+    double* host;                        // mapped host memory: two slots of (residual, done, iterations)
     double rtol;
     int32_t max_iter;
     mutable int32_t last_iter;           // statistics of the last solve
@@ -390,6 +460,8 @@ int create(const PoissonDesc& d, pp_poisson** out, char* err, size_t errn) {
     P->d = d;
     P->type = nullptr;
     P->coef = P->vec = P->part = P->sc = nullptr;
+    P->host = nullptr;
+    P->regular = nullptr;
     P->rtol = 1e-10;
     P->max_iter = 500;
     P->last_iter = 0;
@@ -427,8 +499,11 @@ int create(const PoissonDesc& d, pp_poisson** out, char* err, size_t errn) {
 }
 
 static void free_conductors(pp_poisson* P) {
-    for (void* q : {(void*)P->type, (void*)P->coef, (void*)P->vec, (void*)P->part, (void*)P->sc})
+    for (void* q : {(void*)P->type, (void*)P->coef, (void*)P->vec, (void*)P->part, (void*)P->sc, (void*)P->regular})
         if (q) (void)hipFree(q);
+    if (P->host) (void)hipHostFree(P->host);
+    P->host = nullptr;
+    P->regular = nullptr;
     P->type = nullptr;
     P->coef = P->vec = P->part = P->sc = nullptr;
     P->h_type.clear();
@@ -475,8 +550,10 @@ static void gemm(const pp_poissonk::Gemm& g, int64_t batch, hipStream_t s) {
     }
 }
 
-// applies S along every axis of `in` (nx, ny, nz) into `out`, via `tmp`; the last product is scaled
-static void transform3(const pp_poisson* P, const double* in, double* tmp, double* out, double scale, hipStream_t s) {
+// applies S along every axis of `in` (nx, ny, nz) into `out`, via `tmp` (z, y, x); the last product is scaled by
+// alpha, then multiplied by divide / eigenvalues (if divide is not 0) and set to 0 on the conductor nodes of type
+static void transform3(const pp_poisson* P, const double* in, double* tmp, double* out, double alpha, double divide,
+                       const int32_t* type, hipStream_t s) {
     const int64_t nx = P->d.n[0], ny = P->d.n[1], nz = P->d.n[2];
     pp_poissonk::Gemm g;
     // z: out (nx ny x nz) = in (nx ny x nz) . S_z  (S symmetric)
@@ -486,21 +563,27 @@ static void transform3(const pp_poisson* P, const double* in, double* tmp, doubl
     g = {P->S[1], out, tmp, ny, nz, ny, ny, nz, nz, 0, ny * nz, ny * nz, 1.0};
     gemm(g, nx, s);
     // x: out (nx x ny nz) = S_x (nx x nx) . tmp (nx x ny nz)
-    g = {P->S[0], tmp, out, nx, ny * nz, nx, nx, ny * nz, ny * nz, 0, 0, 0, scale};
+    g = {P->S[0], tmp, out, nx, ny * nz, nx, nx, ny * nz, ny * nz, 0, 0, 0, alpha, type};
+    if (divide != 0.0) {
+        g.lx = P->lam[0];
+        g.ly = P->lam[1];
+        g.lz = P->lam[2];
+        g.nz = (int)nz;
+        g.scale = divide;
+    }
     gemm(g, 1, s);
 }
 
-// out = A_box^-1 in * scale, A_box the 7-point operator of the box without conductors (exact, by sine transforms)
-static void box_inverse(const pp_poisson* P, const double* in, double* out, double scale, hipStream_t s) {
+// out = A_box^-1 in * scale, A_box the 7-point operator of the box without conductors (exact, by sine transforms);
+// type: 0 on conductor nodes
+static void box_inverse(const pp_poisson* P, const double* in, double* out, double scale, const int32_t* type,
+                        hipStream_t s) {
     const int nx = P->d.n[0], ny = P->d.n[1], nz = P->d.n[2];
-    const int64_t cells = (int64_t)nx * ny * nz;
     double* a = P->work;
-    double* b = P->work + cells;
-    transform3(P, in, a, b, 1.0, s);                        // b = S in
+    double* b = P->work + (int64_t)nx * ny * nz;
     const double norm = (2.0 / (nx + 1)) * (2.0 / (ny + 1)) * (2.0 / (nz + 1));
-    hipLaunchKernelGGL(pp_poissonk::k_divide, dim3(blocks(cells)), dim3(256), 0, s, b, P->lam[0], P->lam[1], P->lam[2],
-                       nx, ny, nz, scale);                  // b = S in * scale / lambda
-    transform3(P, b, a, out, norm, s);                      // out = S b * prod 2/(n+1)
+    transform3(P, in, a, b, 1.0, scale, nullptr, s);        // b = S in * scale / lambda
+    transform3(P, b, a, out, norm, 0.0, type, s);           // out = S b * prod 2/(n+1)
 }
 
 // ---- electrode-bounded domains ------------------------------------------------------------------
@@ -650,6 +733,7 @@ static int build_operator(pp_poisson* P, char* err, size_t errn) {
     }
     // poisson_amg.py:293-444: Shortley-Weller rows (conductor rows become diagonal rows here)
     std::vector<double> coef((size_t)7 * N, 0.0);
+    std::vector<uint8_t> regular((size_t)N, 0);
     const double box_diag = (2.0 / (d.h[0] * d.h[0]) + 2.0 / (d.h[1] * d.h[1])) + 2.0 / (d.h[2] * d.h[2]);
     const int64_t stride[3] = {(int64_t)ny * nz, nz, 1};
     for (int i = 0; i < nx; ++i)
@@ -662,6 +746,7 @@ static int build_operator(pp_poisson* P, char* err, size_t errn) {
                 }
                 const int ijk[3] = {i, j, k};
                 double diag = 0.0;
+                bool plain = true;
                 for (int a = 0; a < 3; ++a) {
                     const double h = d.h[a];
                     const bool has_p = ijk[a] + 1 < d.n[a], has_m = ijk[a] > 0;
@@ -669,17 +754,25 @@ static int build_operator(pp_poisson* P, char* err, size_t errn) {
                     const bool cond_m = has_m && P->h_type[(size_t)(t - stride[a])] == 2;
                     const double hp = cond_p ? std::max(P->h_dist[(size_t)t * 6 + 2 * a], h * 1e-3) : h;
                     const double hm = cond_m ? std::max(P->h_dist[(size_t)t * 6 + 2 * a + 1], h * 1e-3) : h;
+                    plain = plain && !cond_p && !cond_m;
                     diag += 2.0 / (hp * hm);
                     if (has_p && !cond_p) coef[(size_t)(1 + 2 * a) * N + t] = -2.0 / (hp * (hp + hm));
                     if (has_m && !cond_m) coef[(size_t)(2 + 2 * a) * N + t] = -2.0 / (hm * (hp + hm));
                 }
                 coef[(size_t)t] = diag;
+                regular[(size_t)t] = plain ? 1 : 0;
+                if (plain) P->box[0] = diag;
             }
+    for (int a = 0; a < 3; ++a) P->box[1 + a] = -2.0 / (d.h[a] * (d.h[a] + d.h[a]));
     const bool ok = hipMalloc(&P->type, sizeof(int32_t) * N) == hipSuccess &&
                     hipMalloc(&P->coef, sizeof(double) * 7 * N) == hipSuccess &&
                     hipMalloc(&P->vec, sizeof(double) * 9 * N) == hipSuccess &&
-                    hipMalloc(&P->part, sizeof(double) * 3 * pp_poissonk::kDotBlocks) == hipSuccess &&
+                    hipMalloc(&P->regular, (size_t)N) == hipSuccess &&
+                    hipMemcpy(P->regular, regular.data(), (size_t)N, hipMemcpyHostToDevice) == hipSuccess &&
+                    hipMalloc(&P->part, sizeof(double) * 2 * pp_poissonk::kDotBlocks) == hipSuccess &&
                     hipMalloc(&P->sc, sizeof(double) * pp_poissonk::kScalars) == hipSuccess &&
+                    hipHostMalloc(reinterpret_cast<void**>(&P->host), sizeof(double) * 8, hipHostMallocDefault) ==
+                        hipSuccess &&
                     hipMemcpy(P->type, P->h_type.data(), sizeof(int32_t) * N, hipMemcpyHostToDevice) == hipSuccess &&
                     hipMemcpy(P->coef, coef.data(), sizeof(double) * 7 * N, hipMemcpyHostToDevice) == hipSuccess;
     if (!ok) {
@@ -712,12 +805,14 @@ void stats(const pp_poisson* P, int32_t* iterations, double* residual) {
 // BiCGSTAB with right preconditioning, for A phi = rho / eps0 with the Shortley-Weller rows.  The
 // preconditioner is the box solve with its result set to 0 on conductor nodes, so every iterate is 0 there
 // (and the residual too, since conductor rows are diagonal with b = 0); it starts from that preconditioned b.
-// Reads one residual norm per iteration to the host.
+// An iteration is 18 launches (it was 32), the dot products inside the passes that have their vectors at hand.  The
+// host waits for the residual of one iteration while the next one is enqueued already: that one changes nothing once
+// the device has found the tolerance reached.
 static hipError_t solve_conductors(const pp_poisson* P, const double* rho, double* phi, hipStream_t s) {
     using namespace pp_poissonk;
     const PoissonDesc& d = P->d;
     const int64_t N = (int64_t)d.n[0] * d.n[1] * d.n[2];
-    const unsigned g = blocks(N);
+    const unsigned g = blocks(N), gd = g < (unsigned)kDotBlocks ? g : (unsigned)kDotBlocks;
     double* x = phi;
     double* r = P->vec;
     double* r0 = P->vec + N;
@@ -730,71 +825,66 @@ static hipError_t solve_conductors(const pp_poisson* P, const double* rho, doubl
     double* b = P->vec + 8 * N;
     SwOperator A;
     for (int q = 0; q < 7; ++q) A.coef[q] = P->coef + (size_t)q * N;
+    A.regular = P->regular;
+    for (int q = 0; q < 4; ++q) A.box[q] = P->box[q];
     A.nx = d.n[0];
     A.ny = d.n[1];
     A.nz = d.n[2];
-    auto dots = [&](const double* a0, const double* b0, const double* a1, const double* b1, const double* a2,
-                    const double* b2, int nq, int slot) {
-        Dots D{{a0, a1, a2}, {b0, b1, b2}, nq};
-        hipLaunchKernelGGL(k_dots, dim3(kDotBlocks), dim3(256), 0, s, D, N, P->part);
-        hipLaunchKernelGGL(k_dots_finish, dim3(1), dim3(256), 0, s, P->part, nq, P->sc, slot);
+    double* host_dev = nullptr;
+    hipError_t e = hipHostGetDevicePointer(reinterpret_cast<void**>(&host_dev), P->host, 0);
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    for (int k = 0; k < 2 && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+    auto scalars = [&](int stage, int slot) {
+        hipLaunchKernelGGL(k_scalars, dim3(1), dim3(256), 0, s, P->part, (int)gd, stage, P->rtol, P->sc,
+                           slot < 0 ? nullptr : host_dev + 4 * slot);
     };
-    auto upd = [&](int which, double* u0, double* u1, const double* w0, const double* w1, const double* w2,
-                   const double* w3) {
-        hipLaunchKernelGGL(k_bicg_update, dim3(g), dim3(256), 0, s, which, N, P->sc, u0, u1, w0, w1, w2, w3);
+    auto wait = [&](int slot) {     // true: go on
+        if (e == hipSuccess) e = hipEventSynchronize(ev[slot]);
+        return e == hipSuccess && P->host[4 * slot + 1] == 0.0;
     };
-    auto precond = [&](const double* in, double* out) {
-        box_inverse(P, in, out, 1.0, s);
-        hipLaunchKernelGGL(k_mask, dim3(g), dim3(256), 0, s, 1, N, P->type, nullptr, out);
-    };
-    hipLaunchKernelGGL(k_mask, dim3(g), dim3(256), 0, s, 0, N, P->type, rho, b);     // b = rho / eps0, 0 on conductors
-    precond(b, x);                                                                  // x0 = K^-1 b
-    hipLaunchKernelGGL(k_sw_apply, dim3(g), dim3(256), 0, s, A, x, r);
-    upd(3, r, nullptr, b, nullptr, nullptr, nullptr);                               // r = b - A x0
-    upd(4, r0, nullptr, r, nullptr, nullptr, nullptr);
-    upd(4, p, nullptr, r, nullptr, nullptr, nullptr);
-    upd(5, v, nullptr, nullptr, nullptr, nullptr, nullptr);                         // v = 0
-    hipLaunchKernelGGL(k_scalars, dim3(1), dim3(64), 0, s, P->sc, 0);
-    dots(b, b, r, r, nullptr, nullptr, 2, kBB);
-    double host[2];
-    hipError_t e = hipMemcpyAsync(host, P->sc + kBB, sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(host + 1, P->sc + kRR, sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return e;
-    const double bnorm = std::sqrt(host[0]);
-    double res = bnorm > 0.0 ? std::sqrt(host[1]) / bnorm : 0.0;
-    int it = 0;
-    while (res > P->rtol && it < P->max_iter) {
-        dots(r0, r, nullptr, nullptr, nullptr, nullptr, 1, kRho);
-        hipLaunchKernelGGL(k_scalars, dim3(1), dim3(64), 0, s, P->sc, 1);
-        if (it > 0) upd(0, p, nullptr, r, v, nullptr, nullptr);                     // p = r + beta (p - omega v)
-        precond(p, ph);
-        hipLaunchKernelGGL(k_sw_apply, dim3(g), dim3(256), 0, s, A, ph, v);
-        dots(r0, v, nullptr, nullptr, nullptr, nullptr, 1, kR0V);
-        hipLaunchKernelGGL(k_scalars, dim3(1), dim3(64), 0, s, P->sc, 2);
-        upd(1, sv, nullptr, r, v, nullptr, nullptr);                                 // s = r - alpha v
-        precond(sv, sh);
-        hipLaunchKernelGGL(k_sw_apply, dim3(g), dim3(256), 0, s, A, sh, tv);
-        dots(tv, sv, tv, tv, nullptr, nullptr, 2, kTS);
-        hipLaunchKernelGGL(k_scalars, dim3(1), dim3(64), 0, s, P->sc, 3);
-        upd(2, x, r, ph, sh, sv, tv);                                               // x += alpha ph + omega sh; r = s - omega t
-        dots(r, r, nullptr, nullptr, nullptr, nullptr, 1, kRR);
-        e = hipMemcpyAsync(host + 1, P->sc + kRR, sizeof(double), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return e;
-        res = std::sqrt(host[1]) / bnorm;
-        ++it;
-        if (!(res == res)) break;                                                   // breakdown (NaN)
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_mask, dim3(g), dim3(256), 0, s, 0, N, P->type, rho, b);    // b = rho / eps0, 0 on conductors
+        box_inverse(P, b, x, 1.0, P->type, s);                                          // x0 = K^-1 b
+        hipLaunchKernelGGL(k_sw_start, dim3(gd), dim3(256), 0, s, A, x, b, r, r0, p, P->part);
+        scalars(0, 0);
+        e = hipEventRecord(ev[0], s);
+        bool more = wait(0);
+        for (int it = 0; more && it < P->max_iter; ++it) {
+            const int slot = (it + 1) & 1;
+            if (it > 0) hipLaunchKernelGGL(k_bicg_p, dim3(g), dim3(256), 0, s, N, P->sc, p, r, v);
+            box_inverse(P, p, ph, 1.0, P->type, s);
+            hipLaunchKernelGGL(k_sw_apply, dim3(gd), dim3(256), 0, s, A, ph, v, r0, P->part);
+            scalars(1, -1);
+            hipLaunchKernelGGL(k_bicg_s, dim3(g), dim3(256), 0, s, N, P->sc, sv, r, v);
+            box_inverse(P, sv, sh, 1.0, P->type, s);
+            hipLaunchKernelGGL(k_sw_apply, dim3(gd), dim3(256), 0, s, A, sh, tv, sv, P->part);
+            scalars(2, -1);
+            hipLaunchKernelGGL(k_bicg_x, dim3(gd), dim3(256), 0, s, N, P->sc, x, r, ph, sh, sv, tv, r0, P->part);
+            scalars(3, slot);
+            if (e == hipSuccess) e = hipEventRecord(ev[slot], s);
+            more = it == 0 ? e == hipSuccess : wait(slot ^ 1);      // the iteration before this one
+        }
     }
-    hipLaunchKernelGGL(k_mask, dim3(g), dim3(256), 0, s, 1, N, P->type, nullptr, x);  // phi = 0 on conductors
-    P->last_iter = it;
-    P->last_res = res;
-    return hipGetLastError();
+    const hipError_t se = hipStreamSynchronize(s);      // whatever is enqueued still writes the slots
+    if (e == hipSuccess) e = se;
+    if (e == hipSuccess) {
+        double sc[kScalars];
+        e = hipMemcpyAsync(sc, P->sc, sizeof(sc), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e == hipSuccess) {
+            P->last_iter = (int)sc[kIter];
+            P->last_res = sc[kRes];
+            hipLaunchKernelGGL(k_mask, dim3(g), dim3(256), 0, s, 1, N, P->type, nullptr, x);   // phi = 0 on conductors
+        }
+    }
+    for (hipEvent_t q : ev)
+        if (q) (void)hipEventDestroy(q);
+    return e == hipSuccess ? hipGetLastError() : e;
 }
 
 hipError_t solve(const pp_poisson* P, const double* rho, double* phi, hipStream_t s) {
     if (P->coef) return solve_conductors(P, rho, phi, s);
-    box_inverse(P, rho, phi, 1.0 / kEps0, s);
+    box_inverse(P, rho, phi, 1.0 / kEps0, nullptr, s);
     return hipGetLastError();
 }
 
