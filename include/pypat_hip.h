@@ -238,6 +238,11 @@ int pp_spline_eval(const pp_spline* s, const double* pts, int64_t m, int32_t str
 /* Fused multi-step push: Pusher.track_batch step loop (pusher.py:966-990) /
    push_batch (pusher.py:699-801) when nsteps == 1. */
 int pp_push(const pp_push_args* args, pp_stream s);
+/* One push of a few particles held in host arrays: r, v (n, 3) in, r_out, v_out (n, 3) out (velocities also for the
+   u-state algorithms), n <= PP_PUSH_ROWS_MAX.  args: as for pp_push, on the library's stream; the state pointers, ids,
+   alive, dt_pp, histories and kick_only are not used (null / 0).  Blocking. */
+#define PP_PUSH_ROWS_MAX 8192
+int pp_push_rows(const pp_push_args* args, const double* r, const double* v, double* r_out, double* v_out);
 /* pp_push through fields that are sums of terms, E (or B) = sum_k weight_k term_k accumulated from zero in the
    given order: CompositeField.__call__ (field.py:621-645) inside the step loop, so a track through an external
    map plus a self-field map on another grid needs no field arrays.  terms: host array of 1..PP_MAX_SUM_TERMS

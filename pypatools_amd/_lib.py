@@ -65,6 +65,7 @@ class PPBunch(ctypes.Structure):
     ]
 
 
+PUSH_ROWS_MAX = 8192
 MAX_SUM_TERMS = 6                                # include/pypat_hip.h PP_MAX_SUM_TERMS
 SUM_TO_B, SUM_PLAIN, SUM_SAME_CELL = 1, 2, 4     # pp_sum_flags
 SPLINE_NEAREST_MODE, SPLINE_RGI = 1, 2          # pp_spline_flags
@@ -131,6 +132,7 @@ SIGNATURES = {
     "pp_memcpy_h2d_async": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
     "pp_memcpy_d2h_pair": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, c_void_p, c_void_p, ctypes.c_size_t,
                                      c_void_p]),
+    "pp_push_rows": (c_int32, [ctypes.POINTER(PPPushArgs), c_void_p, c_void_p, c_void_p, c_void_p]),
     "pp_release_staging": (c_int32, []),
     "pp_memcpy_d2h_async": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
     "pp_event_query": (c_int32, [c_void_p, ctypes.POINTER(c_int32)]),

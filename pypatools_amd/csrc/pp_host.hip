@@ -159,10 +159,6 @@ int pp_memcpy_d2h_pair(void* dst0, const void* src0, size_t bytes0, void* dst1, 
     return PP_OK;
 }
 
-int pp_release_staging(void) {
-    pp_copy::release();
-    return PP_OK;
-}
 
 int pp_memcpy_d2d(void* dst, const void* src, size_t bytes, pp_stream s) {
     if (!bytes) return PP_OK;
@@ -726,6 +722,100 @@ static int push_impl(const pp_push_args* a, const pp_mesh* mesh, const pp_sum_te
     else
         e = pp_fast::launch_push(a->algorithm, a->precision, p, a->block_size, stream_of(s));
     if (e != hipSuccess) return hip_fail(e, "push launch");
+    return PP_OK;
+}
+
+// Memory of one small push in flight: 12 n doubles of mapped pinned memory (rows in and out) and the state's 6 n on the
+// device.  At most kRowSets are kept (1.2 MB each), given back by pp_release_staging; further callers allocate their own
+// for the call.
+struct RowSet {
+    double* host;
+    double* dev;
+    int device;
+};
+constexpr int kRowSets = 4;
+static std::mutex g_rows_mu;
+static RowSet g_rows[kRowSets];
+static int g_nrows = 0;
+
+static void free_row_set(RowSet& q) {
+    if (q.host) (void)hipHostFree(q.host);
+    if (q.dev) (void)hipFree(q.dev);
+}
+
+static int take_row_set(RowSet& q) {
+    {
+        std::lock_guard<std::mutex> lk(g_rows_mu);
+        for (int k = 0; k < g_nrows; ++k)
+            if (g_rows[k].device == g_device) {
+                q = g_rows[k];
+                g_rows[k] = g_rows[--g_nrows];
+                return PP_OK;
+            }
+    }
+    q = {nullptr, nullptr, g_device};
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&q.host), sizeof(double) * 12 * PP_PUSH_ROWS_MAX,
+                                 hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&q.dev), sizeof(double) * 6 * PP_PUSH_ROWS_MAX);
+    if (e != hipSuccess) {
+        free_row_set(q);
+        return hip_fail(e, "row buffers");
+    }
+    return PP_OK;
+}
+
+static void put_row_set(RowSet& q) {
+    {
+        std::lock_guard<std::mutex> lk(g_rows_mu);
+        if (g_nrows < kRowSets) {
+            g_rows[g_nrows++] = q;
+            return;
+        }
+    }
+    free_row_set(q);
+}
+
+// A push of one particle is all latency: six arrays allocated and freed, four copies with a wait each, four layout
+// kernels and the push took 175 us.  Here the rows go through mapped pinned memory, which the two layout kernels read
+// and write themselves: three launches and one wait, 31 us a call (the push itself 7).
+int pp_push_rows(const pp_push_args* a, const double* r, const double* v, double* r_out, double* v_out) {
+    int rc = ensure_init();
+    if (rc) return rc;
+    if (!a || !r || !v || !r_out || !v_out) return fail(PP_ERR_INVALID, "null argument");
+    if (a->n < 0 || a->n > PP_PUSH_ROWS_MAX)
+        return fail(PP_ERR_INVALID, "pp_push_rows takes at most %d particles", PP_PUSH_ROWS_MAX);
+    if (a->x || a->y || a->z || a->vx || a->vy || a->vz || a->ids || a->alive || a->dt_pp || a->r_hist || a->v_hist ||
+        a->kick_only)
+        return fail(PP_ERR_INVALID, "pp_push_rows takes no state, ids, mask, dt_pp, histories or kick");
+    if (a->n == 0) return PP_OK;
+    const int64_t n = a->n;
+    const bool ustate = a->algorithm == PP_ALG_BORIS_REL || a->algorithm == PP_ALG_VAY;
+    RowSet q;
+    if ((rc = take_row_set(q))) return rc;
+    double* rows = nullptr;
+    hipError_t e = hipHostGetDevicePointer(reinterpret_cast<void**>(&rows), q.host, 0);
+    const pp_strict::StateView st = {q.dev, q.dev + n, q.dev + 2 * n, q.dev + 3 * n, q.dev + 4 * n, q.dev + 5 * n};
+    const size_t bytes = sizeof(double) * 3 * n;
+    memcpy(q.host, r, bytes);
+    memcpy(q.host + 3 * n, v, bytes);
+    const double c2 = kClight * kClight;
+    if (e == hipSuccess) e = pp_strict::launch_rows_to_state(rows, st, n, ustate, c2, g_stream);
+    if (e == hipSuccess) {
+        pp_push_args p = *a;
+        p.x = st.x; p.y = st.y; p.z = st.z;
+        p.vx = st.vx; p.vy = st.vy; p.vz = st.vz;
+        rc = push_impl(&p, nullptr, nullptr, 0, nullptr);
+    }
+    if (e == hipSuccess && !rc) e = pp_strict::launch_state_to_rows(st, rows + 6 * n, n, ustate, c2, g_stream);
+    const hipError_t se = hipStreamSynchronize(g_stream);     // also after a failure: the set is reused
+    if (e == hipSuccess) e = se;
+    if (e == hipSuccess && !rc) {
+        memcpy(r_out, q.host + 6 * n, bytes);
+        memcpy(v_out, q.host + 9 * n, bytes);
+    }
+    put_row_set(q);
+    if (rc) return rc;
+    if (e != hipSuccess) return hip_fail(e, "push of rows");
     return PP_OK;
 }
 
@@ -1374,6 +1464,13 @@ int pp_bunch_v_to_u(double* vx, double* vy, double* vz, const pp_bunch* bunches,
 
 int pp_u_to_v(double* ux, double* uy, double* uz, int64_t m, pp_stream s) {
     return util_common(PP_UT_U2V, ux, uy, uz, nullptr, m, s);
+}
+
+int pp_release_staging(void) {
+    pp_copy::release();
+    std::lock_guard<std::mutex> lk(g_rows_mu);
+    while (g_nrows > 0) free_row_set(g_rows[--g_nrows]);
+    return PP_OK;
 }
 
 }  // extern "C"

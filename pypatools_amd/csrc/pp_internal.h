@@ -168,6 +168,13 @@ hipError_t launch_velocity_rows(const double* vx, const double* vy, const double
                                 hipStream_t s);
 hipError_t launch_velocity_convert(double* vx, double* vy, double* vz, const pp_bunch* bunches, const int32_t* group,
                                    int64_t n, double c2, hipStream_t s);
+// rows: positions (n, 3), then velocities (n, 3)
+struct StateView {
+    double *x, *y, *z, *vx, *vy, *vz;
+};
+hipError_t launch_rows_to_state(const double* rows, const StateView& st, int64_t n, bool ustate, double c2,
+                                hipStream_t s);
+hipError_t launch_state_to_rows(const StateView& st, double* rows, int64_t n, bool ustate, double c2, hipStream_t s);
 hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s);
 hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s);
 hipError_t launch_interleave(const double* src, const MapDesc& d, double* raw, hipStream_t s);
@@ -212,7 +219,7 @@ constexpr int kMomentBlocks = 1024;   // partials per reduction pass
 // spline interpolators (pp_spline.hip)
 namespace pp_splk {
 struct SplineDesc {
-    const double* coef;        // [ncomp][N0][N1][N2], last axis fastest (N = n + 2 pad)
+    const double* coef;        // [N0][N1][N2][ncomp] (N = n + 2 pad)
     const double* axis[3];     // node coordinates, n[a] each
     int64_t n[3];              // nodes per axis (1 for unused axes)
     int64_t N[3];              // coefficient extent per axis

@@ -114,6 +114,37 @@ __global__ void __launch_bounds__(256) k_velocity_convert(double* vx, double* vy
     vz[i] = u.z;
 }
 
+// Host rows (mapped pinned memory) to state slots, v as u where ustate; and state slots back to host rows.
+__global__ void __launch_bounds__(64) k_rows_to_state(const double* __restrict__ rows, StateView st, int64_t n, int ustate,
+                                                      double c2) {
+    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (i >= n) return;
+    const d3 r = load3(rows, i);
+    d3 v = load3(rows + 3 * n, i);
+    if (ustate) v = rgamma(v, c2) * v;
+    st.x[i] = r.x;
+    st.y[i] = r.y;
+    st.z[i] = r.z;
+    st.vx[i] = v.x;
+    st.vy[i] = v.y;
+    st.vz[i] = v.z;
+}
+
+__global__ void __launch_bounds__(64) k_state_to_rows(StateView st, double* __restrict__ rows, int64_t n, int ustate,
+                                                      double c2) {
+    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (i >= n) return;
+    d3 v = mk3(st.vx[i], st.vy[i], st.vz[i]);
+    if (ustate) v = v_from_u(v, c2);
+    rows[3 * i] = st.x[i];
+    rows[3 * i + 1] = st.y[i];
+    rows[3 * i + 2] = st.z[i];
+    double* w = rows + 3 * n;
+    w[3 * i] = v.x;
+    w[3 * i + 1] = v.y;
+    w[3 * i + 2] = v.z;
+}
+
 __global__ void k_add_i64(int64_t* p, int64_t v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *p += v;
 }
@@ -465,6 +496,17 @@ hipError_t launch_velocity_rows(const double* vx, const double* vy, const double
 hipError_t launch_velocity_convert(double* vx, double* vy, double* vz, const pp_bunch* bunches, const int32_t* group,
                                    int64_t n, double c2, hipStream_t s) {
     hipLaunchKernelGGL(k_velocity_convert, dim3(grid_for(n, 256)), dim3(256), 0, s, vx, vy, vz, bunches, group, n, c2);
+    return hipGetLastError();
+}
+
+hipError_t launch_rows_to_state(const double* rows, const StateView& st, int64_t n, bool ustate, double c2,
+                                hipStream_t s) {
+    hipLaunchKernelGGL(k_rows_to_state, dim3(grid_for(n, 64)), dim3(64), 0, s, rows, st, n, ustate ? 1 : 0, c2);
+    return hipGetLastError();
+}
+
+hipError_t launch_state_to_rows(const StateView& st, double* rows, int64_t n, bool ustate, double c2, hipStream_t s) {
+    hipLaunchKernelGGL(k_state_to_rows, dim3(grid_for(n, 64)), dim3(64), 0, s, st, rows, n, ustate ? 1 : 0, c2);
     return hipGetLastError();
 }
 

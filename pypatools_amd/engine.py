@@ -21,7 +21,7 @@ import numpy as np
 from . import _lib
 from .device import DeviceArray, to_host_pair
 from .field import (CompositeField, Field, RFField, ScaledField, compile_sum, compile_term, evaluate_on_device,
-                    is_time_dependent, rf_source)
+                    is_time_dependent, rf_source, same_nodes)
 from .interpolators import DeviceFieldMap
 
 REFERENCE_ALGORITHMS = ["leapfrog", "boris", "rk4", "yoshida", "vay_rel", "rk4_rel", "yoshida_rel"]
@@ -187,7 +187,7 @@ def _fused_map(fe, fb, fp64=True):
     se, sb = be._grid_source(), bb._grid_source()
     if se is None or sb is None or se[2] != sb[2] or len(se[0]) != len(sb[0]):
         return None
-    if not all(np.array_equal(a, b) for a, b in zip(se[0], sb[0])):
+    if not all(same_nodes(a, b) for a, b in zip(se[0], sb[0])):
         return None
     key = (id(be), id(bb), bool(fp64))
     hit = _FUSED_CACHE.get(key)
@@ -203,7 +203,8 @@ class FieldPair:
 
     def __init__(self, efield, bfield):
         self.efield, self.bfield = efield, bfield
-        self.tE, self.tB = compile_term(efield), compile_term(bfield)
+        # maps of their own are built only where E and B do not share a fused one
+        self.tE, self.tB = compile_term(efield, False), compile_term(bfield, False)
         self.direct = self.tE is not None and self.tB is not None
         self.time_dependent = is_time_dependent(efield) or is_time_dependent(bfield)
         self.map = None
@@ -215,6 +216,11 @@ class FieldPair:
                 self.tE.comp0 = 0
                 self.tB.map = fm.handle
                 self.tB.comp0 = 3
+        if self.map is None:
+            if self.tE is not None:
+                self.tE = compile_term(efield)
+            if self.tB is not None:
+                self.tB = compile_term(bfield)
         # fields that are sums of direct terms: pp_push_sum evaluates them inside the step loop
         self.sum = None if self.direct else compile_sum(efield, bfield)
 
@@ -419,8 +425,10 @@ class Tracker:
         v = np.ascontiguousarray(v, dtype=np.float64).reshape(-1, 3)
         if r.shape[0] == 0:
             return r.copy(), v.copy()
-        st = ParticleState.from_host(r, v)
         fp = FieldPair(efield, bfield)
+        if dt_pp is None and fp.direct and r.shape == v.shape and r.shape[0] <= _lib.PUSH_ROWS_MAX:
+            return self._push_rows(r, v, fp, dt, t)
+        st = ParticleState.from_host(r, v)
         dtp = DeviceArray.from_host(np.asarray(dt_pp, dtype=np.float64)) if dt_pp is not None else None
         ustate = self.algorithm in U_STATE
         if ustate:
@@ -436,6 +444,24 @@ class Tracker:
         if ustate:
             st.u_to_v()
         return st.to_host()
+
+    def _push_rows(self, r, v, fp, dt, t):
+        """single_step of a few particles: their rows go through mapped host memory (pp_push_rows)."""
+        a = _lib.PPPushArgs()
+        a.algorithm = _lib.ALG_IDS[self.algorithm]
+        a.precision = _lib.PRECISIONS[self.precision]
+        a.n = r.shape[0]
+        a.dt = float(dt)
+        a.q_over_m = self.qm
+        a.nsteps = 1
+        a.efield, a.bfield = fp.tE, fp.tB
+        rf = self._rf(fp, t, dt, 1)
+        if rf is not None:
+            a.rf_table, a.rf_step0, a.rf_nsteps = rf[0].ptr, rf[1], rf[2]
+        a.block_size = self.block_size
+        rn, vn = np.empty_like(r), np.empty_like(v)
+        _lib.call("pp_push_rows", a, r.ctypes.data, v.ctypes.data, rn.ctypes.data, vn.ctypes.data)
+        return rn, vn
 
     def _velocity_record(self, st, out_aos, ustate, live_only=False):
         alive = st.alive.ptr if live_only and st.alive is not None else None

@@ -241,7 +241,7 @@ class Field(FieldBase):
             return None
         g0 = comps[0].grid
         for c in comps[1:]:
-            if len(c.grid) != len(g0) or not all(np.array_equal(a, b) for a, b in zip(c.grid, g0)):
+            if len(c.grid) != len(g0) or not all(same_nodes(a, b) for a, b in zip(c.grid, g0)):
                 return None
         return comps
 
@@ -268,7 +268,7 @@ class Field(FieldBase):
             self._dev_map = DeviceFieldMap(src[0], src[1], 0.0, src[2])
         return self._dev_map
 
-    def _term(self):
+    def _term(self, with_map=True):
         """The device term of this field (PPField), or None if it needs per-component evaluation."""
         t = _lib.PPField()
         t.scale1 = 1.0
@@ -283,7 +283,8 @@ class Field(FieldBase):
         if self._grid_source() is None:
             return None
         t.kind = _lib.FIELD_MAP
-        t.map = self.device_map().handle
+        if with_map:
+            t.map = self.device_map().handle
         t.comp0 = 0
         t.scale1 = float(self._scaling)
         return t
@@ -394,17 +395,22 @@ def _precision_of(f):
     return "fp64"
 
 
-def compile_term(f):
-    """A PPField the push kernels read directly, or None.
+def same_nodes(a, b):
+    """Equal node arrays (components of a map usually hold the same array objects)."""
+    return a is b or np.array_equal(a, b)
+
+
+def compile_term(f, with_map=True):
+    """A PPField the push kernels read directly, or None (with_map=False: map terms without their device map).
 
     Field                      -> CONST / MAP term (scale1 = Field.scaling)
     ScaledField(Field)         -> same term with scale2 / offset
     RFField(Field or Scaled)   -> same term with the cos/sin column of the rf table
     """
     if isinstance(f, Field):
-        return f._term()
+        return f._term(with_map)
     if isinstance(f, ScaledField) and isinstance(f.field, Field):
-        t = f.field._term()
+        t = f.field._term(with_map)
         if t is None:
             return None
         t.scale2 = float(f.scale)
@@ -413,7 +419,7 @@ def compile_term(f):
         t.has_offset = 1
         return t
     if isinstance(f, RFField):
-        t = compile_term(f.field)
+        t = compile_term(f.field, with_map)
         if t is None or t.rf != _lib.RF_NONE:
             return None
         t.rf = _lib.RF_COS if f.mode == "cos" else _lib.RF_SIN
@@ -471,7 +477,7 @@ def compile_sum(efield, bfield):
 
     def same(a, b):
         return (a is not None and b is not None and a[2] == b[2] and len(a[0]) == len(b[0])
-                and all(np.array_equal(u, v) for u, v in zip(a[0], b[0])))
+                and all(same_nodes(u, v) for u, v in zip(a[0], b[0])))
 
     # B's first term follows the first E term on its grid: both then share one cell lookup
     nb = sum(1 for e in listed if e[2] & _lib.SUM_TO_B)
