@@ -203,6 +203,11 @@ int pp_event_sync(pp_event e);
 int pp_map_create(const double* values, int32_t ncomp, int32_t nx, int32_t ny, int32_t nz,
                   const double* gx, const double* gy, const double* gz, double fill_value, int32_t flags,
                   pp_map** out);
+/* The same from one (nx, ny, nz) grid per component, in host memory or (on_device) in device memory, there on the
+   library's stream. */
+int pp_map_create_parts(const double* const* parts, int32_t on_device, int32_t ncomp, int32_t nx, int32_t ny, int32_t nz,
+                        const double* gx, const double* gy, const double* gz, double fill_value, int32_t flags,
+                        pp_map** out);
 int pp_map_destroy(pp_map* map);
 int pp_map_bytes(const pp_map* map, size_t* bytes);
 

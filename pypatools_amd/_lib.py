@@ -137,6 +137,8 @@ SIGNATURES = {
     "pp_memcpy_d2h_async": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
     "pp_event_query": (c_int32, [c_void_p, ctypes.POINTER(c_int32)]),
     "pp_event_sync": (c_int32, [c_void_p]),
+    "pp_map_create_parts": (c_int32, [ctypes.POINTER(c_void_p), c_int32, c_int32, c_int32, c_int32, c_int32, c_void_p,
+                                      c_void_p, c_void_p, ctypes.c_double, c_int32, ctypes.POINTER(c_void_p)]),
     "pp_map_create": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_void_p,
                                 ctypes.c_double, c_int32, ctypes.POINTER(c_void_p)]),
     "pp_map_destroy": (c_int32, [c_void_p]),

@@ -297,11 +297,20 @@ static int map_alloc(pp_map* m, size_t bytes, void** out) {
 
 int pp_map_create(const double* values, int32_t ncomp, int32_t nx, int32_t ny, int32_t nz, const double* gx,
                   const double* gy, const double* gz, double fill_value, int32_t flags, pp_map** out) {
+    const double* parts[6] = {};
+    if (values && ncomp >= 1 && ncomp <= 6 && nx >= 1 && ny >= 1 && nz >= 1)
+        for (int c = 0; c < ncomp; ++c) parts[c] = values + (int64_t)c * nx * ny * nz;
+    return pp_map_create_parts(values ? parts : nullptr, 0, ncomp, nx, ny, nz, gx, gy, gz, fill_value, flags, out);
+}
+
+int pp_map_create_parts(const double* const* parts, int32_t on_device, int32_t ncomp, int32_t nx, int32_t ny, int32_t nz,
+                        const double* gx, const double* gy, const double* gz, double fill_value, int32_t flags,
+                        pp_map** out) {
     int rc = ensure_init();
     if (rc) return rc;
     if (!out) return fail(PP_ERR_INVALID, "null output handle");
     *out = nullptr;
-    if (!values || !gx || !gy || !gz) return fail(PP_ERR_INVALID, "null map input");
+    if (!parts || !gx || !gy || !gz) return fail(PP_ERR_INVALID, "null map input");
     if (ncomp < 1 || ncomp > 6) return fail(PP_ERR_INVALID, "ncomp must be 1..6, got %d", ncomp);
     const int32_t n[3] = {nx, ny, nz};
     const double* g[3] = {gx, gy, gz};
@@ -314,6 +323,8 @@ int pp_map_create(const double* values, int32_t ncomp, int32_t nx, int32_t ny, i
     const bool periodic = (flags & PP_MAP_PERIODIC_Z) != 0;
     if (periodic && nz < 2) return fail(PP_ERR_INVALID, "periodic z needs at least 2 z nodes");
     if ((int64_t)nx * ny * nz > (int64_t)1 << 31) return fail(PP_ERR_INVALID, "map too large");
+    for (int c = 0; c < ncomp; ++c)
+        if (!parts[c]) return fail(PP_ERR_INVALID, "component %d is null", c);
 
     pp_map* m = new pp_map();
     memset(m, 0, sizeof(*m));
@@ -363,15 +374,25 @@ int pp_map_create(const double* values, int32_t ncomp, int32_t nx, int32_t ny, i
     }
     if ((rc = map_alloc(m, sizeof(double) * nodes * ncomp, &p))) { pp_map_destroy(m); return rc; }
     d.raw = static_cast<const double*>(p);
-    const size_t src_bytes = sizeof(double) * (size_t)nx * ny * nz * ncomp;
-    void* src = nullptr;
-    hipError_t ue = hipMalloc(&src, src_bytes);
-    if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "hipMalloc (field map)"); }
-    const pp_copy::Region up = {const_cast<double*>(values), src, src_bytes};
-    ue = pp_copy::transfer(&up, 1, false, g_device, s);
-    if (ue == hipSuccess) ue = pp_strict::launch_interleave(static_cast<const double*>(src), d, static_cast<double*>(p), s);
-    if (ue == hipSuccess) ue = hipStreamSynchronize(s);
-    (void)hipFree(src);
+    const size_t part = (size_t)nx * ny * nz;
+    MapParts src = {};
+    void* tmp = nullptr;
+    hipError_t ue = hipSuccess;
+    if (on_device) {
+        for (int c = 0; c < ncomp; ++c) src.comp[c] = parts[c];
+    } else {
+        ue = hipMalloc(&tmp, sizeof(double) * part * ncomp);
+        if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "hipMalloc (field map)"); }
+        pp_copy::Region up[6];
+        for (int c = 0; c < ncomp; ++c) {
+            src.comp[c] = static_cast<double*>(tmp) + c * part;
+            up[c] = {const_cast<double*>(parts[c]), static_cast<double*>(tmp) + c * part, sizeof(double) * part};
+        }
+        ue = pp_copy::transfer(up, ncomp, false, g_device, s);
+    }
+    if (ue == hipSuccess) ue = pp_strict::launch_interleave(src, d, static_cast<double*>(p), s);
+    if (ue == hipSuccess && tmp) ue = hipStreamSynchronize(s);
+    if (tmp) (void)hipFree(tmp);
     if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "map upload"); }
     const int64_t ncell = (int64_t)d.nc[0] * d.nc[1] * d.nc[2];
     double* c64 = nullptr;

@@ -42,6 +42,11 @@ struct FieldDev {
     MapDesc map;
 };
 
+// device grids of a map's components
+struct MapParts {
+    const double* comp[6];
+};
+
 struct PushParams {
     int64_t n;
     double* x; double* y; double* z;
@@ -177,7 +182,7 @@ hipError_t launch_rows_to_state(const double* rows, const StateView& st, int64_t
 hipError_t launch_state_to_rows(const StateView& st, double* rows, int64_t n, bool ustate, double c2, hipStream_t s);
 hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s);
 hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s);
-hipError_t launch_interleave(const double* src, const MapDesc& d, double* raw, hipStream_t s);
+hipError_t launch_interleave(const MapParts& src, const MapDesc& d, double* raw, hipStream_t s);
 hipError_t launch_build_coef(const MapDesc& d, double* c64, float* c32, hipStream_t s);
 }  // namespace pp_strict
 

@@ -154,17 +154,16 @@ __global__ void __launch_bounds__(256) k_fill(double* p, double v, int64_t n) {
     if (i < n) p[i] = v;
 }
 
-// Node table [node][ncomp] from the components' grids src[comp][nx][ny][nz] (a periodic z axis gets node 0 again
+// Node table [node][ncomp] from the components' grids [nx][ny][nz] (a periodic z axis gets node 0 again
 // as its last).  Writes are contiguous; reads run along ncomp streams.
-__global__ void __launch_bounds__(256) k_interleave(const double* __restrict__ src, const MapDesc d,
-                                                    double* __restrict__ raw) {
+__global__ void __launch_bounds__(256) k_interleave(const MapParts src, const MapDesc d, double* __restrict__ raw) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t ngz = d.ng[2], nodes = (int64_t)d.ng[0] * d.ng[1] * ngz;
     if (t >= nodes * d.ncomp) return;
     const int64_t node = t / d.ncomp, comp = t - node * d.ncomp;
     const int64_t col = node / ngz, k = node - col * ngz;
     const int64_t nz = d.n[2];
-    raw[t] = src[(comp * d.n[0] * d.n[1] + col) * nz + (k < nz ? k : 0)];
+    raw[t] = src.comp[comp][col * nz + (k < nz ? k : 0)];
 }
 
 // Per-cell trilinear coefficients of every component from the raw node table.
@@ -520,7 +519,7 @@ hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_interleave(const double* src, const MapDesc& d, double* raw, hipStream_t s) {
+hipError_t launch_interleave(const MapParts& src, const MapDesc& d, double* raw, hipStream_t s) {
     const int64_t work = (int64_t)d.ng[0] * d.ng[1] * d.ng[2] * d.ncomp;
     hipLaunchKernelGGL(k_interleave, dim3(grid_for(work, 256)), dim3(256), 0, s, src, d, raw);
     return hipGetLastError();

@@ -93,7 +93,12 @@ class Field(FieldBase):
         if field is not None:
             self._field = field
         self._dev_map = None
+        self._dev_values = None         # (3, nodes) device copy of the component grids, where they come from the device
         self._dev_spline = None
+
+    def __getstate__(self):
+        # copies and pickles take the host grids; the device copy of them stays with its field
+        return {**self.__dict__, "_dev_values": None}
 
     # ---- core API ----------------------------------------------------------
     def __call__(self, pts):
@@ -265,7 +270,12 @@ class Field(FieldBase):
             src = self._grid_source()
             if src is None:
                 raise ValueError("field has no gridded components")
-            self._dev_map = DeviceFieldMap(src[0], src[1], 0.0, src[2])
+            if self._dev_values is not None:
+                n = self._dev_values.shape[1]
+                self._dev_map = DeviceFieldMap(src[0], [self._dev_values.view_ptr(k * n) for k in range(3)], 0.0, src[2])
+                self._dev_values = None
+            else:
+                self._dev_map = DeviceFieldMap(src[0], src[1], 0.0, src[2])
         return self._dev_map
 
     def _term(self, with_map=True):

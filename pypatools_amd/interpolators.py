@@ -40,15 +40,22 @@ def grid_to_axes(points):
 
 
 class DeviceFieldMap:
-    """A device map of ``ncomp`` components on one grid (pp_map_create)."""
+    """A device map of ``ncomp`` components on one grid (pp_map_create_parts); the components are arrays, or
+    addresses of device buffers of the grid's size."""
 
     def __init__(self, points, components, fill_value=0.0, periodic_z=False, fp32=True, coefficients=True,
                  fp64=True):
         axes = grid_to_axes(points)
         shape = tuple(len(a) for a in axes)
-        vals = np.empty((len(components),) + shape, dtype=np.float64)
+        on_device = all(isinstance(v, int) for v in components)
+        parts = (ctypes.c_void_p * len(components))()
+        keep = []
         for c, v in enumerate(components):
-            vals[c] = np.asarray(v, dtype=np.float64).reshape(shape)
+            if not on_device:
+                v = np.ascontiguousarray(np.asarray(v, dtype=np.float64).reshape(shape))
+                keep.append(v)
+                v = v.ctypes.data
+            parts[c] = v
         flags = 0
         if periodic_z:
             flags |= _lib.MAP_PERIODIC_Z
@@ -59,8 +66,7 @@ class DeviceFieldMap:
         if not fp64:
             flags |= _lib.MAP_NO_FP64
         h = ctypes.c_void_p()
-        vals = np.ascontiguousarray(vals)
-        _lib.call("pp_map_create", vals.ctypes.data, len(components), shape[0], shape[1], shape[2],
+        _lib.call("pp_map_create_parts", parts, 1 if on_device else 0, len(components), shape[0], shape[1], shape[2],
                   axes[0].ctypes.data, axes[1].ctypes.data, axes[2].ctypes.data, float(fill_value), flags,
                   ctypes.byref(h))
         self.handle = h.value

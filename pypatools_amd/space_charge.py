@@ -24,7 +24,7 @@ import warnings
 import numpy as np
 
 from . import _lib
-from .device import DeviceArray
+from .device import DeviceArray, to_host_pair
 
 
 INTERIOR, BOUNDARY, CONDUCTOR = 0, 1, 2       # poisson_amg.py:86-90
@@ -134,25 +134,36 @@ class SpaceChargeSolver:
         self._solve_rho()
         return self.phi.to_host().reshape(self.cells)
 
-    def _field(self):
+    def _potential_and_field(self):
+        """phi and the field on the host; the field keeps a device copy of its grids, from which its map is built."""
         from .field import Field
-        vals = {a: e.to_host().reshape(self.cells) for a, e in zip("xyz", self.E)}
-        return Field.from_arrays(self.grid(), vals, label=f"Space-charge E-field (turn {self.turn_count})", dim=3)
+        dev = DeviceArray((3, self.n_dofs))
+        for k, e in enumerate(self.E):
+            _lib.call("pp_memcpy_d2d", dev.view_ptr(k * self.n_dofs), e.ptr, e.nbytes, None)
+        phi, ex = to_host_pair(self.phi, self.E[0])
+        ey, ez = to_host_pair(self.E[1], self.E[2])
+        vals = {a: e.reshape(self.cells) for a, e in zip("xyz", (ex, ey, ez))}
+        E = Field.from_arrays(self.grid(), vals, label=f"Space-charge E-field (turn {self.turn_count})", dim=3)
+        E._dev_values = dev
+        return phi.reshape(self.cells), E
 
     def solve(self, particles, charges):
         """poisson_amg.py:616-797: (phi_3d, E_field) for positions (N, 3) [m] and charges (N,) [C]."""
-        p = np.ascontiguousarray(np.asarray(particles, dtype=np.float64).reshape(-1, 3).T)
+        p = np.ascontiguousarray(particles, dtype=np.float64).reshape(-1, 3)
         q = np.ascontiguousarray(charges, dtype=np.float64).reshape(-1)
-        n = p.shape[1]
+        n = p.shape[0]
         if q.shape[0] != n:
             raise ValueError("particles and charges differ in length")
-        dp = DeviceArray.from_host(p) if n else DeviceArray((3,))
+        rows = DeviceArray.from_host(p) if n else DeviceArray((3,))
+        dp = DeviceArray((3, max(n, 1)))
         dq = DeviceArray.from_host(q) if n else DeviceArray((1,))
+        if n:
+            _lib.call("pp_aos_to_soa", rows.ptr, n, dp.view_ptr(0), dp.view_ptr(n), dp.view_ptr(2 * n), None)
         self._solve_device(dp.view_ptr(0), dp.view_ptr(n), dp.view_ptr(2 * n), dq.ptr, 0.0, n)
-        return self.phi.to_host().reshape(self.cells), self._field()
+        return self._potential_and_field()
 
     def solve_state(self, state, charge_per_particle, alive=None):
         """The same from a device-resident ParticleState with one charge per particle (no host copy of the state)."""
         self._solve_device(state.x.ptr, state.y.ptr, state.z.ptr, None, charge_per_particle, state.n,
                            alive.ptr if alive is not None else None)
-        return self.phi.to_host().reshape(self.cells), self._field()
+        return self._potential_and_field()
