@@ -157,7 +157,8 @@ int pp_memcpy_d2h(void* dst, const void* src, size_t bytes, pp_stream s);
 /* Two device buffers to the host in one blocking call (their copies share the staging threads). */
 int pp_memcpy_d2h_pair(void* dst0, const void* src0, size_t bytes0, void* dst1, const void* src1, size_t bytes1,
                        pp_stream s);
-/* Frees the pinned staging buffers (at most 48 MiB) that large copies keep. */
+/* Frees what the library keeps between calls: pinned staging buffers (at most 48 MiB), row buffers of small pushes
+   (at most 5 MB) and freed device blocks (at most 1 GiB; pp_mem_info counts them as free). */
 int pp_release_staging(void);
 int pp_memcpy_d2d(void* dst, const void* src, size_t bytes, pp_stream s);
 int pp_fill_f64(double* dptr, double value, int64_t count, pp_stream s);   /* kernel fill, graph-safe */
