@@ -441,6 +441,8 @@ hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s) {
         PP_STRICT_CASES(false, kFieldsUniform)
     } else if (fields == kFieldsMap3d) {
         PP_STRICT_CASES(false, kFieldsMap3d)
+    } else if (fields == kFieldsMap3dRF) {
+        PP_STRICT_CASES(false, kFieldsMap3dRF)
     } else if (fields == kFieldsFusedStatic) {
         PP_STRICT_CASES(false, kFieldsFusedStatic)
     } else if (fields == kFieldsFusedRF) {
