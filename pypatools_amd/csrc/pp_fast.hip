@@ -678,10 +678,28 @@ DEV void hot_rf_row(const HotRF& rf, int64_t gs, HotRFRow& row) {
 #endif
 }
 
+// Whether full wavefronts stage their cells in LDS (HotMap::stage_exec, a rule on the launch's size): known in the
+// builds for large and for small launches, read from the map in the loss builds.  One build deciding by the map cost
+// large launches 0.7 % (2.19e11 against 2.205e11 particle-steps/s, Boris, 1e6 particles): the compiler laid the scan
+// out twice.
+enum { kStageAlways = 0, kStageNever = 1, kStageByMap = 2 };
+
+template <int STAGE>
+DEV bool stages_cells(const HotMap& m) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (STAGE == kStageNever) return false;
+    else if constexpr (STAGE == kStageAlways) return __builtin_amdgcn_ballot_w64(true) == ~0ull;
+    else return __builtin_amdgcn_ballot_w64(true) == m.stage_exec;
+#else
+    (void)m;
+    return false;
+#endif
+}
+
 // REUSE (the RK4 kernels, whose four stages and successive steps mostly stay in the same cells): the
 // wavefront remembers the cells it staged through LDS last; while every lane is still in its cell, the
 // coefficients are read from the same slots without a new staging (same values, same result).
-template <bool PERIODIC, bool RF = false, bool REUSE = false>
+template <int STAGE, bool PERIODIC, bool RF = false, bool REUSE = false>
 struct HotFE32 {
     const HotMap& m;
     __amdgpu_buffer_rsrc_t rs;
@@ -747,7 +765,7 @@ struct HotFE32 {
                 done = true;
             }
         }
-        // Three ways to the cell coefficients, chosen per wavefront (stage_exec 0: the first and the last only):
+        // Three ways to the cell coefficients, chosen per wavefront (small launches: the first and the last only):
         //  - all lanes in one cell (common right after a cell sort): the cell's
         //    192 B are read once through the scalar cache;
         //  - a full wavefront over at most kStageSlots distinct cells: each
@@ -762,7 +780,7 @@ struct HotFE32 {
 #pragma unroll
             for (int c = 0; c < 6; ++c) v[c] = ceval_s(q + c * 8, wx, wy, wz);
             done = true;
-        } else if (__builtin_amdgcn_ballot_w64(true) == m.stage_exec) {
+        } else if (stages_cells<STAGE>(m)) {
             uint32_t myslot = 0;
             const int ns = distinct_cells(cell, myslot);
             if (ns > 0) {
@@ -794,7 +812,7 @@ struct HotFE32 {
 // FP64-fast gather: 384 B cells ([comp][8 doubles]).  A full wavefront over at most
 // kStageSlots distinct cells stages them through LDS (24 lanes x 16 B per cell, two cells
 // per load instruction); other wavefronts gather per lane.  Both read the same doubles.
-template <bool PERIODIC, bool RF = false, bool REUSE = false>
+template <int STAGE, bool PERIODIC, bool RF = false, bool REUSE = false>
 struct HotFE64 {
     const HotMap& m;
     __amdgpu_buffer_rsrc_t rs;
@@ -827,7 +845,7 @@ struct HotFE64 {
                 done = true;
             }
         }
-        if (!done && __builtin_amdgcn_ballot_w64(true) == m.stage_exec) {
+        if (!done && stages_cells<STAGE>(m)) {
             const int ns = distinct_cells(cell, slot);
             if (ns > 0) {
                 stage_cells<24>(wv, stage_list(), rs, 384u, ns, cell, slot, lanes);
@@ -911,7 +929,7 @@ constexpr int kHotMeshWaves = 4;
 // Every launch with an alive mask takes a loss build, k_hot_mesh with a mesh and k_hot<..., true> without:
 // both run the same step arithmetic, so per-step launches tested on the host and fused launches agree bit
 // for bit, and the mesh test's registers stay out of the build without it.
-template <int ALG, bool MIXED, bool PERIODIC, bool RF, bool LOSS, bool MESH>
+template <int STAGE, int ALG, bool MIXED, bool PERIODIC, bool RF, bool LOSS, bool MESH>
 DEV void hot_body(const HotParams& p) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.n) return;
@@ -927,11 +945,11 @@ DEV void hot_body(const HotParams& p) {
         if constexpr (ALG == PP_ALG_BORIS || ALG == PP_ALG_BORIS_REL || ALG == PP_ALG_VAY) {
             if (!live) return;
             if constexpr (MIXED) {
-                const HotFE32<PERIODIC, RF> fe{p.m, rs, hot_scale(p.m, 1.0), p.rf};
+                const HotFE32<STAGE, PERIODIC, RF> fe{p.m, rs, hot_scale(p.m, 1.0), p.rf};
                 fe.begin_step(p.step0);
                 v = kick_mixed<ALG>(i, r, v, dt, p.step0, fe, ac);
             } else {
-                const HotFE64<PERIODIC, RF> fe{p.m, rs, p.rf};
+                const HotFE64<STAGE, PERIODIC, RF> fe{p.m, rs, p.rf};
                 fe.begin_step(p.step0);
                 v = kick64<ALG>(i, r, v, dt, p.step0, fe, ac);
             }
@@ -944,8 +962,8 @@ DEV void hot_body(const HotParams& p) {
     const float h = (float)(0.5 * p.qm * dt);
     constexpr bool PRE = kPrescaled<ALG>;
     constexpr bool REUSE = ALG == PP_ALG_RK4 || ALG == PP_ALG_RK4_REL;
-    const HotFE32<PERIODIC, RF, REUSE> fe32{p.m, rs, hot_scale(p.m, PRE ? 0.5 * p.qm * dt : 1.0), p.rf};
-    const HotFE64<PERIODIC, RF, REUSE> fe64{p.m, rs, p.rf};
+    const HotFE32<STAGE, PERIODIC, RF, REUSE> fe32{p.m, rs, hot_scale(p.m, PRE ? 0.5 * p.qm * dt : 1.0), p.rf};
+    const HotFE64<STAGE, PERIODIC, RF, REUSE> fe64{p.m, rs, p.rf};
     const bool rec_on = p.r_hist != nullptr;
     int64_t rec_left = p.rec_every - (p.step0 % p.rec_every);
     int64_t rec_idx = p.step0 / p.rec_every + 1;
@@ -999,13 +1017,20 @@ DEV void hot_body(const HotParams& p) {
 template <int ALG, bool MIXED, bool PERIODIC, bool RF, bool LOSS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kHotLossWaves<ALG, MIXED, LOSS>)))
 k_hot(const HotParams p) {
-    hot_body<ALG, MIXED, PERIODIC, RF, LOSS, false>(p);
+    hot_body<LOSS ? kStageByMap : kStageAlways, ALG, MIXED, PERIODIC, RF, LOSS, false>(p);
+}
+
+// launches without an alive mask that gather per lane (gather_direct)
+template <int ALG, bool MIXED, bool PERIODIC, bool RF>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kHotLossWaves<ALG, MIXED, false>)))
+k_hot_direct(const HotParams p) {
+    hot_body<kStageNever, ALG, MIXED, PERIODIC, RF, false, false>(p);
 }
 
 template <int ALG, bool MIXED, bool PERIODIC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kHotMeshWaves)))
 k_hot_mesh(const HotParams p) {
-    hot_body<ALG, MIXED, PERIODIC, false, true, true>(p);
+    hot_body<kStageByMap, ALG, MIXED, PERIODIC, false, true, true>(p);
 }
 
 // ---------------------------------------------------------------------------
@@ -1015,34 +1040,34 @@ k_hot_mesh(const HotParams p) {
 // ---------------------------------------------------------------------------
 
 // Half-step velocity kick of a staggered bunch (the kick_only launches of the single-bunch path).
-template <int ALG, bool MIXED, bool PERIODIC>
+template <int STAGE, int ALG, bool MIXED, bool PERIODIC>
 DEV d3 batch_kick(int64_t i, d3 r, d3 v, double dtk, const HotMap& m, __amdgpu_buffer_rsrc_t rs,
                   const AlgConst& ac) {
-    if constexpr (MIXED) return kick_mixed<ALG>(i, r, v, dtk, 0, HotFE32<PERIODIC>{m, rs, hot_scale(m, 1.0), HotRF{}}, ac);
-    else return kick64<ALG>(i, r, v, dtk, 0, HotFE64<PERIODIC>{m, rs, HotRF{}}, ac);
+    if constexpr (MIXED) return kick_mixed<ALG>(i, r, v, dtk, 0, HotFE32<STAGE, PERIODIC>{m, rs, hot_scale(m, 1.0), HotRF{}}, ac);
+    else return kick64<ALG>(i, r, v, dtk, 0, HotFE64<STAGE, PERIODIC>{m, rs, HotRF{}}, ac);
 }
 
 // ns steps from step0; kick_start / kick_end: the staggering half kicks before the first and after
 // the last step (pp_bunch_flags), for the staggered algorithms only.
-template <int ALG, bool MIXED, bool PERIODIC>
+template <int STAGE, int ALG, bool MIXED, bool PERIODIC>
 DEV void batch_steps(int64_t i, d3& r, d3& v, int64_t step0, int64_t ns, double dt, const HotMap& m,
                      __amdgpu_buffer_rsrc_t rs, const AlgConst& ac, bool kick_start, bool kick_end) {
     constexpr bool STAGGERED = ALG == PP_ALG_BORIS || ALG == PP_ALG_BORIS_REL || ALG == PP_ALG_VAY;
     if constexpr (STAGGERED) {
-        if (kick_start) v = batch_kick<ALG, MIXED, PERIODIC>(i, r, v, -0.5 * dt, m, rs, ac);
+        if (kick_start) v = batch_kick<STAGE, ALG, MIXED, PERIODIC>(i, r, v, -0.5 * dt, m, rs, ac);
     }
     d3 vrec = v;
     const float h = (float)(0.5 * ac.qm * dt);
     constexpr bool PRE = kPrescaled<ALG>;
     constexpr bool REUSE = ALG == PP_ALG_RK4 || ALG == PP_ALG_RK4_REL;
-    const HotFE32<PERIODIC, false, REUSE> fe32{m, rs, hot_scale(m, PRE ? 0.5 * ac.qm * dt : 1.0), HotRF{}};
-    const HotFE64<PERIODIC, false, REUSE> fe64{m, rs, HotRF{}};
+    const HotFE32<STAGE, PERIODIC, false, REUSE> fe32{m, rs, hot_scale(m, PRE ? 0.5 * ac.qm * dt : 1.0), HotRF{}};
+    const HotFE64<STAGE, PERIODIC, false, REUSE> fe64{m, rs, HotRF{}};
     for (int64_t s = 0; s < ns; ++s) {
         if constexpr (MIXED) step_mixed<ALG, PRE>(i, r, v, vrec, dt, h, step0 + s, fe32, ac);
         else step64<ALG>(i, r, v, vrec, dt, step0 + s, fe64, ac);
     }
     if constexpr (STAGGERED) {
-        if (kick_end) v = batch_kick<ALG, MIXED, PERIODIC>(i, r, v, 0.5 * dt, m, rs, ac);
+        if (kick_end) v = batch_kick<STAGE, ALG, MIXED, PERIODIC>(i, r, v, 0.5 * dt, m, rs, ac);
     }
 }
 
@@ -1060,9 +1085,8 @@ constexpr bool batch_class_has(int alg) {
            (CLASS == PP_TILES_RK4) == (alg == PP_ALG_RK4 || alg == PP_ALG_RK4_REL);
 }
 
-template <bool MIXED, bool PERIODIC, int CLASS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBatchWaves<MIXED, CLASS>)))
-k_batched(const BatchParams p) {
+template <int STAGE, bool MIXED, bool PERIODIC, int CLASS>
+DEV void batched_body(const BatchParams& p) {
     const int64_t t = blockIdx.x;
     if (t >= p.ntiles) return;
     const int32_t b = p.tile_bunch[t];
@@ -1098,43 +1122,43 @@ k_batched(const BatchParams p) {
     switch (bd.algorithm) {
         case PP_ALG_BORIS:
             if constexpr (batch_class_has<CLASS>(PP_ALG_BORIS))
-                batch_steps<PP_ALG_BORIS, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
+                batch_steps<STAGE, PP_ALG_BORIS, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
             else
                 return;
             break;
         case PP_ALG_VAY:
             if constexpr (batch_class_has<CLASS>(PP_ALG_VAY))
-                batch_steps<PP_ALG_VAY, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
+                batch_steps<STAGE, PP_ALG_VAY, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
             else
                 return;
             break;
         case PP_ALG_VAY_REL:
             if constexpr (batch_class_has<CLASS>(PP_ALG_VAY_REL))
-                batch_steps<PP_ALG_VAY_REL, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
+                batch_steps<STAGE, PP_ALG_VAY_REL, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
             else
                 return;
             break;
         case PP_ALG_BORIS_REL:
             if constexpr (batch_class_has<CLASS>(PP_ALG_BORIS_REL))
-                batch_steps<PP_ALG_BORIS_REL, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
+                batch_steps<STAGE, PP_ALG_BORIS_REL, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
             else
                 return;
             break;
         case PP_ALG_RK4:
             if constexpr (batch_class_has<CLASS>(PP_ALG_RK4))
-                batch_steps<PP_ALG_RK4, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
+                batch_steps<STAGE, PP_ALG_RK4, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
             else
                 return;
             break;
         case PP_ALG_RK4_REL:
             if constexpr (batch_class_has<CLASS>(PP_ALG_RK4_REL))
-                batch_steps<PP_ALG_RK4_REL, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
+                batch_steps<STAGE, PP_ALG_RK4_REL, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
             else
                 return;
             break;
         case PP_ALG_LEAPFROG:
             if constexpr (batch_class_has<CLASS>(PP_ALG_LEAPFROG))
-                batch_steps<PP_ALG_LEAPFROG, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
+                batch_steps<STAGE, PP_ALG_LEAPFROG, MIXED, PERIODIC>(i, r, v, step0, ns, bd.dt, m, rs, ac, kick_start, kick_end);
             else
                 return;
             break;
@@ -1146,6 +1170,19 @@ k_batched(const BatchParams p) {
     p.vx[i] = v.x;
     p.vy[i] = v.y;
     p.vz[i] = v.z;
+}
+
+template <bool MIXED, bool PERIODIC, int CLASS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBatchWaves<MIXED, CLASS>)))
+k_batched(const BatchParams p) {
+    batched_body<kStageAlways, MIXED, PERIODIC, CLASS>(p);
+}
+
+// batches whose launches gather per lane (gather_direct)
+template <bool MIXED, bool PERIODIC, int CLASS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBatchWaves<MIXED, CLASS>)))
+k_batched_direct(const BatchParams p) {
+    batched_body<kStageNever, MIXED, PERIODIC, CLASS>(p);
 }
 
 // ---------------------------------------------------------------------------
@@ -1185,6 +1222,16 @@ hipError_t launch_gather_probe(const float* table, uint32_t bytes, uint32_t ncel
 
 template <int CLASS>
 static void launch_batched_class(bool mixed, bool periodic, const BatchParams& p, dim3 g, dim3 b, hipStream_t s) {
+    if (p.maps[0].stage_exec == 0) {        // the same for every map of a batch
+        if (mixed) {
+            if (periodic) hipLaunchKernelGGL((k_batched_direct<true, true, CLASS>), g, b, 0, s, p);
+            else hipLaunchKernelGGL((k_batched_direct<true, false, CLASS>), g, b, 0, s, p);
+        } else {
+            if (periodic) hipLaunchKernelGGL((k_batched_direct<false, true, CLASS>), g, b, 0, s, p);
+            else hipLaunchKernelGGL((k_batched_direct<false, false, CLASS>), g, b, 0, s, p);
+        }
+        return;
+    }
     if (mixed) {
         if (periodic) hipLaunchKernelGGL((k_batched<true, true, CLASS>), g, b, 0, s, p);
         else hipLaunchKernelGGL((k_batched<true, false, CLASS>), g, b, 0, s, p);
@@ -1287,6 +1334,15 @@ hipError_t launch_push_sum(int alg, int prec, const PushParams& p, const SumPara
         else hipLaunchKernelGGL((k_hot<A, false, false, RFV, LV>), g, b, 0, s, p);                     \
     }
 
+#define PP_HOT_DIRECT_LAUNCH(A, RFV)                                                                    \
+    if (mixed) {                                                                                        \
+        if (periodic) hipLaunchKernelGGL((k_hot_direct<A, true, true, RFV>), g, b, 0, s, p);           \
+        else hipLaunchKernelGGL((k_hot_direct<A, true, false, RFV>), g, b, 0, s, p);                   \
+    } else {                                                                                            \
+        if (periodic) hipLaunchKernelGGL((k_hot_direct<A, false, true, RFV>), g, b, 0, s, p);          \
+        else hipLaunchKernelGGL((k_hot_direct<A, false, false, RFV>), g, b, 0, s, p);                  \
+    }
+
 #define PP_HOT_MESH_LAUNCH(A)                                                                           \
     if (mixed) {                                                                                        \
         if (periodic) hipLaunchKernelGGL((k_hot_mesh<A, true, true>), g, b, 0, s, p);                  \
@@ -1303,8 +1359,12 @@ hipError_t launch_push_sum(int alg, int prec, const PushParams& p, const SumPara
             PP_HOT_MESH_LAUNCH(A)                                                                       \
         } else if (loss) {                                                                              \
             PP_HOT_LAUNCH(A, false, true)                                                               \
+        } else if (rf && direct) {                                                                      \
+            PP_HOT_DIRECT_LAUNCH(A, true)                                                               \
         } else if (rf) {                                                                                \
             PP_HOT_LAUNCH(A, true, false)                                                               \
+        } else if (direct) {                                                                            \
+            PP_HOT_DIRECT_LAUNCH(A, false)                                                              \
         } else {                                                                                        \
             PP_HOT_LAUNCH(A, false, false)                                                              \
         }                                                                                               \
@@ -1317,6 +1377,7 @@ hipError_t launch_hot(int alg, int prec, bool periodic, const HotParams& p, int 
     const bool rf = p.rf.table != nullptr;
     const bool loss = p.alive != nullptr;
     if (loss && rf) return hipErrorInvalidValue;
+    const bool direct = p.m.stage_exec == 0;
     switch (alg) {
         PP_HOT_CASE(PP_ALG_LEAPFROG)
         PP_HOT_CASE(PP_ALG_BORIS)

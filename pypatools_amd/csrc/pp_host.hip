@@ -600,9 +600,10 @@ static int make_field(const pp_field& f, int precision, FieldDev& out) {
 // How a launch over n particles gathers: per lane while the chip holds at most two wavefronts per SIMD (256 CUs
 // of 4), through cells staged in LDS above that.  Staging reads each distinct cell of a wavefront once, but its
 // scan, cell list, load and LDS passes are one serial chain; with few wavefronts to hide it the 12 (24) loads per
-// lane return sooner.  Measured, 200 steps through a periodic 64 x 64 x 128 map, FP32-mixed, per lane / staged
+// lane return sooner.  Measured with one build for both, 200 steps through a periodic 64 x 64 x 128 map, FP32-mixed, per lane / staged
 // in ms: rk4_rel 2e4 particles 0.57 / 1.07, 1e5 0.97 / 1.25, 1.5e5 1.37 / 1.31, 3e5 2.26 / 1.97; boris 0.20 / 0.29,
-// 0.34 / 0.40, 0.39 / 0.40, 0.58 / 0.44.
+// 0.34 / 0.40, 0.39 / 0.40, 0.58 / 0.44.  Builds of their own took another 20 % off the RK4 launches per lane (rk4_rel,
+// 97 x 81 x 113 map, 1000 / 2e4 / 1e5 particles: 0.96 / 0.80 / 1.03 -> 0.77 / 0.63 / 0.80).
 static bool gather_direct(int64_t n) { return n <= 2 * 4 * 256 * 64; }
 
 static void fill_hot_map(const MapDesc& m, const void* coef, uint64_t bytes, int64_t n, HotMap& h) {
