@@ -16,6 +16,7 @@ Extensions (no reference symbol): ``periodic_z`` maps, ``RFField`` time
 dependence ``F(x) cos(omega t + phase)``, and the ``precision`` of evaluation.
 """
 import os
+import threading
 import warnings
 from abc import ABC, abstractmethod
 
@@ -70,6 +71,8 @@ _FIELD_KWARGS = ("label", "dim", "field", "scaling", "units", "debug", "method",
 
 class Field(FieldBase):
     """0-D (constant), 1-D (z), 2-D (x, y) or 3-D gridded field."""
+
+    _map_lock = threading.Lock()        # device maps are built by one thread at a time
 
     def __init__(self, label="Field", dim=0, field=None, scaling=1.0, units="m", debug=False, method="linear",
                  interpolator_backend="auto", periodic_z=False, precision="fp64"):
@@ -265,18 +268,29 @@ class Field(FieldBase):
                                             cval=c0.fill_value)
         return self._dev_spline
 
+    def _attach_device_grids(self, dev):
+        """dev: a (3, nodes) device copy of the component grids."""
+        self._dev_values = dev
+
+    def _drop_device_grids(self):
+        self._dev_values = None
+
     def device_map(self):
-        if self._dev_map is None:
-            src = self._grid_source()
-            if src is None:
-                raise ValueError("field has no gridded components")
-            if self._dev_values is not None:
-                n = self._dev_values.shape[1]
-                self._dev_map = DeviceFieldMap(src[0], [self._dev_values.view_ptr(k * n) for k in range(3)], 0.0, src[2])
-                self._dev_values = None
-            else:
-                self._dev_map = DeviceFieldMap(src[0], src[1], 0.0, src[2])
-        return self._dev_map
+        # threads that evaluate a field for the first time together get one map; the copy it is made from is held
+        # until the constructor has returned
+        with self._map_lock:
+            if self._dev_map is None:
+                src = self._grid_source()
+                if src is None:
+                    raise ValueError("field has no gridded components")
+                dev = self._dev_values
+                if dev is not None:
+                    n = dev.shape[1]
+                    self._dev_map = DeviceFieldMap(src[0], [dev.view_ptr(k * n) for k in range(3)], 0.0, src[2])
+                    self._drop_device_grids()
+                else:
+                    self._dev_map = DeviceFieldMap(src[0], src[1], 0.0, src[2])
+            return self._dev_map
 
     def _term(self, with_map=True):
         """The device term of this field (PPField), or None if it needs per-component evaluation."""

@@ -144,7 +144,7 @@ class SpaceChargeSolver:
         ey, ez = to_host_pair(self.E[1], self.E[2])
         vals = {a: e.reshape(self.cells) for a, e in zip("xyz", (ex, ey, ez))}
         E = Field.from_arrays(self.grid(), vals, label=f"Space-charge E-field (turn {self.turn_count})", dim=3)
-        E._dev_values = dev
+        E._attach_device_grids(dev)
         return phi.reshape(self.cells), E
 
     def solve(self, particles, charges):

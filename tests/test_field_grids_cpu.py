@@ -1,0 +1,115 @@
+"""Building the device map of a solve's field (its grids come with a device copy): which values it takes, what keeps
+the copy alive while it is read, and what gives it back.  The map constructor is a stand-in, so nothing runs on a
+device."""
+import threading
+
+import numpy as np
+import pytest
+
+from pypatools_amd import engine, field
+from pypatools_amd.field import Field
+
+CELLS = (4, 3, 5)
+N = 4 * 3 * 5
+
+
+class Copy:
+    """Stands for the (3, nodes) DeviceArray of the grids."""
+    shape = (3, N)
+
+    def __init__(self):
+        self.freed = False
+        self.ptr = 4096
+
+    def view_ptr(self, offset):
+        return self.ptr + 8 * offset
+
+    def free(self):
+        self.freed = True
+
+    def __del__(self):
+        self.freed = True
+
+
+class Map:
+    """Records what a device map is made from."""
+    made = []
+
+    def __init__(self, points, components, fill_value=0.0, periodic_z=False, **kw):
+        self.points, self.components, self.kw = points, components, kw
+        self.handle = id(self)
+        self.from_device = not any(isinstance(c, np.ndarray) for c in components)
+        Map.made.append(self)
+
+
+@pytest.fixture
+def solved(monkeypatch):
+    """A field as a solve returns it."""
+    Map.made = []
+    monkeypatch.setattr(field, "DeviceFieldMap", Map)
+    monkeypatch.setattr(engine, "DeviceFieldMap", Map)
+    monkeypatch.setattr(engine, "_FUSED_CACHE", {})
+
+    def make():
+        axes = {a: np.linspace(-1.0, 1.0, n) for a, n in zip("xyz", CELLS)}
+        E = Field.from_arrays(axes, {a: np.full(CELLS, float(k)) for k, a in enumerate("xyz")})
+        dev = Copy()
+        E._attach_device_grids(dev)
+        return E, dev
+    return make
+
+
+def test_map_comes_from_the_device_copy_once(solved):
+    E, _ = solved()
+    m = E.device_map()
+    assert m.from_device and E.device_map() is m and len(Map.made) == 1
+
+
+def test_two_threads_make_one_map_from_a_living_copy(solved, monkeypatch):
+    """The second thread enters device_map while the first is inside the constructor."""
+    E, dev = solved()
+    alive = dev.__dict__                    # outlives the copy itself
+    del dev
+    inside, entered, seen = threading.Event(), threading.Event(), []
+
+    class Slow(Map):
+        def __init__(self, *a, **k):
+            super().__init__(*a, **k)
+            inside.set()
+            if len(Map.made) == 1:
+                entered.wait(5)
+            seen.append(alive["freed"])
+    monkeypatch.setattr(field, "DeviceFieldMap", Slow)
+    got, errors = [], []
+
+    def work(first):
+        try:
+            if not first:
+                inside.wait(5)
+                threading.Timer(0.2, entered.set).start()
+            got.append(E.device_map())
+        except Exception as e:              # noqa: BLE001 - reported below
+            errors.append(e)
+    ts = [threading.Thread(target=work, args=(k == 0,)) for k in range(2)]
+    [t.start() for t in ts]
+    [t.join(10) for t in ts]
+    assert not errors
+    assert len(Map.made) == 1 and got[0] is got[1]
+    assert seen == [False]                  # the copy was there until the constructor had returned
+
+
+def test_copy_lives_until_the_constructor_returns(solved, monkeypatch):
+    """A solve (or another user) that gives the copy back meanwhile does not free it under the reader."""
+    E, dev = solved()
+    alive = dev.__dict__
+    del dev
+    seen = []
+
+    class Interrupted(Map):
+        def __init__(self, *a, **k):
+            E._drop_device_grids()
+            seen.append(alive["freed"])
+            super().__init__(*a, **k)
+    monkeypatch.setattr(field, "DeviceFieldMap", Interrupted)
+    E.device_map()
+    assert seen == [False] and alive["freed"]
