@@ -96,7 +96,7 @@ class Field(FieldBase):
         if field is not None:
             self._field = field
         self._dev_map = None
-        self._dev_values = None         # (3, nodes) device copy of the component grids, where they come from the device
+        self._dev_values = None         # device copy of the component grids (_attach_device_grids)
         self._dev_spline = None
 
     def __getstate__(self):
@@ -238,7 +238,7 @@ class Field(FieldBase):
         comps = self._shared_grid_components()
         if comps is None or any(c.order != 1 for c in comps):
             return None
-        return comps[0].grid, [c.values for c in comps], self._periodic_z
+        return comps[0].grid, [c.node_values() for c in comps], self._periodic_z
 
     def _shared_grid_components(self):
         """The three HipInterpolator components when they share one grid, else None."""
@@ -264,16 +264,28 @@ class Field(FieldBase):
             if self._periodic_z:
                 raise NotImplementedError("periodic_z maps are interpolated linearly only")
             c0 = comps[0]
-            self._dev_spline = DeviceSpline(c0.grid, [c.values for c in comps], c0.order, rgi=c0.rgi,
+            self._dev_spline = DeviceSpline(c0.grid, [c.node_values() for c in comps], c0.order, rgi=c0.rgi,
                                             cval=c0.fill_value)
         return self._dev_spline
 
     def _attach_device_grids(self, dev):
-        """dev: a (3, nodes) device copy of the component grids."""
-        self._dev_values = dev
+        """dev: a (3, nodes) device copy of the component grids as they are now."""
+        self._dev_values = dev, [self._field[c] for c in "xyz"]
 
     def _drop_device_grids(self):
         self._dev_values = None
+
+    def _device_grids(self, points):
+        """The device copy of the grids, or None where it may no longer be equal to them: a component was replaced,
+        its values were handed out, or the axes no longer have its nodes."""
+        attached = self._dev_values
+        if attached is None:
+            return None
+        dev, comps = attached
+        if (any(self._field.get(c) is not k or k.values_given_out for c, k in zip("xyz", comps))
+                or int(np.prod([len(p) for p in points])) != dev.shape[1]):
+            return None
+        return dev
 
     def device_map(self):
         # threads that evaluate a field for the first time together get one map; the copy it is made from is held
@@ -283,13 +295,13 @@ class Field(FieldBase):
                 src = self._grid_source()
                 if src is None:
                     raise ValueError("field has no gridded components")
-                dev = self._dev_values
+                dev = self._device_grids(src[0])
                 if dev is not None:
                     n = dev.shape[1]
                     self._dev_map = DeviceFieldMap(src[0], [dev.view_ptr(k * n) for k in range(3)], 0.0, src[2])
-                    self._drop_device_grids()
                 else:
                     self._dev_map = DeviceFieldMap(src[0], src[1], 0.0, src[2])
+                self._drop_device_grids()
             return self._dev_map
 
     def _term(self, with_map=True):

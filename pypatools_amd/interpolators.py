@@ -192,13 +192,30 @@ class HipInterpolator:
             raise ValueError(f"Values shape {self.values.shape} does not match grid shape {expected}")
         self._bounds = tuple((float(g[0]), float(g[-1])) for g in self.grid)
         self.periodic_z = periodic_z
+        self.values_given_out = False
         self._map = None
         self._splines = {}
 
+    @property
+    def values(self):
+        """The node values.  Whoever has read them may edit them, now or later: from then on a device copy of
+        them made elsewhere is not taken for them any more (values_given_out)."""
+        self.values_given_out = True
+        return self.__dict__["values"]
+
+    @values.setter
+    def values(self, v):
+        self.values_given_out = True
+        self.__dict__["values"] = v
+
+    def node_values(self):
+        """The node values, to be read only."""
+        return self.__dict__["values"]
+
     def device_map(self):
         if self._map is None:
-            self._map = DeviceFieldMap(self.grid, [self.values, self.values, self.values], self.fill_value,
-                                       self.periodic_z)
+            v = self.node_values()
+            self._map = DeviceFieldMap(self.grid, [v, v, v], self.fill_value, self.periodic_z)
         return self._map
 
     def device_spline(self, order):
@@ -206,7 +223,7 @@ class HipInterpolator:
         if self.periodic_z:
             raise NotImplementedError("periodic_z maps are interpolated linearly only")
         if order not in self._splines:
-            self._splines[order] = DeviceSpline(self.grid, [self.values], order, nearest_mode=self.bounds_error,
+            self._splines[order] = DeviceSpline(self.grid, [self.node_values()], order, nearest_mode=self.bounds_error,
                                                 rgi=self.rgi and order == 0,
                                                 cval=0.0 if self.bounds_error else self.fill_value)
         return self._splines[order]

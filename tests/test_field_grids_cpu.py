@@ -1,6 +1,8 @@
 """Building the device map of a solve's field (its grids come with a device copy): which values it takes, what keeps
 the copy alive while it is read, and what gives it back.  The map constructor is a stand-in, so nothing runs on a
 device."""
+import copy
+import pickle
 import threading
 
 import numpy as np
@@ -113,3 +115,53 @@ def test_copy_lives_until_the_constructor_returns(solved, monkeypatch):
     monkeypatch.setattr(field, "DeviceFieldMap", Interrupted)
     E.device_map()
     assert seen == [False] and alive["freed"]
+
+
+def _values(E, m):
+    assert not m.from_device
+    for k, c in enumerate("xyz"):
+        np.testing.assert_array_equal(m.components[k], E._field[c].values)
+
+
+def _edit_in_place(E):
+    E._field["y"].values[1, 1, 1] = 7.0
+
+
+def _rebind_values(E):
+    E._field["z"].values = np.full(CELLS, 9.0)
+
+
+def _keep_and_edit(E):
+    kept = E._field["x"].values
+    kept *= 3.0
+
+
+def _replace_component(E):
+    axes = {a: np.linspace(-1.0, 1.0, n) for a, n in zip("xyz", CELLS)}
+    E._field["x"] = Field.from_arrays(axes, {a: np.full(CELLS, 5.0) for a in "xyz"})._field["x"]
+
+
+def _replace_field(E):
+    axes = {a: np.linspace(-1.0, 1.0, 2 * n) for a, n in zip("xyz", CELLS)}
+    E._field = Field.from_arrays(axes, {a: np.ones([2 * n for n in CELLS]) for a in "xyz"})._field
+
+
+@pytest.mark.parametrize("edit", [_edit_in_place, _rebind_values, _keep_and_edit, _replace_component, _replace_field])
+def test_edited_host_grids_count(solved, edit):
+    E, _ = solved()
+    edit(E)
+    _values(E, E.device_map())
+
+
+def test_axes_of_another_length_do_not_take_the_copy(solved):
+    """The map constructor reads as many values as the axes have nodes."""
+    E, _ = solved()
+    for c in "xyz":
+        E._field[c].grid = tuple(np.linspace(-1.0, 1.0, 2 * n) for n in CELLS)
+    assert not E.device_map().from_device
+
+
+def test_copies_and_pickles_take_the_host_grids(solved):
+    E, _ = solved()
+    for twin in (copy.copy(E), copy.deepcopy(E), pickle.loads(pickle.dumps(E))):
+        _values(twin, twin.device_map())
