@@ -195,6 +195,8 @@ def _fused_map(fe, fb, fp64=True):
         return hit[2]
     m = DeviceFieldMap(se[0], se[1] + sb[1], 0.0, se[2], fp64=fp64)
     _FUSED_CACHE[key] = (be, bb, m)
+    for f in (be, bb):      # a solve's field that is pushed through the shared map needs no map of its own
+        f._drop_device_grids()
     return m
 
 

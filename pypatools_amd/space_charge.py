@@ -20,6 +20,7 @@ fields of a push.
 """
 import ctypes
 import warnings
+import weakref
 
 import numpy as np
 
@@ -33,6 +34,8 @@ INTERIOR, BOUNDARY, CONDUCTOR = 0, 1, 2       # poisson_amg.py:86-90
 class SpaceChargeSolver:
     """Box mesh of mesh_cells = (nx, ny, nz) cell-centre nodes spanning domain_extent = (Lx, Ly, Lz) [m],
     optionally bounded by an electrode assembly (grounded conductors)."""
+
+    _last_field = None      # weak reference to the field of the last solve
 
     def __init__(self, domain_extent, mesh_cells, electrode_assembly=None, solver_tol=1e-10, max_iterations=500):
         self.extent = tuple(float(v) for v in domain_extent)
@@ -135,8 +138,12 @@ class SpaceChargeSolver:
         return self.phi.to_host().reshape(self.cells)
 
     def _potential_and_field(self):
-        """phi and the field on the host; the field keeps a device copy of its grids, from which its map is built."""
+        """phi and the field on the host; the field keeps a device copy of its grids, from which its map is built.
+        Only the latest field does: kept for a whole run of unevaluated fields, the copies would fill the device."""
         from .field import Field
+        last = self._last_field() if self._last_field is not None else None
+        if last is not None:
+            last._drop_device_grids()
         dev = DeviceArray((3, self.n_dofs))
         for k, e in enumerate(self.E):
             _lib.call("pp_memcpy_d2d", dev.view_ptr(k * self.n_dofs), e.ptr, e.nbytes, None)
@@ -145,6 +152,7 @@ class SpaceChargeSolver:
         vals = {a: e.reshape(self.cells) for a, e in zip("xyz", (ex, ey, ez))}
         E = Field.from_arrays(self.grid(), vals, label=f"Space-charge E-field (turn {self.turn_count})", dim=3)
         E._attach_device_grids(dev)
+        self._last_field = weakref.ref(E)
         return phi.reshape(self.cells), E
 
     def solve(self, particles, charges):

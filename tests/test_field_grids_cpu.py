@@ -161,6 +161,42 @@ def test_axes_of_another_length_do_not_take_the_copy(solved):
     assert not E.device_map().from_device
 
 
+def test_a_fused_map_gives_the_copy_back(solved):
+    E, dev = solved()
+    axes = {a: np.linspace(-1.0, 1.0, n) for a, n in zip("xyz", CELLS)}
+    B = Field.from_arrays(axes, {a: np.ones(CELLS) for a in "xyz"})
+    alive = dev.__dict__
+    del dev
+    m = engine._fused_map(E, B)
+    assert alive["freed"] and not m.from_device
+    for k, c in enumerate("xyz"):
+        np.testing.assert_array_equal(m.components[k], np.full(CELLS, float(k)))
+    _values(E, E.device_map())
+
+
+def test_fields_of_earlier_turns_hold_no_copy(solved, monkeypatch):
+    """A program that keeps the field of every turn unevaluated keeps one device copy, not one per turn."""
+    from pypatools_amd import space_charge
+    copies = []
+
+    class Dev(Copy):
+        def __init__(self, shape, *a):
+            super().__init__()
+            self.shape, self.nbytes = shape, 8 * N
+            if shape == (3, N):
+                copies.append(self.__dict__)
+    monkeypatch.setattr(space_charge, "DeviceArray", Dev)
+    monkeypatch.setattr(space_charge._lib, "call", lambda *a: None)
+    monkeypatch.setattr(space_charge, "to_host_pair", lambda a, b: (np.zeros(N), np.zeros(N)))
+    s = space_charge.SpaceChargeSolver.__new__(space_charge.SpaceChargeSolver)
+    s.cells, s.extent, s.n_dofs, s.turn_count = CELLS, (1.0, 1.0, 1.0), N, 0
+    s.h = tuple(L / n for L, n in zip(s.extent, s.cells))
+    s.phi, s.E = Dev((N,)), [Dev((N,)) for _ in range(3)]
+    kept = [s._potential_and_field()[1] for _ in range(5)]
+    assert [c["freed"] for c in copies] == [True] * 4 + [False]
+    assert kept[-1].device_map().from_device and not kept[0].device_map().from_device
+
+
 def test_copies_and_pickles_take_the_host_grids(solved):
     E, _ = solved()
     for twin in (copy.copy(E), copy.deepcopy(E), pickle.loads(pickle.dumps(E))):
