@@ -73,6 +73,7 @@ class Field(FieldBase):
     """0-D (constant), 1-D (z), 2-D (x, y) or 3-D gridded field."""
 
     _map_lock = threading.Lock()        # device maps are built by one thread at a time
+    _dev_values = None                  # device copy of the component grids (_attach_device_grids)
 
     def __init__(self, label="Field", dim=0, field=None, scaling=1.0, units="m", debug=False, method="linear",
                  interpolator_backend="auto", periodic_z=False, precision="fp64"):
@@ -96,12 +97,11 @@ class Field(FieldBase):
         if field is not None:
             self._field = field
         self._dev_map = None
-        self._dev_values = None         # device copy of the component grids (_attach_device_grids)
         self._dev_spline = None
 
     def __getstate__(self):
         # copies and pickles take the host grids; the device copy of them stays with its field
-        return {**self.__dict__, "_dev_values": None}
+        return {k: v for k, v in self.__dict__.items() if k != "_dev_values"}
 
     # ---- core API ----------------------------------------------------------
     def __call__(self, pts):

@@ -201,3 +201,12 @@ def test_copies_and_pickles_take_the_host_grids(solved):
     E, _ = solved()
     for twin in (copy.copy(E), copy.deepcopy(E), pickle.loads(pickle.dumps(E))):
         _values(twin, twin.device_map())
+
+
+def test_fields_saved_before_device_copies_existed(solved):
+    """A field whose saved state knows nothing of the device copy builds its map from its grids."""
+    E, _ = solved()
+    state = {k: v for k, v in E.__dict__.items() if "dev_values" not in k and "device_grids" not in k}
+    old = Field.__new__(Field)
+    old.__dict__.update(state)
+    _values(old, old.device_map())
