@@ -369,8 +369,6 @@ class Tracker:
             # resynchronised velocities into the last record; particles that were lost keep theirs
             self._velocity_record(st, _row(vh, n_records - 1, M), ustate, live_only=True)
         r_hist, v_hist = to_host_pair(rh, vh)
-        if elec is not None:
-            active[:] = st.alive.to_host().astype(bool)
         if verbose:
             print(f"Tracking complete: {nsteps} steps, {M} particles")
         if return_state:
@@ -552,6 +550,7 @@ class Tracker:
             _lib.call("pp_push_lossy", a, elec.handle, None)
             step += k
         st.unsort()
+        active[:] = st.alive.to_host().astype(bool)
 
     def _rk4_stage_loop(self, st, fp, nsteps, dt, t0, hist, dtp, verbose):
         """_rk4_step_batch (pusher.py:803-892) with fields evaluated between device stage kernels."""
