@@ -366,8 +366,8 @@ class Tracker:
             self._slow_loop(st, fp, nsteps, dt, t0, rf, hist, elec, active, dtp, verbose)
         if alg in STAGGERED:
             self._kick(st, fp, fused, 0.5 * dt, nsteps, rf, t0, dt)
-            # resynchronised velocities into the last record; particles that were lost keep theirs
-            self._velocity_record(st, _row(vh, n_records - 1, M), ustate, live_only=True)
+            # resynchronised velocities into the last record; of a batch, particles that were lost keep theirs
+            self._velocity_record(st, _row(vh, n_records - 1, M), ustate, live_only=batch)
         r_hist, v_hist = to_host_pair(rh, vh)
         if verbose:
             print(f"Tracking complete: {nsteps} steps, {M} particles")
