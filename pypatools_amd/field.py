@@ -298,7 +298,8 @@ class Field(FieldBase):
                 dev = self._device_grids(src[0])
                 if dev is not None:
                     n = dev.shape[1]
-                    self._dev_map = DeviceFieldMap(src[0], [dev.view_ptr(k * n) for k in range(3)], 0.0, src[2])
+                    self._dev_map = DeviceFieldMap(src[0], [dev.view_ptr(k * n) for k in range(3)], 0.0, src[2],
+                                                   on_device=True)
                 else:
                     self._dev_map = DeviceFieldMap(src[0], src[1], 0.0, src[2])
                 self._drop_device_grids()

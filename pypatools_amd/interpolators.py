@@ -41,13 +41,12 @@ def grid_to_axes(points):
 
 class DeviceFieldMap:
     """A device map of ``ncomp`` components on one grid (pp_map_create_parts); the components are arrays, or
-    addresses of device buffers of the grid's size."""
+    with ``on_device`` the addresses of device buffers of the grid's size."""
 
     def __init__(self, points, components, fill_value=0.0, periodic_z=False, fp32=True, coefficients=True,
-                 fp64=True):
+                 fp64=True, on_device=False):
         axes = grid_to_axes(points)
         shape = tuple(len(a) for a in axes)
-        on_device = all(isinstance(v, int) for v in components)
         parts = (ctypes.c_void_p * len(components))()
         keep = []
         for c, v in enumerate(components):
