@@ -62,7 +62,7 @@ constexpr size_t kPoolBlock = (size_t)256 << 20, kPoolBytes = (size_t)1 << 30;
 struct DeviceBlock {
     size_t bytes;
     int device;
-    bool idle;
+    enum { kUsed, kFreeing, kIdle } state;
 };
 
 std::mutex g_pool_mu;
@@ -112,7 +112,7 @@ hipError_t device_alloc(void** out, size_t bytes) {
         for (auto it = g_idle.rbegin(); it != g_idle.rend(); ++it) {
             DeviceBlock& b = g_blocks[*it];
             if (b.bytes != size || b.device != device) continue;
-            b.idle = false;
+            b.state = DeviceBlock::kUsed;
             *out = *it;
             g_idle.erase(std::next(it).base());
             g_idle_bytes -= size;
@@ -124,7 +124,7 @@ hipError_t device_alloc(void** out, size_t bytes) {
             drop_idle(0);
             e = hipMalloc(out, size);
         }
-        if (e == hipSuccess) g_blocks[*out] = DeviceBlock{size, device, false};
+        if (e == hipSuccess) g_blocks[*out] = DeviceBlock{size, device, DeviceBlock::kUsed};
         return e;
     } catch (const std::bad_alloc&) {
         if (*out) (void)hipFree(*out);
@@ -136,23 +136,21 @@ hipError_t device_alloc(void** out, size_t bytes) {
 hipError_t device_free(void* p) {
     if (!p) return hipSuccess;
     bool pooled = false;
+    int current = 0, device = 0;
     {
         std::lock_guard<std::mutex> lk(g_pool_mu);
         const auto it = g_blocks.find(p);
         if (it != g_blocks.end()) {
-            if (it->second.idle) return hipErrorInvalidValue;       // freed before
+            if (it->second.state != DeviceBlock::kUsed) return hipErrorInvalidValue;    // freed before, or just now
             pooled = g_captures.load() == 0;
-            if (!pooled) g_blocks.erase(it);
+            device = it->second.device;
+            if (pooled) it->second.state = DeviceBlock::kFreeing;
+            else g_blocks.erase(it);
         }
     }
     if (!pooled) return hipFree(p);
-    // the block counts as in use until nothing on the device can touch it any more
-    int current = 0, device = 0;
+    // the block is nobody's until nothing on the device can touch it any more
     hipError_t e = hipGetDevice(&current);
-    {
-        std::lock_guard<std::mutex> lk(g_pool_mu);
-        device = g_blocks[p].device;
-    }
     if (e == hipSuccess && device != current) e = hipSetDevice(device);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (device != current) (void)hipSetDevice(current);
@@ -169,7 +167,7 @@ hipError_t device_free(void* p) {
         g_blocks.erase(p);
         return hipFree(p);
     }
-    b.idle = true;
+    b.state = DeviceBlock::kIdle;
     g_idle_bytes += b.bytes;
     drop_idle(kPoolBytes);
     return hipSuccess;

@@ -1,0 +1,42 @@
+"""Host code of the library on a stand-in for the HIP runtime (tests/native): compiled with the host compiler, no
+device.  Each case is a program of its own; a hang ends at its time limit."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.join(ROOT, "tests", "native")
+
+
+@pytest.fixture(scope="session")
+def native(tmp_path_factory):
+    """Builds one of tests/native/*.cpp; kernels and launchers stay unresolved (the cases launch none)."""
+    built = {}
+
+    def build(name):
+        if name not in built:
+            if shutil.which("g++") is None or not os.path.isdir("/opt/rocm/include/hip"):
+                pytest.skip("needs g++ and the HIP headers")
+            exe = str(tmp_path_factory.mktemp("native") / name)
+            cmd = ["g++", "-std=c++17", "-O1", "-g", "-x", "c++", "-D__HIP_PLATFORM_AMD__", "-pthread",
+                   "-I/opt/rocm/include", "-I", os.path.join(ROOT, "include"),
+                   "-I", os.path.join(ROOT, "pypatools_amd", "csrc"), os.path.join(HERE, name + ".cpp"), "-o", exe,
+                   "-Wl,--unresolved-symbols=ignore-all"]
+            res = subprocess.run(cmd, capture_output=True, text=True)
+            assert res.returncode == 0, res.stderr[-4000:]
+            built[name] = exe
+        return built[name]
+    return build
+
+
+def run(exe, case):
+    res = subprocess.run([exe, case], capture_output=True, text=True, timeout=60)
+    assert res.returncode == 0, f"{case}: exit {res.returncode}\n{res.stderr}"
+
+
+@pytest.mark.parametrize("case", ["reuse_waits", "double_free"])
+def test_device_blocks(native, case):
+    run(native("test_blocks"), case)
