@@ -11,6 +11,7 @@
 #include <iterator>
 #include <mutex>
 #include <new>
+#include <shared_mutex>
 #include <unordered_map>
 #include <vector>
 
@@ -56,7 +57,7 @@ hipStream_t stream_of(pp_stream s) { return s ? static_cast<hipStream_t>(s) : g_
 // particles) to 3.6 ms (1e6).  Freed blocks of up to 256 MiB are kept, at most 1 GiB in all, the oldest going first, and
 // serve later requests of the same size class (eight classes per factor of two) on the same device.  Like hipFree a free
 // waits for the device, so no stream still uses a kept block.  While a stream is being captured, frees and allocations
-// go to the runtime as they are.
+// go to the runtime as they are; a capture does not begin while a free waits for the device (g_capture_mu).
 constexpr size_t kPoolBlock = (size_t)256 << 20, kPoolBytes = (size_t)1 << 30;
 
 struct DeviceBlock {
@@ -70,6 +71,7 @@ std::unordered_map<void*, DeviceBlock> g_blocks;     // every block of a size cl
 std::deque<void*> g_idle;                            // idle ones, oldest first
 size_t g_idle_bytes = 0;
 std::atomic<int> g_captures{0};
+std::shared_mutex g_capture_mu;     // shared: a free that waits for the device; exclusive: a capture that begins
 
 size_t size_class(size_t bytes) {
     size_t top = 256;
@@ -135,6 +137,7 @@ hipError_t device_alloc(void** out, size_t bytes) {
 
 hipError_t device_free(void* p) {
     if (!p) return hipSuccess;
+    std::shared_lock<std::shared_mutex> no_capture(g_capture_mu);
     bool pooled = false;
     int current = 0, device = 0;
     {
@@ -148,12 +151,16 @@ hipError_t device_free(void* p) {
             else g_blocks.erase(it);
         }
     }
-    if (!pooled) return hipFree(p);
+    if (!pooled) {
+        no_capture.unlock();
+        return hipFree(p);
+    }
     // the block is nobody's until nothing on the device can touch it any more
     hipError_t e = hipGetDevice(&current);
     if (e == hipSuccess && device != current) e = hipSetDevice(device);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (device != current) (void)hipSetDevice(current);
+    no_capture.unlock();
     std::lock_guard<std::mutex> lk(g_pool_mu);
     DeviceBlock& b = g_blocks[p];
     if (e != hipSuccess) {
@@ -1059,6 +1066,7 @@ int pp_graph_begin(pp_stream s) {
     int rc = ensure_init();
     if (rc) return rc;
     if (!s) return fail(PP_ERR_INVALID, "graph capture needs a created stream");
+    std::unique_lock<std::shared_mutex> no_free(g_capture_mu);
     g_captures.fetch_add(1);
     const hipError_t e = hipStreamBeginCapture(static_cast<hipStream_t>(s), hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
