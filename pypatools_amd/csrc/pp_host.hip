@@ -13,6 +13,7 @@
 #include <new>
 #include <shared_mutex>
 #include <unordered_map>
+#include <unordered_set>
 #include <vector>
 
 #include "pp_internal.h"
@@ -70,8 +71,17 @@ std::mutex g_pool_mu;
 std::unordered_map<void*, DeviceBlock> g_blocks;     // every block of a size class, in use or idle
 std::deque<void*> g_idle;                            // idle ones, oldest first
 size_t g_idle_bytes = 0;
-std::atomic<int> g_captures{0};
 std::shared_mutex g_capture_mu;     // shared: a free that waits for the device; exclusive: a capture that begins
+std::mutex g_capturing_mu;
+std::unordered_set<hipStream_t> g_capturing;        // streams with a capture open
+std::atomic<int> g_captures{0};                     // their number
+
+bool note_capture(hipStream_t s, bool open) {       // false: it was so already
+    std::lock_guard<std::mutex> lk(g_capturing_mu);
+    const bool changed = open ? g_capturing.insert(s).second : g_capturing.erase(s) == 1;
+    g_captures.store((int)g_capturing.size());
+    return changed;
+}
 
 size_t size_class(size_t bytes) {
     size_t top = 256;
@@ -319,7 +329,17 @@ int pp_stream_create(pp_stream* s) {
 }
 
 int pp_stream_destroy(pp_stream s) {
-    if (s) HIP_TRY(hipStreamDestroy(static_cast<hipStream_t>(s)), "hipStreamDestroy");
+    if (!s) return PP_OK;
+    // destroyed while it records: its capture ends with it (noted first, since the handle may be given out again)
+    const bool open = note_capture(static_cast<hipStream_t>(s), false);
+    const hipError_t e = hipStreamDestroy(static_cast<hipStream_t>(s));
+    if (e != hipSuccess) {
+        try {
+            if (open) (void)note_capture(static_cast<hipStream_t>(s), true);
+        } catch (const std::bad_alloc&) {
+        }
+        return hip_fail(e, "hipStreamDestroy");
+    }
     return PP_OK;
 }
 
@@ -1066,11 +1086,17 @@ int pp_graph_begin(pp_stream s) {
     int rc = ensure_init();
     if (rc) return rc;
     if (!s) return fail(PP_ERR_INVALID, "graph capture needs a created stream");
-    std::unique_lock<std::shared_mutex> no_free(g_capture_mu);
-    g_captures.fetch_add(1);
-    const hipError_t e = hipStreamBeginCapture(static_cast<hipStream_t>(s), hipStreamCaptureModeThreadLocal);
+    const hipStream_t st = static_cast<hipStream_t>(s);
+    std::lock_guard<std::shared_mutex> no_free(g_capture_mu);
+    bool added = false;
+    try {
+        added = note_capture(st, true);
+    } catch (const std::bad_alloc&) {
+        return fail(PP_ERR_NOMEM, "begin capture: out of host memory");
+    }
+    const hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
-        g_captures.fetch_sub(1);
+        if (added) (void)note_capture(st, false);       // else: the capture that is open already goes on
         return hip_fail(e, "begin capture");
     }
     return PP_OK;
@@ -1079,11 +1105,11 @@ int pp_graph_begin(pp_stream s) {
 int pp_graph_end(pp_stream s, pp_graph* g) {
     if (!s || !g) return fail(PP_ERR_INVALID, "null argument");
     hipGraph_t graph;
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    const bool capturing = hipStreamIsCapturing(static_cast<hipStream_t>(s), &status) == hipSuccess &&
-                           status != hipStreamCaptureStatusNone;
     const hipError_t ce = hipStreamEndCapture(static_cast<hipStream_t>(s), &graph);
-    if (capturing) g_captures.fetch_sub(1);
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;     // an end by the wrong thread leaves it open
+    if (ce == hipSuccess || hipStreamIsCapturing(static_cast<hipStream_t>(s), &status) != hipSuccess ||
+        status == hipStreamCaptureStatusNone)
+        (void)note_capture(static_cast<hipStream_t>(s), false);
     if (ce != hipSuccess) return hip_fail(ce, "end capture");
     hipGraphExec_t exec;
     hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);

@@ -37,6 +37,6 @@ def run(exe, case):
     assert res.returncode == 0, f"{case}: exit {res.returncode}\n{res.stderr}"
 
 
-@pytest.mark.parametrize("case", ["reuse_waits", "double_free", "free_and_capture"])
+@pytest.mark.parametrize("case", ["reuse_waits", "double_free", "free_and_capture", "destroyed_stream"])
 def test_device_blocks(native, case):
     run(native("test_blocks"), case)
