@@ -378,16 +378,16 @@ int create(const double* v, int64_t nv, const int32_t* idx, int64_t nt, pp_mesh*
     if (m->nnodes > 0) {
         pp_bvh::MeshDev d{};
         const size_t rbytes = sizeof(pp_bvh::Range) * cand.ranges.size();
-        bool ok = hipMalloc(&m->nodes, sizeof(Node) * m->nnodes) == hipSuccess &&
-                  hipMalloc(&m->tris, sizeof(Tri) * (size_t)nt) == hipSuccess &&
-                  hipMalloc(&m->ranges, rbytes) == hipSuccess &&
-                  hipMalloc(&m->clear, cand.clear.size()) == hipSuccess &&
-                  hipMalloc(&m->dev, sizeof(pp_bvh::MeshDev)) == hipSuccess;
+        bool ok = pp_pool::raw_alloc(&m->nodes, sizeof(Node) * m->nnodes) == hipSuccess &&
+                  pp_pool::raw_alloc(&m->tris, sizeof(Tri) * (size_t)nt) == hipSuccess &&
+                  pp_pool::raw_alloc(&m->ranges, rbytes) == hipSuccess &&
+                  pp_pool::raw_alloc(&m->clear, cand.clear.size()) == hipSuccess &&
+                  pp_pool::raw_alloc(&m->dev, sizeof(pp_bvh::MeshDev)) == hipSuccess;
         const bool lists = !cand.cells.empty();
         if (ok && lists)
-            ok = hipMalloc(&m->cells, sizeof(int32_t) * cand.cells.size()) == hipSuccess &&
+            ok = pp_pool::raw_alloc(&m->cells, sizeof(int32_t) * cand.cells.size()) == hipSuccess &&
                  (cand.cell_tris.empty() ||
-                  hipMalloc(&m->cell_tris, sizeof(int32_t) * cand.cell_tris.size()) == hipSuccess);
+                  pp_pool::raw_alloc(&m->cell_tris, sizeof(int32_t) * cand.cell_tris.size()) == hipSuccess);
         if (ok) {
             d.nodes = m->nodes;
             d.tris = m->tris;

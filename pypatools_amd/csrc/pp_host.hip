@@ -100,21 +100,27 @@ void drop_idle(size_t keep) {       // g_pool_mu held
     }
 }
 
+}  // namespace
+
+hipError_t pp_pool::raw_alloc_bytes(void** out, size_t bytes) {
+    hipError_t e = hipMalloc(out, bytes);
+    if (e == hipErrorOutOfMemory && g_captures.load() == 0) {
+        (void)hipGetLastError();
+        {
+            std::lock_guard<std::mutex> lk(g_pool_mu);
+            drop_idle(0);
+        }
+        e = hipMalloc(out, bytes);
+    }
+    return e;
+}
+
+namespace {
+
 hipError_t device_alloc(void** out, size_t bytes) {
     *out = nullptr;
     if (bytes == 0) bytes = 256;
-    if (bytes > kPoolBlock || g_captures.load() > 0) {
-        hipError_t e = hipMalloc(out, bytes);
-        if (e == hipErrorOutOfMemory && g_captures.load() == 0) {
-            (void)hipGetLastError();
-            {
-                std::lock_guard<std::mutex> lk(g_pool_mu);
-                drop_idle(0);
-            }
-            e = hipMalloc(out, bytes);
-        }
-        return e;
-    }
+    if (bytes > kPoolBlock || g_captures.load() > 0) return pp_pool::raw_alloc_bytes(out, bytes);
     const size_t size = size_class(bytes);
     int device = 0;
     hipError_t e = hipGetDevice(&device);
@@ -934,7 +940,7 @@ static int take_row_set(RowSet& q) {
     q = {nullptr, nullptr, g_device};
     hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&q.host), sizeof(double) * 12 * PP_PUSH_ROWS_MAX,
                                  hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&q.dev), sizeof(double) * 6 * PP_PUSH_ROWS_MAX);
+    if (e == hipSuccess) e = pp_pool::raw_alloc(&q.dev, sizeof(double) * 6 * PP_PUSH_ROWS_MAX);
     if (e != hipSuccess) {
         free_row_set(q);
         return hip_fail(e, "row buffers");

@@ -186,6 +186,15 @@ hipError_t launch_interleave(const MapParts& src, const MapDesc& d, double* raw,
 hipError_t launch_build_coef(const MapDesc& d, double* c64, float* c32, hipStream_t s);
 }  // namespace pp_strict
 
+// device memory beside the kept blocks (pp_host.hip): hipMalloc, which drops the kept blocks where it fails
+namespace pp_pool {
+hipError_t raw_alloc_bytes(void** p, size_t bytes);
+template <class T>
+hipError_t raw_alloc(T** p, size_t bytes) {
+    return raw_alloc_bytes(reinterpret_cast<void**>(p), bytes);
+}
+}  // namespace pp_pool
+
 // blocking copies of ordinary host memory (pp_copy.hip): every region of a call, all to the host or all to the device
 namespace pp_copy {
 struct Region {

@@ -478,12 +478,12 @@ int create(const PoissonDesc& d, pp_poisson** out, char* err, size_t errn) {
             const double s = sin(pi * (double)(k + 1) / (2.0 * (double)(n + 1)));
             lam[k] = 4.0 / (d.h[a] * d.h[a]) * (s * s);
         }
-        ok = ok && hipMalloc(&P->S[a], sizeof(double) * n * n) == hipSuccess &&
-             hipMalloc(&P->lam[a], sizeof(double) * n) == hipSuccess &&
+        ok = ok && pp_pool::raw_alloc(&P->S[a], sizeof(double) * n * n) == hipSuccess &&
+             pp_pool::raw_alloc(&P->lam[a], sizeof(double) * n) == hipSuccess &&
              hipMemcpy(P->S[a], S.data(), sizeof(double) * n * n, hipMemcpyHostToDevice) == hipSuccess &&
              hipMemcpy(P->lam[a], lam.data(), sizeof(double) * n, hipMemcpyHostToDevice) == hipSuccess;
     }
-    ok = ok && hipMalloc(&P->work, sizeof(double) * 2 * cells) == hipSuccess;
+    ok = ok && pp_pool::raw_alloc(&P->work, sizeof(double) * 2 * cells) == hipSuccess;
     if (!ok) {
         snprintf(err, errn, "device allocation for the Poisson solver failed");
         for (int a = 0; a < 3; ++a) {
@@ -764,13 +764,13 @@ static int build_operator(pp_poisson* P, char* err, size_t errn) {
                 if (plain) P->box[0] = diag;
             }
     for (int a = 0; a < 3; ++a) P->box[1 + a] = -2.0 / (d.h[a] * (d.h[a] + d.h[a]));
-    const bool ok = hipMalloc(&P->type, sizeof(int32_t) * N) == hipSuccess &&
-                    hipMalloc(&P->coef, sizeof(double) * 7 * N) == hipSuccess &&
-                    hipMalloc(&P->vec, sizeof(double) * 9 * N) == hipSuccess &&
-                    hipMalloc(&P->regular, (size_t)N) == hipSuccess &&
+    const bool ok = pp_pool::raw_alloc(&P->type, sizeof(int32_t) * N) == hipSuccess &&
+                    pp_pool::raw_alloc(&P->coef, sizeof(double) * 7 * N) == hipSuccess &&
+                    pp_pool::raw_alloc(&P->vec, sizeof(double) * 9 * N) == hipSuccess &&
+                    pp_pool::raw_alloc(&P->regular, (size_t)N) == hipSuccess &&
                     hipMemcpy(P->regular, regular.data(), (size_t)N, hipMemcpyHostToDevice) == hipSuccess &&
-                    hipMalloc(&P->part, sizeof(double) * 2 * pp_poissonk::kDotBlocks) == hipSuccess &&
-                    hipMalloc(&P->sc, sizeof(double) * pp_poissonk::kScalars) == hipSuccess &&
+                    pp_pool::raw_alloc(&P->part, sizeof(double) * 2 * pp_poissonk::kDotBlocks) == hipSuccess &&
+                    pp_pool::raw_alloc(&P->sc, sizeof(double) * pp_poissonk::kScalars) == hipSuccess &&
                     hipHostMalloc(reinterpret_cast<void**>(&P->host), sizeof(double) * 8, hipHostMallocDefault) ==
                         hipSuccess &&
                     hipMemcpy(P->type, P->h_type.data(), sizeof(int32_t) * N, hipMemcpyHostToDevice) == hipSuccess &&

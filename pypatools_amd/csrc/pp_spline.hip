@@ -399,7 +399,7 @@ hipError_t create(const double* values, int64_t ncomp, int ndim, const int64_t* 
     const int64_t ncoef = ncomp * d.N[0] * d.N[1] * d.N[2];
     hipError_t e;
     auto alloc = [&](size_t bytes, void** p) {
-        e = hipMalloc(p, bytes ? bytes : 256);
+        e = pp_pool::raw_alloc(p, bytes ? bytes : 256);
         if (e == hipSuccess) s->allocs[s->nalloc++] = *p;
         return e == hipSuccess;
     };

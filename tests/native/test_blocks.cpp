@@ -87,6 +87,22 @@ static void destroyed_stream() {
     CHECK(get(MIB) == a && frees == 0);
 }
 
+// allocations of the other modules take kept blocks' memory when there is no other
+static void other_allocations() {
+    budget = 64 * MIB;
+    void* p[4];
+    for (auto& q : p) q = get(16 * MIB);
+    for (auto& q : p) CHECK(pp_free(q) == PP_OK);
+    size_t free_bytes = 0, total = 0;
+    CHECK(pp_mem_info(&free_bytes, &total) == PP_OK && free_bytes == budget);
+    double* d = nullptr;
+    CHECK(pp_pool::raw_alloc(&d, 40 * MIB) == hipSuccess && d);
+    CHECK(hipGetLastError() == hipSuccess);     // the first attempt left no error behind
+    int32_t* big = nullptr;
+    CHECK(pp_pool::raw_alloc(&big, 40 * MIB) == hipErrorOutOfMemory && !big);
+    CHECK(hipFree(d) == hipSuccess);
+}
+
 int main(int argc, char** argv) {
     CHECK(argc == 2 && pp_init(0) == PP_OK);
     const std::string w = argv[1];
@@ -94,6 +110,7 @@ int main(int argc, char** argv) {
     else if (w == "double_free") double_free();
     else if (w == "free_and_capture") free_and_capture();
     else if (w == "destroyed_stream") destroyed_stream();
+    else if (w == "other_allocations") other_allocations();
     else CHECK(!"unknown case");
     return 0;
 }

@@ -37,6 +37,18 @@ def run(exe, case):
     assert res.returncode == 0, f"{case}: exit {res.returncode}\n{res.stderr}"
 
 
-@pytest.mark.parametrize("case", ["reuse_waits", "double_free", "free_and_capture", "destroyed_stream"])
+@pytest.mark.parametrize("case", ["reuse_waits", "double_free", "free_and_capture", "destroyed_stream", "other_allocations"])
 def test_device_blocks(native, case):
     run(native("test_blocks"), case)
+
+
+def test_no_module_allocates_past_the_kept_blocks():
+    """hipMalloc itself fails while freed blocks are kept that could serve the request."""
+    csrc = os.path.join(ROOT, "pypatools_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        if name != "pp_host.hip":
+            with open(os.path.join(csrc, name)) as f:
+                assert "hipMalloc(" not in f.read(), name
+    with open(os.path.join(csrc, "pp_host.hip")) as f:
+        blocks, rest = f.read().split("int ensure_init()", 1)
+    assert "hipMalloc(" in blocks and "hipMalloc(" not in rest
