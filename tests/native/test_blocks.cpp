@@ -103,6 +103,27 @@ static void other_allocations() {
     CHECK(hipFree(d) == hipSuccess);
 }
 
+// at most 1 GiB is kept, the oldest blocks go first, and all of it goes back on request
+static void bound_and_release() {
+    void* p[8];
+    for (auto& q : p) q = get(200 * MIB);
+    for (auto& q : p) CHECK(pp_free(q) == PP_OK);
+    CHECK(used == 4 * 208 * MIB);       // the size class of 200 MiB is 208 MiB; a fifth would pass 1 GiB
+    for (int k = 0; k < 8; ++k) CHECK(blocks.count(p[k]) == (k < 4 ? 0u : 1u));
+    CHECK(pp_release_staging() == PP_OK && used == 0);
+}
+
+// a kept block is not handed out on another device
+static void devices_apart() {
+    void* a = get(MIB);
+    CHECK(pp_free(a) == PP_OK);
+    CHECK(pp_init(1) == PP_OK);
+    void* b = get(MIB);
+    CHECK(b != a);
+    CHECK(pp_init(0) == PP_OK && pp_free(b) == PP_OK && device == 0);
+    CHECK(get(MIB) == a);
+}
+
 int main(int argc, char** argv) {
     CHECK(argc == 2 && pp_init(0) == PP_OK);
     const std::string w = argv[1];
@@ -111,6 +132,8 @@ int main(int argc, char** argv) {
     else if (w == "free_and_capture") free_and_capture();
     else if (w == "destroyed_stream") destroyed_stream();
     else if (w == "other_allocations") other_allocations();
+    else if (w == "bound_and_release") bound_and_release();
+    else if (w == "devices_apart") devices_apart();
     else CHECK(!"unknown case");
     return 0;
 }

@@ -37,7 +37,8 @@ def run(exe, case):
     assert res.returncode == 0, f"{case}: exit {res.returncode}\n{res.stderr}"
 
 
-@pytest.mark.parametrize("case", ["reuse_waits", "double_free", "free_and_capture", "destroyed_stream", "other_allocations"])
+@pytest.mark.parametrize("case", ["reuse_waits", "double_free", "free_and_capture", "destroyed_stream", "other_allocations",
+                                  "bound_and_release", "devices_apart"])
 def test_device_blocks(native, case):
     run(native("test_blocks"), case)
 
