@@ -6,6 +6,7 @@
 
 #include "hip_on_host.h"
 
+#include "pp_copy.hip"
 #include "pp_host.hip"
 
 namespace pp_beam {
