@@ -93,6 +93,13 @@ struct Job {
         if (e != hipSuccess) error.compare_exchange_strong(none, (int)e);
     }
 
+    // false also where the query fails: the wait for the event reports that
+    static bool not_ready(hipEvent_t ev) {
+        if (hipEventQuery(ev) != hipErrorNotReady) return false;
+        (void)hipGetLastError();        // the answer, not an error of this thread's next launch
+        return true;
+    }
+
     bool start(int t, size_t c, int slot) {     // DMA of chunk c from or into thread t's slot
         char* pin = pinned + (size_t)(2 * t + slot) * kSlotBytes;
         const Chunk& q = chunks[c];
@@ -117,7 +124,7 @@ struct Job {
             for (size_t c = t, turn = 0; c < n; c += threads, ++turn) {
                 const int slot = (int)(turn & 1);
                 hipEvent_t ev = events[2 * t + slot];
-                while (error.load() == 0 && hipEventQuery(ev) == hipErrorNotReady) {
+                while (error.load() == 0 && not_ready(ev)) {
                     if (filled < n) {
                         populate(chunks[filled].host, chunks[filled].bytes);
                         filled += threads;

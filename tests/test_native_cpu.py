@@ -53,3 +53,8 @@ def test_no_module_allocates_past_the_kept_blocks():
     with open(os.path.join(csrc, "pp_host.hip")) as f:
         blocks, rest = f.read().split("int ensure_init()", 1)
     assert "hipMalloc(" in blocks and "hipMalloc(" not in rest
+
+
+@pytest.mark.parametrize("case", ["bytes", "no_error_left"])
+def test_copies(native, case):
+    run(native("test_copy"), case)
