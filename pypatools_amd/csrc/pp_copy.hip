@@ -4,14 +4,14 @@
 // The runtime moves pageable memory in pieces through one staging buffer and one thread: 6 to 11 GB/s, of which
 // most is page faults of a fresh destination (results are new arrays).  Here a few threads share a transfer; each
 // owns two pinned slots and every T-th chunk, so DMA, host copies and page faults overlap, and while the stream is
-// still computing the threads already fault the destination's pages in.
+// still computing the threads already fault the destination's pages in; then the caller's thread alone waits for it.
 #include <hip/hip_runtime.h>
 #include <string.h>
 #include <sys/mman.h>
 #include <unistd.h>
 
 #include <atomic>
-#include <chrono>
+#include <condition_variable>
 #include <mutex>
 #include <new>
 #include <system_error>
@@ -87,6 +87,17 @@ struct Job {
     char* pinned;
     hipEvent_t* events;             // 2 per thread
     std::atomic<int> error{0};      // first hipError_t
+    std::mutex mu;                  // caller_waits: until the caller's thread has its first chunk, the others sleep
+    std::condition_variable awake;
+    bool caller_waits = true;
+
+    void wake() {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            caller_waits = false;
+        }
+        awake.notify_all();
+    }
 
     void note(hipError_t e) {
         int none = 0;
@@ -110,7 +121,13 @@ struct Job {
         return e == hipSuccess;
     }
 
+    // t = 0: the caller's thread
     void run(int t) {
+        copy(t);
+        if (t == 0) wake();     // also where it gave up
+    }
+
+    void copy(int t) {
         if (hipSetDevice(device) != hipSuccess) {
             note(hipErrorInvalidDevice);
             return;
@@ -120,23 +137,28 @@ struct Job {
             for (int k = 0; k < 2; ++k)
                 if ((size_t)(t + k * threads) < n && !start(t, t + k * threads, k)) return;
             size_t filled = t;
-            int waits = 0;
             for (size_t c = t, turn = 0; c < n; c += threads, ++turn) {
                 const int slot = (int)(turn & 1);
                 hipEvent_t ev = events[2 * t + slot];
+                int polls = 0;      // of about 0.5 us
                 while (error.load() == 0 && not_ready(ev)) {
                     if (filled < n) {
                         populate(chunks[filled].host, chunks[filled].bytes);
                         filled += threads;
-                    } else if (++waits < 400) {     // about 0.2 ms of polling, then leave the core to others
+                    } else if (++polls < 400) {
                         std::this_thread::yield();
                     } else {
-                        std::this_thread::sleep_for(std::chrono::microseconds(20));
+                        break;
                     }
+                }
+                if (t != 0 && turn == 0) {
+                    std::unique_lock<std::mutex> lk(mu);
+                    if (polls == 400) awake.wait(lk, [this] { return !caller_waits; });
                 }
                 if (error.load()) return;
                 const hipError_t e = hipEventSynchronize(ev);
                 note(e);
+                if (t == 0 && turn == 0) wake();
                 if (e != hipSuccess) return;
                 memcpy(chunks[c].host, pinned + (size_t)(2 * t + slot) * kSlotBytes, chunks[c].bytes);
                 if (c + 2 * threads < n && !start(t, c + 2 * threads, slot)) return;
