@@ -128,7 +128,8 @@ struct Job {
     }
 
     void copy(int t) {
-        if (hipSetDevice(device) != hipSuccess) {
+        // a thread starts on device 0; the caller's has been set
+        if (t != 0 && hipSetDevice(device) != hipSuccess) {
             note(hipErrorInvalidDevice);
             return;
         }
@@ -188,6 +189,25 @@ hipError_t plain(const Region* r, int n, bool to_host, hipStream_t s) {
     return hipStreamSynchronize(s);
 }
 
+// The library's device is current while this lives: events belong to the device that is current when they are made,
+// and have to belong to the stream's.
+struct OnDevice {
+    int before = 0;
+    hipError_t error;
+    explicit OnDevice(int device) : device_(device) {
+        error = hipGetDevice(&before);
+        if (error == hipSuccess && before != device_) error = hipSetDevice(device_);
+    }
+    ~OnDevice() {
+        if (error == hipSuccess && before != device_) (void)hipSetDevice(before);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+
+private:
+    int device_;
+};
+
 }  // namespace
 
 hipError_t transfer(const Region* r, int n, bool to_host, int device, hipStream_t s) {
@@ -205,6 +225,8 @@ hipError_t transfer(const Region* r, int n, bool to_host, int device, hipStream_
         if (hipPointerGetAttributes(&at, r[k].host) != hipSuccess) (void)hipGetLastError();
         else if (at.type != hipMemoryTypeUnregistered) return plain(r, n, to_host, s);
     }
+    const OnDevice guard(device);
+    if (guard.error != hipSuccess) return guard.error;
     const int set = acquire();
     if (set < 0) return plain(r, n, to_host, s);
     // a thread per MiB: starting one costs about as much as copying 0.3 MiB
@@ -237,7 +259,7 @@ hipError_t transfer(const Region* r, int n, bool to_host, int device, hipStream_
                 }
             }
             job.run(0);
-            for (int t = up; t < threads; ++t) job.run(t);      // shares of threads that could not be started
+            for (int t = up; t < threads; ++t) job.copy(t);     // shares of threads that could not be started
             for (int t = 1; t < up; ++t) pool[t].join();
             rc = (hipError_t)job.error.load();
         }
