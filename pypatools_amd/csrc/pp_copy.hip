@@ -217,7 +217,7 @@ hipError_t transfer(const Region* r, int n, bool to_host, int device, hipStream_
         total += r[k].bytes;
         ordinary = ordinary && (!r[k].bytes || (r[k].host && r[k].dev));
     }
-    if (!ordinary || total < kSmallBytes || (!to_host && total >= kManyBytes && total < kUploadBytes))
+    if (device < 0 || !ordinary || total < kSmallBytes || (!to_host && total >= kManyBytes && total < kUploadBytes))
         return plain(r, n, to_host, s);
     for (int k = 0; k < n; ++k) {       // pinned (or device) memory is copied in place by the runtime
         hipPointerAttribute_t at;
