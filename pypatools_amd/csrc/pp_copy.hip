@@ -27,18 +27,22 @@
 namespace pp_copy {
 namespace {
 
-// Where the lines lie, runtime / here in ms:
-//   to a fresh array   0.25 MB 0.17 / 0.04   0.5 MB 0.24 / 0.05   1 MB 0.23 / 0.15   4 MB 0.42 / 0.29   16 MB 1.95 / 0.65
-//                      128 MB 13.2 / 3.5
-//   from the host      0.25 MB 0.11 / 0.04   0.5 MB 0.21 / 0.05   1 MB 0.05 / 0.10   16 MB 0.46 / 0.57   32 MB 1.07 / 0.92
-//                      128 MB 4.6 / 3.4
-// (from 1 MB the runtime pins the caller's pages and copies in place, which a fresh destination has to fault first)
+// Where the lines lie, runtime / here in us:
+//   to the host, fresh array   32 KB 13 / 9   128 KB 30 / 13   512 KB 93 / 37   1 MB 230 / 150   4 MB 420 / 290
+//                              16 MB 1950 / 650   128 MB 13200 / 3500
+//   to the host, reused array  32 KB 9 / 9    128 KB 14 / 13   512 KB 29 / 28
+//   from the host              32 KB 9-21 / 9   128 KB 13-58 / 11   512 KB 23 / 22   1 MB 50 / 100   16 MB 460 / 570
+//                              32 MB 1070 / 920   128 MB 4600 / 3400
+// (from 1 MB the runtime pins the caller's pages and copies in place, which a fresh destination has to fault first.
+// Below it a piece and a wait for the stream are all there is: in two pieces with an event each, made and destroyed,
+// 128 KB took 33 us either way and 512 KB 46.)
 constexpr size_t kSmallBytes = (size_t)16 << 10;    // below: the runtime's own path
-constexpr size_t kManyBytes = (size_t)1 << 20;      // below: one thread
+constexpr size_t kManyBytes = (size_t)1 << 20;      // below: one piece a region, no threads
 constexpr size_t kUploadBytes = (size_t)32 << 20;   // uploads from kManyBytes to here: the runtime's own path
 constexpr int kMaxThreads = 6;
 constexpr size_t kSlotBytes = (size_t)2 << 20;
 constexpr size_t kSetBytes = 2 * kMaxThreads * kSlotBytes;
+static_assert(kManyBytes <= kSlotBytes, "one_piece");
 constexpr int kMaxSets = 2;     // at most 48 MiB pinned; a third concurrent transfer takes the runtime's own path
 
 std::mutex g_mu;
@@ -189,6 +193,25 @@ hipError_t plain(const Region* r, int n, bool to_host, hipStream_t s) {
     return hipStreamSynchronize(s);
 }
 
+// Regions of less than one slot in all: through it as they are.
+hipError_t one_piece(const Region* r, int n, bool to_host, char* pin, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    size_t o = 0;
+    for (int k = 0; k < n && e == hipSuccess; o += r[k].bytes, ++k) {
+        if (!r[k].bytes) continue;
+        if (!to_host) memcpy(pin + o, r[k].host, r[k].bytes);
+        e = to_host ? hipMemcpyAsync(pin + o, r[k].dev, r[k].bytes, hipMemcpyDeviceToHost, s)
+                    : hipMemcpyAsync(r[k].dev, pin + o, r[k].bytes, hipMemcpyHostToDevice, s);
+        if (to_host) populate(static_cast<char*>(r[k].host), r[k].bytes);
+    }
+    const hipError_t se = hipStreamSynchronize(s);      // also after a failure: the slot serves others next
+    if (e == hipSuccess) e = se;
+    o = 0;
+    for (int k = 0; k < n && to_host && e == hipSuccess; o += r[k].bytes, ++k)
+        if (r[k].bytes) memcpy(r[k].host, pin + o, r[k].bytes);
+    return e;
+}
+
 // The library's device is current while this lives: events belong to the device that is current when they are made,
 // and have to belong to the stream's.
 struct OnDevice {
@@ -229,8 +252,13 @@ hipError_t transfer(const Region* r, int n, bool to_host, int device, hipStream_
     if (guard.error != hipSuccess) return guard.error;
     const int set = acquire();
     if (set < 0) return plain(r, n, to_host, s);
+    if (total < kManyBytes) {
+        const hipError_t e = one_piece(r, n, to_host, static_cast<char*>(g_sets[set]), s);
+        give_back(set);
+        return e;
+    }
     // a thread per MiB: starting one costs about as much as copying 0.3 MiB
-    int threads = total < kManyBytes ? 1 : (int)(total >> 20) + 1;
+    int threads = (int)(total >> 20) + 1;
     threads = threads > kMaxThreads ? kMaxThreads : threads;
     size_t piece = (total / (2 * threads) + 4095) & ~(size_t)4095;
     if (piece > kSlotBytes) piece = kSlotBytes;

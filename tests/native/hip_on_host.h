@@ -19,7 +19,7 @@ inline std::map<void*, size_t> blocks;          // live device blocks
 inline std::map<void*, size_t> pinned;          // live pinned blocks
 inline std::vector<size_t> mallocs;             // sizes asked of hipMalloc, in order
 inline size_t budget = (size_t)1 << 44, used = 0;
-inline std::atomic<int> device_syncs{0}, event_syncs{0}, event_queries{0}, frees{0}, bad_frees{0};
+inline std::atomic<int> device_syncs{0}, event_syncs{0}, event_queries{0}, events_made{0}, copies{0}, frees{0}, bad_frees{0};
 inline std::set<hipStream_t> capturing;
 inline std::function<void()> on_device_sync;    // called inside hipDeviceSynchronize
 inline std::function<bool(hipEvent_t)> event_ready;     // null: every event is complete
@@ -142,6 +142,7 @@ hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, c
 }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    ++events_made;
     *e = reinterpret_cast<hipEvent_t>(malloc(1));
     std::lock_guard<std::recursive_mutex> lk(mu);
     event_device[*e] = device;
@@ -169,6 +170,7 @@ hipError_t hipEventSynchronize(hipEvent_t e) {
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind, hipStream_t) {
+    ++copies;
     memcpy(d, s, bytes);
     return hipSuccess;
 }

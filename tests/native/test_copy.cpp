@@ -93,6 +93,19 @@ static void no_device_yet() {
         }
 }
 
+// small transfers are one copy a region and one wait for the stream: no events, no threads
+static void small_in_one_piece() {
+    for (size_t n : {16 * KIB, 100 * KIB + 3, MIB - 5})
+        for (int to_host = 0; to_host < 2; ++to_host) {
+            Pair p(n - 4), q(4);
+            copies = 0;
+            const Region two[2] = {{to_host ? q.b.data() : q.a.data(), to_host ? q.a.data() : q.b.data(), 4},
+                                   {to_host ? p.b.data() : p.a.data(), to_host ? p.a.data() : p.b.data(), n - 4}};
+            CHECK(pp_copy::transfer(two, 2, to_host, 0, nullptr) == hipSuccess);
+            CHECK(p.a == p.b && q.a == q.b && copies == 2 && events_made == 0 && event_queries == 0);
+        }
+}
+
 int main(int argc, char** argv) {
     CHECK(argc == 2);
     const std::string w = argv[1];
@@ -101,6 +114,7 @@ int main(int argc, char** argv) {
     else if (w == "one_waiter") one_waiter();
     else if (w == "devices_kept") devices_kept();
     else if (w == "no_device_yet") no_device_yet();
+    else if (w == "small_in_one_piece") small_in_one_piece();
     else CHECK(!"unknown case");
     return 0;
 }

@@ -55,6 +55,7 @@ def test_no_module_allocates_past_the_kept_blocks():
     assert "hipMalloc(" in blocks and "hipMalloc(" not in rest
 
 
-@pytest.mark.parametrize("case", ["bytes", "no_error_left", "one_waiter", "devices_kept", "no_device_yet"])
+@pytest.mark.parametrize("case", ["bytes", "no_error_left", "one_waiter", "devices_kept", "no_device_yet",
+                                  "small_in_one_piece"])
 def test_copies(native, case):
     run(native("test_copy"), case)
