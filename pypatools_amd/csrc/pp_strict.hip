@@ -434,7 +434,9 @@ hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s) {
     const dim3 g(grid_for(p.n, block)), b(block);
     const int fields = fields_case(p);
     if (p.mesh) {
-        if (fields == kFieldsFusedStatic) PP_STRICT_CASES(true, kFieldsFusedStatic)
+        if (fields == kFieldsMap3dAny) PP_STRICT_CASES(true, kFieldsMap3dAny)
+        else if (fields == kFieldsMap3dAnyRF) PP_STRICT_CASES(true, kFieldsMap3dAnyRF)
+        else if (fields == kFieldsFusedStatic) PP_STRICT_CASES(true, kFieldsFusedStatic)
         else if (fields == kFieldsFusedRF) PP_STRICT_CASES(true, kFieldsFusedRF)
         else PP_STRICT_CASES(true, kFieldsGeneral)
     } else if (fields == kFieldsUniform) {
@@ -443,6 +445,10 @@ hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s) {
         PP_STRICT_CASES(false, kFieldsMap3d)
     } else if (fields == kFieldsMap3dRF) {
         PP_STRICT_CASES(false, kFieldsMap3dRF)
+    } else if (fields == kFieldsMap3dAny) {
+        PP_STRICT_CASES(false, kFieldsMap3dAny)
+    } else if (fields == kFieldsMap3dAnyRF) {
+        PP_STRICT_CASES(false, kFieldsMap3dAnyRF)
     } else if (fields == kFieldsFusedStatic) {
         PP_STRICT_CASES(false, kFieldsFusedStatic)
     } else if (fields == kFieldsFusedRF) {
