@@ -256,7 +256,7 @@ struct RowFE64 {
         const MapDesc& m = p.E.map;
         const double rfv = rf != PP_RF_NONE ? rf_factor(p, gs, stage, rf) : 1.0;
         if (m.periodic) z = wrap_periodic(z, m.lo[2], m.L, m.inv_d[2] * m.inv_nz);
-        const AxisGuess qx = guess_axis(m, 0, x), qy = guess_axis(m, 1, y), qz = guess_axis(m, 2, z);
+        const AxisGuess qx = guess_axis_3d(m, 0, x), qy = guess_axis_3d(m, 1, y), qz = guess_axis_3d(m, 2, z);
         StrictCell c;
         c.base = ((int64_t)qx.i * m.ng[1] + qy.i) * m.ng[2] + qz.i;
         double f[8];
@@ -393,19 +393,29 @@ static bool row_route(int alg, const PushParams& p) {
 
 static inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
-#define PP_STRICT_CASES(L, U)                                                                                \
-    switch (alg) {                                                                                        \
-        case PP_ALG_LEAPFROG: hipLaunchKernelGGL((k_push64<PP_ALG_LEAPFROG, L, U>), g, b, 0, s, p); break;   \
-        case PP_ALG_BORIS: hipLaunchKernelGGL((k_push64<PP_ALG_BORIS, L, U>), g, b, 0, s, p); break;         \
-        case PP_ALG_RK4: hipLaunchKernelGGL((k_push64<PP_ALG_RK4, L, U>), g, b, 0, s, p); break;             \
-        case PP_ALG_YOSHIDA: hipLaunchKernelGGL((k_push64<PP_ALG_YOSHIDA, L, U>), g, b, 0, s, p); break;     \
-        case PP_ALG_VAY_REL: hipLaunchKernelGGL((k_push64<PP_ALG_VAY_REL, L, U>), g, b, 0, s, p); break;     \
-        case PP_ALG_RK4_REL: hipLaunchKernelGGL((k_push64<PP_ALG_RK4_REL, L, U>), g, b, 0, s, p); break;     \
-        case PP_ALG_YOSHIDA_REL: hipLaunchKernelGGL((k_push64<PP_ALG_YOSHIDA_REL, L, U>), g, b, 0, s, p); break; \
-        case PP_ALG_BORIS_REL: hipLaunchKernelGGL((k_push64<PP_ALG_BORIS_REL, L, U>), g, b, 0, s, p); break; \
-        case PP_ALG_VAY: hipLaunchKernelGGL((k_push64<PP_ALG_VAY, L, U>), g, b, 0, s, p); break;             \
-        default: return hipErrorInvalidValue;                                                             \
+#define PP_STRICT_SINGLE(L, U)                                                                                \
+    case PP_ALG_LEAPFROG: hipLaunchKernelGGL((k_push64<PP_ALG_LEAPFROG, L, U>), g, b, 0, s, p); break;       \
+    case PP_ALG_BORIS: hipLaunchKernelGGL((k_push64<PP_ALG_BORIS, L, U>), g, b, 0, s, p); break;             \
+    case PP_ALG_YOSHIDA: hipLaunchKernelGGL((k_push64<PP_ALG_YOSHIDA, L, U>), g, b, 0, s, p); break;         \
+    case PP_ALG_VAY_REL: hipLaunchKernelGGL((k_push64<PP_ALG_VAY_REL, L, U>), g, b, 0, s, p); break;         \
+    case PP_ALG_YOSHIDA_REL: hipLaunchKernelGGL((k_push64<PP_ALG_YOSHIDA_REL, L, U>), g, b, 0, s, p); break; \
+    case PP_ALG_BORIS_REL: hipLaunchKernelGGL((k_push64<PP_ALG_BORIS_REL, L, U>), g, b, 0, s, p); break;     \
+    case PP_ALG_VAY: hipLaunchKernelGGL((k_push64<PP_ALG_VAY, L, U>), g, b, 0, s, p); break;
+
+#define PP_STRICT_RK4(L, U)                                                                                   \
+    case PP_ALG_RK4: hipLaunchKernelGGL((k_push64<PP_ALG_RK4, L, U>), g, b, 0, s, p); break;                 \
+    case PP_ALG_RK4_REL: hipLaunchKernelGGL((k_push64<PP_ALG_RK4_REL, L, U>), g, b, 0, s, p); break;
+
+#define PP_STRICT_CASES(L, U)                                                                                 \
+    switch (alg) {                                                                                            \
+        PP_STRICT_SINGLE(L, U)                                                                                \
+        PP_STRICT_RK4(L, U)                                                                                   \
+        default: return hipErrorInvalidValue;                                                                 \
     }
+
+// The general build of terms that share no map: with all corners of a lookup in flight it holds two wavefronts per
+// SIMD, plane by plane three.
+constexpr int64_t kGeneralAll = 2 * 4 * 256 * 64;
 
 template <int ALG>
 static void launch_row(const PushParams& p, hipStream_t s) {
@@ -453,6 +463,12 @@ hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s) {
         PP_STRICT_CASES(false, kFieldsFusedStatic)
     } else if (fields == kFieldsFusedRF) {
         PP_STRICT_CASES(false, kFieldsFusedRF)
+    } else if (p.n > kGeneralAll) {
+        switch (alg) {
+            PP_STRICT_SINGLE(false, kFieldsGeneralMany)
+            PP_STRICT_RK4(false, kFieldsGeneral)
+            default: return hipErrorInvalidValue;
+        }
     } else {
         PP_STRICT_CASES(false, kFieldsGeneral)
     }
