@@ -28,17 +28,23 @@ namespace pp_copy {
 namespace {
 
 // Where the lines lie, runtime / here in us:
-//   to the host, fresh array   32 KB 13 / 9   128 KB 30 / 13   512 KB 93 / 37   1 MB 230 / 150   4 MB 420 / 290
-//                              16 MB 1950 / 650   128 MB 13200 / 3500
-//   to the host, reused array  32 KB 9 / 9    128 KB 14 / 13   512 KB 29 / 28
+//   to the host, fresh array   32 KB 13 / 9   128 KB 30 / 13   512 KB 93 / 37   1 MB 234 / 81   4 MB 970 / 650
+//                              8 MB 1940 / 820   16 MB 3890 / 1000   32 MB 7520 / 2020
+//   to the host, reused array  32 KB 9 / 9    128 KB 14 / 13   512 KB 29 / 28   1 MB 64 / 63   4 MB 234 / 187
+//                              8 MB 478 / 343   16 MB 942 / 610   32 MB 1860 / 980
 //   from the host              32 KB 9-21 / 9   128 KB 13-58 / 11   512 KB 23 / 22   1 MB 50 / 100   16 MB 460 / 570
 //                              32 MB 1070 / 920   128 MB 4600 / 3400
 // (from 1 MB the runtime pins the caller's pages and copies in place, which a fresh destination has to fault first.
 // Below it a piece and a wait for the stream are all there is: in two pieces with an event each, made and destroyed,
 // 128 KB took 33 us either way and 512 KB 46.)
+// Threads, 1 / 2 / 3 / 6 of them, us: reused array 1 MB 63 / 134 / 149 / 264, 4 MB 187 / 218 / 241 / 335, 8 MB 376 / 349 /
+// 343 / 427, 16 MB 653 / 552 / 525 / 610; fresh array 1 MB 81 / 166 / 198 / 267, 4 MB 653 / 643 / 611 / 514, 8 MB 1553 /
+// 958 / 816 / 720, 16 MB 3324 / 2082 / 1573 / 996.
 constexpr size_t kSmallBytes = (size_t)16 << 10;    // below: the runtime's own path
 constexpr size_t kManyBytes = (size_t)1 << 20;      // below: one piece a region, no threads
 constexpr size_t kUploadBytes = (size_t)32 << 20;   // uploads from kManyBytes to here: the runtime's own path
+constexpr size_t kAloneBytes = (size_t)5 << 20;     // below: one thread
+constexpr size_t kThreadBytes = (size_t)3 << 20;    // from there another one for each of these
 constexpr int kMaxThreads = 6;
 constexpr size_t kSlotBytes = (size_t)2 << 20;
 constexpr size_t kSetBytes = 2 * kMaxThreads * kSlotBytes;
@@ -257,9 +263,8 @@ hipError_t transfer(const Region* r, int n, bool to_host, int device, hipStream_
         give_back(set);
         return e;
     }
-    // a thread per MiB: starting one costs about as much as copying 0.3 MiB
-    int threads = (int)(total >> 20) + 1;
-    threads = threads > kMaxThreads ? kMaxThreads : threads;
+    const size_t many = total < kAloneBytes ? 1 : 1 + total / kThreadBytes;
+    const int threads = many > (size_t)kMaxThreads ? kMaxThreads : (int)many;
     size_t piece = (total / (2 * threads) + 4095) & ~(size_t)4095;
     if (piece > kSlotBytes) piece = kSlotBytes;
     hipEvent_t events[2 * kMaxThreads] = {};

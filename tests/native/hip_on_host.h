@@ -11,6 +11,7 @@
 #include <map>
 #include <mutex>
 #include <set>
+#include <thread>
 #include <vector>
 
 namespace host_hip {
@@ -21,6 +22,7 @@ inline std::vector<size_t> mallocs;             // sizes asked of hipMalloc, in 
 inline size_t budget = (size_t)1 << 44, used = 0;
 inline std::atomic<int> device_syncs{0}, event_syncs{0}, event_queries{0}, events_made{0}, copies{0}, frees{0}, bad_frees{0};
 inline std::set<hipStream_t> capturing;
+inline std::set<std::thread::id> copiers;        // threads that enqueued copies
 inline std::function<void()> on_device_sync;    // called inside hipDeviceSynchronize
 inline std::function<bool(hipEvent_t)> event_ready;     // null: every event is complete
 inline std::function<void(hipEvent_t)> on_event_sync;
@@ -171,6 +173,10 @@ hipError_t hipEventSynchronize(hipEvent_t e) {
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind, hipStream_t) {
     ++copies;
+    {
+        std::lock_guard<std::recursive_mutex> lk(mu);
+        copiers.insert(std::this_thread::get_id());
+    }
     memcpy(d, s, bytes);
     return hipSuccess;
 }

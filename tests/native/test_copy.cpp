@@ -106,6 +106,20 @@ static void small_in_one_piece() {
         }
 }
 
+// a transfer that one thread does faster starts no others
+static void threads_by_size() {
+    const struct {
+        size_t bytes, threads;
+    } want[] = {{MIB, 1}, {2 * MIB + 1, 1}, {5 * MIB - 1, 1}, {5 * MIB, 2}, {8 * MIB, 3}, {16 * MIB, 6}, {64 * MIB, 6}};
+    for (const auto& w : want) {
+        Pair p(w.bytes);
+        copiers.clear();
+        const Region r = {p.b.data(), p.a.data(), w.bytes};
+        CHECK(pp_copy::transfer(&r, 1, true, 0, nullptr) == hipSuccess);
+        CHECK(p.a == p.b && copiers.size() == w.threads);
+    }
+}
+
 int main(int argc, char** argv) {
     CHECK(argc == 2);
     const std::string w = argv[1];
@@ -115,6 +129,7 @@ int main(int argc, char** argv) {
     else if (w == "devices_kept") devices_kept();
     else if (w == "no_device_yet") no_device_yet();
     else if (w == "small_in_one_piece") small_in_one_piece();
+    else if (w == "threads_by_size") threads_by_size();
     else CHECK(!"unknown case");
     return 0;
 }

@@ -56,6 +56,6 @@ def test_no_module_allocates_past_the_kept_blocks():
 
 
 @pytest.mark.parametrize("case", ["bytes", "no_error_left", "one_waiter", "devices_kept", "no_device_yet",
-                                  "small_in_one_piece"])
+                                  "small_in_one_piece", "threads_by_size"])
 def test_copies(native, case):
     run(native("test_copy"), case)
