@@ -678,7 +678,7 @@ DEV void hot_rf_row(const HotRF& rf, int64_t gs, HotRFRow& row) {
 #endif
 }
 
-// Whether full wavefronts stage their cells in LDS (HotMap::stage_exec, a rule on the launch's size): known in the
+// Whether full wavefronts stage their cells in LDS (HotMap::stage_exec, gather_direct's rule): known in the
 // builds for large and for small launches, read from the map in the loss builds.  One build deciding by the map cost
 // large launches 0.7 % (2.19e11 against 2.205e11 particle-steps/s, Boris, 1e6 particles): the compiler laid the scan
 // out twice.
@@ -1226,7 +1226,7 @@ static void launch_batched_class(bool mixed, bool periodic, const BatchParams& p
         if (mixed) {
             if (periodic) hipLaunchKernelGGL((k_batched_direct<true, true, CLASS>), g, b, 0, s, p);
             else hipLaunchKernelGGL((k_batched_direct<true, false, CLASS>), g, b, 0, s, p);
-        } else {
+        } else if constexpr (CLASS == PP_TILES_SINGLE_GATHER) {     // FP64 RK4 tiles are always staged
             if (periodic) hipLaunchKernelGGL((k_batched_direct<false, true, CLASS>), g, b, 0, s, p);
             else hipLaunchKernelGGL((k_batched_direct<false, false, CLASS>), g, b, 0, s, p);
         }
@@ -1334,14 +1334,17 @@ hipError_t launch_push_sum(int alg, int prec, const PushParams& p, const SumPara
         else hipLaunchKernelGGL((k_hot<A, false, false, RFV, LV>), g, b, 0, s, p);                     \
     }
 
-#define PP_HOT_DIRECT_LAUNCH(A, RFV)                                                                    \
-    if (mixed) {                                                                                        \
-        if (periodic) hipLaunchKernelGGL((k_hot_direct<A, true, true, RFV>), g, b, 0, s, p);           \
-        else hipLaunchKernelGGL((k_hot_direct<A, true, false, RFV>), g, b, 0, s, p);                   \
-    } else {                                                                                            \
-        if (periodic) hipLaunchKernelGGL((k_hot_direct<A, false, true, RFV>), g, b, 0, s, p);          \
-        else hipLaunchKernelGGL((k_hot_direct<A, false, false, RFV>), g, b, 0, s, p);                  \
+// (FP64 RK4 launches are always staged)
+template <int ALG, bool RF>
+static void launch_hot_direct(bool mixed, bool periodic, const HotParams& p, dim3 g, dim3 b, hipStream_t s) {
+    if (mixed) {
+        if (periodic) hipLaunchKernelGGL((k_hot_direct<ALG, true, true, RF>), g, b, 0, s, p);
+        else hipLaunchKernelGGL((k_hot_direct<ALG, true, false, RF>), g, b, 0, s, p);
+    } else if constexpr (ALG != PP_ALG_RK4 && ALG != PP_ALG_RK4_REL) {
+        if (periodic) hipLaunchKernelGGL((k_hot_direct<ALG, false, true, RF>), g, b, 0, s, p);
+        else hipLaunchKernelGGL((k_hot_direct<ALG, false, false, RF>), g, b, 0, s, p);
     }
+}
 
 #define PP_HOT_MESH_LAUNCH(A)                                                                           \
     if (mixed) {                                                                                        \
@@ -1360,11 +1363,11 @@ hipError_t launch_push_sum(int alg, int prec, const PushParams& p, const SumPara
         } else if (loss) {                                                                              \
             PP_HOT_LAUNCH(A, false, true)                                                               \
         } else if (rf && direct) {                                                                      \
-            PP_HOT_DIRECT_LAUNCH(A, true)                                                               \
+            launch_hot_direct<A, true>(mixed, periodic, p, g, b, s);                                    \
         } else if (rf) {                                                                                \
             PP_HOT_LAUNCH(A, true, false)                                                               \
         } else if (direct) {                                                                            \
-            PP_HOT_DIRECT_LAUNCH(A, false)                                                              \
+            launch_hot_direct<A, false>(mixed, periodic, p, g, b, s);                                   \
         } else {                                                                                        \
             PP_HOT_LAUNCH(A, false, false)                                                              \
         }                                                                                               \

@@ -628,18 +628,30 @@ static int make_field(const pp_field& f, int precision, FieldDev& out) {
     return PP_OK;
 }
 
-// How a launch over n particles gathers: per lane while the chip holds at most two wavefronts per SIMD (256 CUs
-// of 4), through cells staged in LDS above that.  Staging reads each distinct cell of a wavefront once, but its
-// scan, cell list, load and LDS passes are one serial chain; with few wavefronts to hide it the 12 (24) loads per
-// lane return sooner.  Measured with one build for both, 200 steps through a periodic 64 x 64 x 128 map, FP32-mixed, per lane / staged
-// in ms: rk4_rel 2e4 particles 0.57 / 1.07, 1e5 0.97 / 1.25, 1.5e5 1.37 / 1.31, 3e5 2.26 / 1.97; boris 0.20 / 0.29,
-// 0.34 / 0.40, 0.39 / 0.40, 0.58 / 0.44.  Builds of their own took another 20 % off the RK4 launches per lane (rk4_rel,
-// 97 x 81 x 113 map, 1000 / 2e4 / 1e5 particles: 0.96 / 0.80 / 1.03 -> 0.77 / 0.63 / 0.80).
-static bool gather_direct(int64_t n) { return n <= 2 * 4 * 256 * 64; }
+// How a launch over n particles gathers: per lane while the chip holds few wavefronts per SIMD (256 CUs of 4), through
+// cells staged in LDS above that.  Staging reads each distinct cell of a wavefront once, but its scan, cell list, load
+// and LDS passes are one serial chain; with few wavefronts to hide it the 12 (FP64: 24) loads per lane return sooner.
+// Per lane over staged, 400 steps through a periodic 64 x 64 x 128 map, bunch of sigma 2 mm / of 0.4 mm (a few cells of
+// the map hold it all, and the RK4 builds keep them staged from step to step):
+//   particles                50000          65536          80000          131072         line, wavefronts per SIMD
+//   FP32-mixed Boris         0.76 / 0.80    0.77 / 0.86    0.91 / 1.07    0.91 / 1.02    two (batches 0.77-0.95 to there)
+//              Vay           0.80 / 0.82    0.81 / 0.88    0.91 / 0.97    0.90 / 0.93    two
+//              RK4           0.56 / 0.73    0.55 / 0.80    0.92 / 1.30    0.94 / 1.15    one
+//              RK4_rel       0.56 / 0.69    0.56 / 0.77    0.87 / 1.19    0.88 / 1.05    one
+//   FP64-fast  Boris         0.84 / 0.92    0.84 / 0.96    1.17 / 1.50    1.18 / 1.39    one
+//              Vay           0.86 / 0.83    0.87 / 0.89    1.05 / 1.26    1.05 / 1.16    one
+//              RK4           1.55 / 2.46    1.75 / 3.00    2.47 / 4.05    2.61 / 4.03    none: 24 loads of 16 bytes a lane
+//              RK4_rel       1.05 / 1.46    1.02 / 1.46    1.68 / 2.39    1.69 / 2.27    and stage, nothing reused
+// Loss builds lie within 0.06 of these, FP64 RK4 ones at 0.87 / 1.23 at 50000.  Each side has builds of its own.
+static bool gather_direct(int64_t n, int precision, bool rk4) {
+    const int64_t one = 4 * 256 * 64;       // particles of one wavefront per SIMD
+    if (precision == PP_PREC_FP64_FAST) return !rk4 && n <= one;
+    return n <= (rk4 ? one : 2 * one);
+}
 
-static void fill_hot_map(const MapDesc& m, const void* coef, uint64_t bytes, int64_t n, HotMap& h) {
+static void fill_hot_map(const MapDesc& m, const void* coef, uint64_t bytes, bool direct, HotMap& h) {
     memset(&h, 0, sizeof(h));
-    h.stage_exec = gather_direct(n) ? 0 : ~0ull;
+    h.stage_exec = direct ? 0 : ~0ull;
     h.coef = coef;
     h.bytes = (uint32_t)bytes;
     h.nc0 = m.nc[0];
@@ -705,7 +717,8 @@ static bool hot_eligible(const pp_push_args* a, const PushParams& p, HotParams& 
     hp.alive = p.alive;
     hp.mesh = p.mesh;
     hp.kick_only = p.kick_only;
-    fill_hot_map(m, coef, bytes, p.n, hp.m);
+    const bool rk4 = a->algorithm == PP_ALG_RK4 || a->algorithm == PP_ALG_RK4_REL;
+    fill_hot_map(m, coef, bytes, gather_direct(p.n, a->precision, rk4), hp.m);
     if (E.rf || B.rf) {
         hp.rf.table = p.rf_table;
         hp.rf.step0 = p.rf_step0;
@@ -1065,7 +1078,8 @@ int pp_push_batched(const pp_batch_args* a, pp_stream s) {
         if (bytes >= 0x7FFFFFFFull) return fail(PP_ERR_UNSUPPORTED, "map %d too large for 32-bit offsets", k);
         if (periodic < 0) periodic = m.periodic;
         else if (periodic != m.periodic) return fail(PP_ERR_UNSUPPORTED, "maps must all be periodic or all not");
-        fill_hot_map(m, coef, bytes, a->n, p.maps[k]);
+        fill_hot_map(m, coef, bytes, gather_direct(a->n, a->precision, a->tile_class != PP_TILES_SINGLE_GATHER),
+                     p.maps[k]);
     }
     p.x = a->x; p.y = a->y; p.z = a->z;
     p.vx = a->vx; p.vy = a->vy; p.vz = a->vz;

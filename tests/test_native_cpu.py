@@ -59,3 +59,8 @@ def test_no_module_allocates_past_the_kept_blocks():
                                   "small_in_one_piece", "threads_by_size"])
 def test_copies(native, case):
     run(native("test_copy"), case)
+
+
+@pytest.mark.parametrize("case", ["gather"])
+def test_routes(native, case):
+    run(native("test_routes"), case)
