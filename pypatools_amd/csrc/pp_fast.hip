@@ -1175,7 +1175,10 @@ DEV void batched_body(const BatchParams& p) {
 template <bool MIXED, bool PERIODIC, int CLASS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBatchWaves<MIXED, CLASS>)))
 k_batched(const BatchParams p) {
-    batched_body<kStageAlways, MIXED, PERIODIC, CLASS>(p);
+    // FP64: the same route by another form, whose register allocation keeps the Boris loop's spills fewer.  400 steps of
+    // 1e6 Boris particles in one bunch / in 32: 5.34 / 7.66 ms as kStageAlways (5.29 / 7.14 at 5 wavefronts), 4.98 /
+    // 6.78 here.
+    batched_body<MIXED ? kStageAlways : kStageByMap, MIXED, PERIODIC, CLASS>(p);
 }
 
 // batches whose launches gather per lane (gather_direct)
