@@ -233,12 +233,13 @@ constexpr int kMomentBlocks = 1024;   // partials per reduction pass
 // spline interpolators (pp_spline.hip)
 namespace pp_splk {
 struct SplineDesc {
-    const double* coef;        // [N0][N1][N2][ncomp] (N = n + 2 pad)
+    const double* coef;        // [ncomp][N0][N1][N2], or [N0][N1][N2][ncomp] (side_by_side); N = n + 2 pad
     const double* axis[3];     // node coordinates, n[a] each
     int64_t n[3];              // nodes per axis (1 for unused axes)
     int64_t N[3];              // coefficient extent per axis
     int64_t ncomp;
     int32_t ndim, order, nearest, rgi, pad;
+    int32_t side_by_side;      // the components of a node next to each other
     double cval;
 };
 }  // namespace pp_splk
