@@ -42,6 +42,11 @@ struct FieldDev {
     MapDesc map;
 };
 
+// Index of node (i, j, k) in a table of at most 2^32 - 1 nodes, ny x nz nodes a plane.
+__host__ __device__ inline uint32_t node_index32(int i, int j, int k, int ny, int nz) {
+    return ((uint32_t)i * (uint32_t)ny + (uint32_t)j) * (uint32_t)nz + (uint32_t)k;
+}
+
 // device grids of a map's components
 struct MapParts {
     const double* comp[6];

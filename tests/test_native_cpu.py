@@ -21,7 +21,7 @@ def native(tmp_path_factory):
             if shutil.which("g++") is None or not os.path.isdir("/opt/rocm/include/hip"):
                 pytest.skip("needs g++ and the HIP headers")
             exe = str(tmp_path_factory.mktemp("native") / name)
-            cmd = ["g++", "-std=c++17", "-O1", "-g", "-x", "c++", "-D__HIP_PLATFORM_AMD__", "-pthread",
+            cmd = ["g++", "-std=c++17", "-O1", "-g", "-ftrapv", "-x", "c++", "-D__HIP_PLATFORM_AMD__", "-pthread",
                    "-I/opt/rocm/include", "-I", os.path.join(ROOT, "include"),
                    "-I", os.path.join(ROOT, "pypatools_amd", "csrc"), os.path.join(HERE, name + ".cpp"), "-o", exe,
                    "-Wl,--unresolved-symbols=ignore-all"]
@@ -61,6 +61,6 @@ def test_copies(native, case):
     run(native("test_copy"), case)
 
 
-@pytest.mark.parametrize("case", ["gather"])
+@pytest.mark.parametrize("case", ["gather", "node_index"])
 def test_routes(native, case):
     run(native("test_routes"), case)
