@@ -21,14 +21,18 @@ static void gather() {
             CHECK(gather_direct(n, w.precision, w.rk4) == (n <= w.limit));
 }
 
-// node indexes of the lean lookup, up to the 2^32 - 1 nodes it admits
+// node indexes of the lean lookup, up to the 2^32 - 1 nodes it admits (-ftrapv: signed overflow aborts)
+__attribute__((noinline)) static uint32_t index_of(const volatile int* q) {
+    return node_index32(q[0], q[1], q[2], q[3], q[4]);
+}
+
 static void node_index() {
-    CHECK(node_index32(0, 0, 0, 7, 9) == 0u && node_index32(1, 2, 3, 7, 9) == 84u);
-    // 46341^2 > 2^31: the last node of a 1 x 65537 x 65535 map is node 2^32 - 2
-    CHECK(node_index32(0, 65536, 65534, 65537, 65535) == 4294967294u);
-    CHECK(node_index32(2, 46340, 30891, 46341, 30892) == 4294698515u);
-    const int n[3] = {1291, 1291, 1291};        // 2151685171 nodes
-    CHECK(node_index32(1290, 1290, 1290, n[1], n[2]) == 2151685170u);
+    const struct {
+        int q[5];
+        uint32_t want;
+    } cases[] = {{{0, 0, 0, 7, 9}, 0u}, {{1, 2, 3, 7, 9}, 84u}, {{0, 65536, 65534, 65537, 65535}, 4294967294u},
+                 {{2, 46340, 30891, 46341, 30892}, 4294698515u}, {{1290, 1290, 1290, 1291, 1291}, 2151685170u}};
+    for (const auto& c : cases) CHECK(index_of(c.q) == c.want);
 }
 
 int main(int argc, char** argv) {
