@@ -552,7 +552,7 @@ int pp_map_create_parts(const double* const* parts, int32_t on_device, int32_t n
         }
         ue = pp_copy::transfer(up, ncomp, false, g_device, s);
     }
-    if (ue == hipSuccess) ue = pp_strict::launch_interleave(src, d, static_cast<double*>(p), s);
+    if (ue == hipSuccess) ue = pp_strict::launch_interleave(src, d, (int64_t)nx * ny, static_cast<double*>(p), s);
     if (ue == hipSuccess && tmp) ue = hipStreamSynchronize(s);
     (void)device_free(tmp);
     if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "map upload"); }

@@ -153,6 +153,12 @@ struct pp_map {
     int device;
 };
 
+// Blocks of 256 threads for a loop over `work` items: at most 2^16 (a launch takes fewer than 2^32 threads an axis).
+inline unsigned loop_blocks(int64_t work) {
+    const int64_t b = (work + 255) / 256;
+    return (unsigned)(b < 1 ? 1 : (b > 65536 ? 65536 : b));
+}
+
 namespace pp_strict {
 hipError_t launch_push(int alg, const PushParams& p, int block, hipStream_t s);
 hipError_t launch_push_sum(int alg, const PushParams& p, const SumParams& t, int block, hipStream_t s);
@@ -187,7 +193,8 @@ hipError_t launch_rows_to_state(const double* rows, const StateView& st, int64_t
 hipError_t launch_state_to_rows(const StateView& st, double* rows, int64_t n, bool ustate, double c2, hipStream_t s);
 hipError_t launch_fill(double* p, double v, int64_t n, hipStream_t s);
 hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s);
-hipError_t launch_interleave(const MapParts& src, const MapDesc& d, double* raw, hipStream_t s);
+// cols z columns of the components into the node table from raw on
+hipError_t launch_interleave(const MapParts& src, const MapDesc& d, int64_t cols, double* raw, hipStream_t s);
 hipError_t launch_build_coef(const MapDesc& d, double* c64, float* c32, hipStream_t s);
 }  // namespace pp_strict
 

@@ -154,16 +154,16 @@ __global__ void __launch_bounds__(256) k_fill(double* p, double v, int64_t n) {
     if (i < n) p[i] = v;
 }
 
-// Node table [node][ncomp] from the components' grids [nx][ny][nz] (a periodic z axis gets node 0 again
+// Node table [node][ncomp] from z columns [cols][nz] of the components' grids (a periodic z axis gets node 0 again
 // as its last).  Writes are contiguous; reads run along ncomp streams.
-__global__ void __launch_bounds__(256) k_interleave(const MapParts src, const MapDesc d, double* __restrict__ raw) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t ngz = d.ng[2], nodes = (int64_t)d.ng[0] * d.ng[1] * ngz;
-    if (t >= nodes * d.ncomp) return;
-    const int64_t node = t / d.ncomp, comp = t - node * d.ncomp;
-    const int64_t col = node / ngz, k = node - col * ngz;
-    const int64_t nz = d.n[2];
-    raw[t] = src.comp[comp][col * nz + (k < nz ? k : 0)];
+__global__ void __launch_bounds__(256) k_interleave(const MapParts src, const MapDesc d, int64_t cols,
+                                                    double* __restrict__ raw) {
+    const int64_t ngz = d.ng[2], nz = d.n[2], n = cols * ngz * d.ncomp;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t node = t / d.ncomp, comp = t - node * d.ncomp;
+        const int64_t col = node / ngz, k = node - col * ngz;
+        raw[t] = src.comp[comp][col * nz + (k < nz ? k : 0)];
+    }
 }
 
 // Per-cell trilinear coefficients of every component from the raw node table.
@@ -543,9 +543,9 @@ hipError_t launch_add_i64(int64_t* p, int64_t v, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_interleave(const MapParts& src, const MapDesc& d, double* raw, hipStream_t s) {
-    const int64_t work = (int64_t)d.ng[0] * d.ng[1] * d.ng[2] * d.ncomp;
-    hipLaunchKernelGGL(k_interleave, dim3(grid_for(work, 256)), dim3(256), 0, s, src, d, raw);
+hipError_t launch_interleave(const MapParts& src, const MapDesc& d, int64_t cols, double* raw, hipStream_t s) {
+    const unsigned g = loop_blocks(cols * d.ng[2] * d.ncomp);
+    hipLaunchKernelGGL(k_interleave, dim3(g), dim3(256), 0, s, src, d, cols, raw);
     return hipGetLastError();
 }
 

@@ -35,11 +35,23 @@ static void node_index() {
     for (const auto& c : cases) CHECK(index_of(c.q) == c.want);
 }
 
+// a looping kernel's grid: enough blocks for few items, fewer than 2^32 threads for any number
+static void grids() {
+    for (int64_t n : {(int64_t)0, (int64_t)1, (int64_t)256, (int64_t)257, (int64_t)1 << 24, ((int64_t)1 << 24) + 1,
+                      (int64_t)720000000 * 6, (int64_t)6 << 31}) {
+        const uint64_t threads = (uint64_t)loop_blocks(n) * 256;
+        CHECK(threads >= 256 && threads < ((uint64_t)1 << 32));
+        CHECK(threads >= (uint64_t)n || threads == ((uint64_t)1 << 24));
+        CHECK(threads < (uint64_t)n + 256 || n == 0);
+    }
+}
+
 int main(int argc, char** argv) {
     CHECK(argc == 2);
     const std::string w = argv[1];
     if (w == "gather") gather();
     else if (w == "node_index") node_index();
+    else if (w == "grids") grids();
     else CHECK(!"unknown case");
     return 0;
 }

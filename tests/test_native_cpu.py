@@ -61,6 +61,6 @@ def test_copies(native, case):
     run(native("test_copy"), case)
 
 
-@pytest.mark.parametrize("case", ["gather", "node_index"])
+@pytest.mark.parametrize("case", ["gather", "node_index", "grids"])
 def test_routes(native, case):
     run(native("test_routes"), case)
