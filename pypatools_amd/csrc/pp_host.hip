@@ -447,6 +447,8 @@ int pp_map_destroy(pp_map* m) {
     return PP_OK;
 }
 
+constexpr size_t kUploadPiece = (size_t)256 << 20;     // values of a map that go up at a time
+
 static int map_alloc(pp_map* m, size_t bytes, void** out) {
     void* p = nullptr;
     hipError_t e = device_alloc(&p, bytes);
@@ -536,23 +538,31 @@ int pp_map_create_parts(const double* const* parts, int32_t on_device, int32_t n
     }
     if ((rc = map_alloc(m, sizeof(double) * nodes * ncomp, &p))) { pp_map_destroy(m); return rc; }
     d.raw = static_cast<const double*>(p);
-    const size_t part = (size_t)nx * ny * nz;
+    const int64_t cols = (int64_t)nx * ny;
+    double* const raw = static_cast<double*>(p);
     MapParts src = {};
     void* tmp = nullptr;
     hipError_t ue = hipSuccess;
     if (on_device) {
         for (int c = 0; c < ncomp; ++c) src.comp[c] = parts[c];
+        ue = pp_strict::launch_interleave(src, d, cols, raw, s);
     } else {
-        ue = device_alloc(&tmp, sizeof(double) * part * ncomp);
+        // in pieces of whole z columns, so that what is needed beside the table stays small
+        const size_t col = sizeof(double) * nz;
+        const int64_t fit = (int64_t)(kUploadPiece / (col * ncomp));
+        const int64_t piece = fit < 1 ? 1 : (fit < cols ? fit : cols);
+        ue = device_alloc(&tmp, col * piece * ncomp);
         if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "hipMalloc (field map)"); }
-        pp_copy::Region up[6];
-        for (int c = 0; c < ncomp; ++c) {
-            src.comp[c] = static_cast<double*>(tmp) + c * part;
-            up[c] = {const_cast<double*>(parts[c]), static_cast<double*>(tmp) + c * part, sizeof(double) * part};
+        for (int c = 0; c < ncomp; ++c) src.comp[c] = static_cast<double*>(tmp) + c * piece * nz;
+        for (int64_t c0 = 0; c0 < cols && ue == hipSuccess; c0 += piece) {
+            const int64_t k = cols - c0 < piece ? cols - c0 : piece;
+            pp_copy::Region up[6];
+            for (int c = 0; c < ncomp; ++c)
+                up[c] = {const_cast<double*>(parts[c] + c0 * nz), const_cast<double*>(src.comp[c]), col * k};
+            ue = pp_copy::transfer(up, ncomp, false, g_device, s);
+            if (ue == hipSuccess) ue = pp_strict::launch_interleave(src, d, k, raw + c0 * d.ng[2] * ncomp, s);
         }
-        ue = pp_copy::transfer(up, ncomp, false, g_device, s);
     }
-    if (ue == hipSuccess) ue = pp_strict::launch_interleave(src, d, (int64_t)nx * ny, static_cast<double*>(p), s);
     if (ue == hipSuccess && tmp) ue = hipStreamSynchronize(s);
     (void)device_free(tmp);
     if (ue != hipSuccess) { pp_map_destroy(m); return hip_fail(ue, "map upload"); }

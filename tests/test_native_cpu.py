@@ -64,3 +64,8 @@ def test_copies(native, case):
 @pytest.mark.parametrize("case", ["gather", "node_index", "grids"])
 def test_routes(native, case):
     run(native("test_routes"), case)
+
+
+@pytest.mark.parametrize("case", ["pieces"])
+def test_maps(native, case):
+    run(native("test_maps"), case)
