@@ -4,8 +4,10 @@
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <deque>
 #include <iterator>
@@ -443,6 +445,7 @@ int pp_event_elapsed_ms(float* ms, pp_event start, pp_event stop) {
 int pp_map_destroy(pp_map* m) {
     if (!m) return PP_OK;
     for (int k = 0; k < m->nalloc; ++k) (void)device_free(m->allocs[k]);
+    for (double* g : m->nodes) free(g);
     delete m;
     return PP_OK;
 }
@@ -509,6 +512,12 @@ int pp_map_create_parts(const double* const* parts, int32_t on_device, int32_t n
             gext[2].push_back(g[2][0] + d.L);
         }
         d.ng[a] = (int32_t)gext[a].size();
+        m->nodes[a] = static_cast<double*>(malloc(sizeof(double) * gext[a].size()));
+        if (!m->nodes[a]) {
+            pp_map_destroy(m);
+            return fail(PP_ERR_NOMEM, "host copy of the map's axes");
+        }
+        memcpy(m->nodes[a], gext[a].data(), sizeof(double) * gext[a].size());
         d.lo[a] = gext[a].front();
         d.hi[a] = gext[a].back();
         d.nc[a] = d.n[a] > 1 ? d.ng[a] - 1 : 1;
@@ -811,6 +820,16 @@ int pp_field_eval(const pp_field* field, int32_t precision, const double* pts, i
     return PP_OK;
 }
 
+// The same nodes on every axis and the same periodicity.
+static bool same_grid(const pp_map& a, const pp_map& b) {
+    if (&a == &b) return true;
+    for (int q = 0; q < 3; ++q)
+        if (a.d.n[q] != b.d.n[q] || a.d.ng[q] != b.d.ng[q] ||
+            !std::equal(a.nodes[q], a.nodes[q] + a.d.ng[q], b.nodes[q]))      // by value: -0 is 0
+            return false;
+    return a.d.periodic == b.d.periodic;
+}
+
 // terms: the fields of pp_push_sum (efield and bfield of the args are then not read), or null
 static int push_impl(const pp_push_args* a, const pp_mesh* mesh, const pp_sum_term* terms, int32_t nterms, pp_stream s) {
     int rc = ensure_init();
@@ -861,12 +880,10 @@ static int push_impl(const pp_push_args* a, const pp_mesh* mesh, const pp_sum_te
             rf = rf || sum.f[k].rf != PP_RF_NONE;
             if (terms[k].flags & PP_SUM_SAME_CELL) {
                 // the shared cell lookup needs a map entry before this one with the same grid
-                const MapDesc* m = nullptr;
+                const pp_map *m = nullptr, *own = terms[k].field.map;
                 for (int32_t q = 0; q < k; ++q)
-                    if (sum.f[q].kind == PP_FIELD_MAP) m = &sum.f[q].map;
-                if (!m || sum.f[k].kind != PP_FIELD_MAP || memcmp(m->n, sum.f[k].map.n, sizeof(m->n)) ||
-                    memcmp(m->lo, sum.f[k].map.lo, sizeof(m->lo)) || memcmp(m->hi, sum.f[k].map.hi, sizeof(m->hi)) ||
-                    m->periodic != sum.f[k].map.periodic)
+                    if (sum.f[q].kind == PP_FIELD_MAP) m = terms[q].field.map;
+                if (!m || sum.f[k].kind != PP_FIELD_MAP || !same_grid(*m, *own))
                     return fail(PP_ERR_INVALID, "term %d does not share the grid of a map before it", k);
             }
         }

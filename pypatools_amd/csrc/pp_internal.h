@@ -147,6 +147,7 @@ struct BatchParams {
 // Host-side map object behind the opaque pp_map handle.
 struct pp_map {
     MapDesc d;
+    double* nodes[3];       // host copy of d.g (ng values each)
     size_t bytes;
     void* allocs[6];
     int nalloc;

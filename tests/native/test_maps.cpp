@@ -18,6 +18,7 @@ hipError_t launch_interleave(const MapParts& src, const MapDesc& d, int64_t cols
                 raw[(c * d.ng[2] + k) * d.ncomp + e] = src.comp[e][c * d.n[2] + (k < d.n[2] ? k : 0)];
     return hipSuccess;
 }
+hipError_t launch_push_sum(int, const PushParams&, const SumParams&, int, hipStream_t) { return hipSuccess; }
 }  // namespace pp_strict
 
 static std::vector<double> axis(int n) {
@@ -50,10 +51,52 @@ static void pieces() {
     }
 }
 
+// A term may share the cell lookup of the map before it only if every node is the same.
+static void same_cell() {
+    std::vector<double> gx = {0, 1, 2.5, 4}, zx = {-0.0, 1, 2.5, 4}, hx = {0, 1.25, 2.5, 4}, one = {0}, v(4, 1.0);
+    const double* parts[3] = {v.data(), v.data(), v.data()};
+    auto make = [&](const std::vector<double>& g) {
+        pp_map* m = nullptr;
+        CHECK(pp_map_create_parts(parts, 0, 3, 1, 1, (int)g.size(), one.data(), one.data(), g.data(), 0.0, PP_MAP_NO_COEF,
+                                  &m) == PP_OK);
+        return m;
+    };
+    pp_map *a = make(gx), *twin = make(zx), *b = make(hx);
+    double state[6] = {};
+    pp_push_args args;
+    memset(&args, 0, sizeof(args));
+    args.algorithm = PP_ALG_BORIS;
+    args.precision = PP_PREC_FP64;
+    args.n = args.nsteps = 1;
+    args.x = state; args.y = state + 1; args.z = state + 2;
+    args.vx = state + 3; args.vy = state + 4; args.vz = state + 5;
+    pp_sum_term t[3];
+    memset(t, 0, sizeof(t));
+    for (auto& q : t) {
+        q.field.kind = PP_FIELD_MAP;
+        q.field.scale1 = q.weight = 1.0;
+    }
+    t[1].flags = PP_SUM_SAME_CELL;
+    t[0].field.map = a;
+    t[1].field.map = twin;
+    CHECK(pp_push_sum(&args, t, 2, nullptr) == PP_OK);
+    t[1].field.map = a;
+    CHECK(pp_push_sum(&args, t, 2, nullptr) == PP_OK);
+    t[1].field.map = b;                                     // same count and ends, another node inside
+    CHECK(pp_push_sum(&args, t, 2, nullptr) == PP_ERR_INVALID);
+    t[1].flags = 0;
+    CHECK(pp_push_sum(&args, t, 2, nullptr) == PP_OK);
+    t[2].field.map = a;                                     // the map before it is b
+    t[2].flags = PP_SUM_SAME_CELL;
+    CHECK(pp_push_sum(&args, t, 3, nullptr) == PP_ERR_INVALID);
+    for (pp_map* m : {a, twin, b}) CHECK(pp_map_destroy(m) == PP_OK);
+}
+
 int main(int argc, char** argv) {
     CHECK(argc == 2 && pp_init(0) == PP_OK);
     const std::string w = argv[1];
     if (w == "pieces") pieces();
+    else if (w == "same_cell") same_cell();
     else CHECK(!"unknown case");
     return 0;
 }
