@@ -366,8 +366,8 @@ __global__ void __launch_bounds__(256) k_push_mixed(const PushParams p) {
     }
 }
 
-// Sums of field terms (SumFE64): every term is evaluated in FP32, weighted and accumulated in FP64, and the
-// sum is rounded to FP32 once, as when the terms come through (n, 3) float64 arrays.
+// Sums of field terms (SumFE64): every term is evaluated in FP32, multiplied by its RF factor, weighted and accumulated in
+// FP64, and the sum is rounded to FP32 once, as when the terms come through (n, 3) float64 arrays.
 struct SumFE32 {
     const PushParams& p;
     const SumParams& t;
@@ -377,7 +377,8 @@ struct SumFE32 {
             const FieldDev& f = t.f[k];
             f3 raw = mkf(0.f, 0.f, 0.f);
             if (f.kind == PP_FIELD_MAP) raw = map_components32(f, x, y, z);
-            const d3 v = tod(finish_term32(f, raw, f.rf != PP_RF_NONE ? (float)rf_factor(p, gs, stage, f.rf) : 1.f));
+            d3 v = tod(finish_term32(f, raw, 1.f));
+            if (f.rf != PP_RF_NONE) v = rf_factor(p, gs, stage, f.rf) * v;
             d3& total = (t.flags[k] & PP_SUM_TO_B) ? b : e;
             total = (t.flags[k] & PP_SUM_PLAIN) ? v : SumFE64::add_weighted(total, t.weight[k], v);
         }
