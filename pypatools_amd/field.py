@@ -497,7 +497,7 @@ def compile_sum(efield, bfield):
             return None
         for g, w, plain in es:
             t = compile_term(g)
-            if t is None:
+            if t is None or (is_time_dependent(g) and rf_source(g) is None):
                 return None
             listed.append((t, w, target | (_lib.SUM_PLAIN if plain else 0), g))
     if len(listed) > _lib.MAX_SUM_TERMS:

@@ -46,3 +46,20 @@ def test_last_velocity_record_of_lost_particles(monkeypatch):
     for batch in (True, False):
         tr.track(np.zeros((2, 3)), np.ones((2, 3)), None, None, 4, 1e-11, 2, batch=batch, electrode_assembly=object())
     assert masks == [None, 4096, None, None]        # record 0 and the last one of either call
+
+
+def test_sums_with_time_dependent_members_of_other_kinds_keep_the_array_route():
+    """A member that declares itself time dependent without being an RFField has no factor for the push kernels; a sum
+    with one is evaluated term by term, as before the sums moved into the step loop."""
+    from pypatools_amd.field import Field, RFField, compile_sum
+    const = {"x": 1.0, "y": 0.0, "z": 2.0}
+    drifting = Field(dim=0, field=const)
+    drifting.time_dependent = True
+    plain, rf = Field(dim=0, field=const), RFField(Field(dim=0, field=const), 1e8)
+    assert compile_sum(plain + plain, plain) is not None
+    assert compile_sum(plain + rf, plain) is not None
+    assert compile_sum(plain + drifting, plain) is None
+    assert compile_sum(rf + drifting, plain) is None
+    assert compile_sum(plain + plain, 2.0 * drifting) is None
+    fp = engine.FieldPair(plain + drifting, plain)
+    assert not fp.fused("boris", "fp64") and not fp.direct
