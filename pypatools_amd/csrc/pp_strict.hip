@@ -256,13 +256,13 @@ struct RowFE64 {
         const MapDesc& m = p.E.map;
         const double rfv = rf != PP_RF_NONE ? rf_factor(p, gs, stage, rf) : 1.0;
         if (m.periodic) z = wrap_periodic(z, m.lo[2], m.L, m.inv_d[2] * m.inv_nz);
-        const AxisGuess qx = guess_axis_3d(m, 0, x), qy = guess_axis_3d(m, 1, y), qz = guess_axis_3d(m, 2, z);
+        const AxisGuess qx = guess_axis(m, 0, x), qy = guess_axis(m, 1, y), qz = guess_axis(m, 2, z);
         StrictCell c;
         c.base = ((int64_t)qx.i * m.ng[1] + qy.i) * m.ng[2] + qz.i;
         double f[8];
         corners(c.base, f);
         if (guess_is_off(m, 0, qx, x) || guess_is_off(m, 1, qy, y) || guess_is_off(m, 2, qz, z)) {
-            c = strict_locate_wrapped(m, x, y, z);
+            c = strict_locate_wrapped<true>(m, x, y, z);
             corners(c.base, f);
         } else {
             const double wx = (x - qx.g0) / (qx.g1 - qx.g0), wy = (y - qy.g0) / (qy.g1 - qy.g0),
