@@ -51,6 +51,28 @@ static void pieces() {
     }
 }
 
+// The layout of small maps, made on the host, is the kernel's: one table on either side of the line, both z forms.
+static void layout() {
+    for (int nz : {5, 6, 60, 70})
+        for (int ncomp : {1, 3, 6})
+            for (int periodic = 0; periodic < 2; ++periodic) {
+                const int n[3] = {4, 5, nz};
+                const int64_t ngz = nz + periodic;
+                const std::vector<double> gx = axis(n[0]), gy = axis(n[1]), gz = axis(nz);
+                std::vector<double> v((size_t)n[0] * n[1] * nz * ncomp);
+                for (size_t k = 0; k < v.size(); ++k) v[k] = (double)k;
+                pp_map* m = nullptr;
+                CHECK(pp_map_create(v.data(), ncomp, n[0], n[1], nz, gx.data(), gy.data(), gz.data(), 0.0,
+                                    PP_MAP_NO_COEF | (periodic ? PP_MAP_PERIODIC_Z : 0), &m) == PP_OK);
+                for (int64_t c = 0; c < (int64_t)n[0] * n[1]; ++c)
+                    for (int64_t k = 0; k < ngz; ++k)
+                        for (int e = 0; e < ncomp; ++e)
+                            CHECK(m->d.raw[(c * ngz + k) * ncomp + e] ==
+                                  v[(size_t)(((int64_t)e * n[0] * n[1] + c) * nz + (k < nz ? k : 0))]);
+                CHECK(pp_map_destroy(m) == PP_OK);
+            }
+}
+
 // A term may share the cell lookup of the map before it only if every node is the same.
 static void same_cell() {
     std::vector<double> gx = {0, 1, 2.5, 4}, zx = {-0.0, 1, 2.5, 4}, hx = {0, 1.25, 2.5, 4}, one = {0}, v(4, 1.0);
@@ -97,6 +119,7 @@ int main(int argc, char** argv) {
     const std::string w = argv[1];
     if (w == "pieces") pieces();
     else if (w == "same_cell") same_cell();
+    else if (w == "layout") layout();
     else CHECK(!"unknown case");
     return 0;
 }
