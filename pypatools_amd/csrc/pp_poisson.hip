@@ -499,8 +499,8 @@ int create(const PoissonDesc& d, pp_poisson** out, char* err, size_t errn) {
 }
 
 static void free_conductors(pp_poisson* P) {
-    for (void* q : {(void*)P->type, (void*)P->coef, (void*)P->vec, (void*)P->part, (void*)P->sc, (void*)P->regular})
-        if (q) (void)hipFree(q);
+    for (void* q : {(void*)P->type, (void*)P->coef, (void*)P->vec, (void*)P->part})
+        if (q) (void)hipFree(q);        // part: with sc and regular
     if (P->host) (void)hipHostFree(P->host);
     P->host = nullptr;
     P->regular = nullptr;
@@ -764,13 +764,13 @@ static int build_operator(pp_poisson* P, char* err, size_t errn) {
                 if (plain) P->box[0] = diag;
             }
     for (int a = 0; a < 3; ++a) P->box[1 + a] = -2.0 / (d.h[a] * (d.h[a] + d.h[a]));
+    // one block: dot partials, scalars, the regular rows' marks
+    const size_t scalars = 2 * pp_poissonk::kDotBlocks + pp_poissonk::kScalars;
     const bool ok = pp_pool::raw_alloc(&P->type, sizeof(int32_t) * N) == hipSuccess &&
                     pp_pool::raw_alloc(&P->coef, sizeof(double) * 7 * N) == hipSuccess &&
                     pp_pool::raw_alloc(&P->vec, sizeof(double) * 9 * N) == hipSuccess &&
-                    pp_pool::raw_alloc(&P->regular, (size_t)N) == hipSuccess &&
-                    hipMemcpy(P->regular, regular.data(), (size_t)N, hipMemcpyHostToDevice) == hipSuccess &&
-                    pp_pool::raw_alloc(&P->part, sizeof(double) * 2 * pp_poissonk::kDotBlocks) == hipSuccess &&
-                    pp_pool::raw_alloc(&P->sc, sizeof(double) * pp_poissonk::kScalars) == hipSuccess &&
+                    pp_pool::raw_alloc(&P->part, sizeof(double) * scalars + (size_t)N) == hipSuccess &&
+                    hipMemcpy(P->part + scalars, regular.data(), (size_t)N, hipMemcpyHostToDevice) == hipSuccess &&
                     hipHostMalloc(reinterpret_cast<void**>(&P->host), sizeof(double) * 8, hipHostMallocDefault) ==
                         hipSuccess &&
                     hipMemcpy(P->type, P->h_type.data(), sizeof(int32_t) * N, hipMemcpyHostToDevice) == hipSuccess &&
@@ -780,6 +780,8 @@ static int build_operator(pp_poisson* P, char* err, size_t errn) {
         snprintf(err, errn, "device allocation for the conductor operator failed");
         return PP_ERR_NOMEM;
     }
+    P->sc = P->part + 2 * pp_poissonk::kDotBlocks;
+    P->regular = reinterpret_cast<uint8_t*>(P->part + scalars);
     return PP_OK;
 }
 
