@@ -233,12 +233,16 @@ class Field(FieldBase):
     # ---- device form ----------------------------------------------------------
     def _grid_source(self):
         """(points, [vx, vy, vz], periodic) of a gridded field, or None."""
-        if self._is_zero or self._dim == 0:
+        comps = self._linear_components()
+        if comps is None:
             return None
+        # c.node_values(), without the calls
+        return comps[0].grid, [c.__dict__["values"] for c in comps], self._periodic_z
+
+    def _linear_components(self):
+        """The components of a field that one device map serves, else None."""
         comps = self._shared_grid_components()
-        if comps is None or any(c.order != 1 for c in comps):
-            return None
-        return comps[0].grid, [c.node_values() for c in comps], self._periodic_z
+        return None if comps is None or any(c.order != 1 for c in comps) else comps
 
     def _shared_grid_components(self):
         """The three HipInterpolator components when they share one grid, else None."""
@@ -317,7 +321,7 @@ class Field(FieldBase):
             for k, c in enumerate("xyz"):
                 t.value[k] = self._scaling * self._field[c]   # field.py:451-453 (times ones(M))
             return t
-        if self._grid_source() is None:
+        if self._linear_components() is None:
             return None
         t.kind = _lib.FIELD_MAP
         if with_map:
