@@ -215,6 +215,15 @@ SIGNATURES = {
 }
 
 
+def _release():
+    _lib.pp_release_staging()
+
+
+def _release_at_exit(pid):
+    if os.getpid() == pid:      # a forked child shares the handles, but may not call the HIP runtime
+        _release()
+
+
 def lib():
     """Load libpypat_hip.so once; raise ImportError if it has not been built."""
     global _lib
@@ -230,7 +239,7 @@ def lib():
                 fn = getattr(h, name)
                 fn.restype = res
                 fn.argtypes = args
-            atexit.register(h.pp_release_staging)
+            atexit.register(_release_at_exit, os.getpid())
             _lib = h
     return _lib
 
