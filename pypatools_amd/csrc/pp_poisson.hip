@@ -807,7 +807,7 @@ void stats(const pp_poisson* P, int32_t* iterations, double* residual) {
 // BiCGSTAB with right preconditioning, for A phi = rho / eps0 with the Shortley-Weller rows.  The
 // preconditioner is the box solve with its result set to 0 on conductor nodes, so every iterate is 0 there
 // (and the residual too, since conductor rows are diagonal with b = 0); it starts from that preconditioned b.
-// An iteration is 18 launches (it was 32), the dot products inside the passes that have their vectors at hand.  The
+// An iteration is 20 launches (the first 19; it was 32), the dot products inside the passes that have their vectors at hand.  The
 // host waits for the residual of one iteration while the next one is enqueued already: that one changes nothing once
 // the device has found the tolerance reached.
 static hipError_t solve_conductors(const pp_poisson* P, const double* rho, double* phi, hipStream_t s) {

@@ -414,7 +414,10 @@ static inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + b
     }
 
 // The general build of terms that share no map: with all corners of a lookup in flight it holds two wavefronts per
-// SIMD, plane by plane three.
+// SIMD, plane by plane three or four.  Over the former build (all corners, the fused map's code in it too), 100 Boris
+// steps through an E map and a constant B / a B map of its own: 0.96 / 1.01 at 1e4 particles, 0.96 / 1.01 at 1e5 (all
+// corners), 0.88 / 0.87 at 2e5, 0.83 / 0.82 at 1e6 (plane by plane; 2.56 -> 2.13 and 3.92 -> 3.22 ms); RK4, which
+// holds two wavefronts either way, keeps all corners (0.90 / 0.92 at 1e6).
 constexpr int64_t kGeneralAll = 2 * 4 * 256 * 64;
 
 template <int ALG>
