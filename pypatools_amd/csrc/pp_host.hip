@@ -495,6 +495,8 @@ int pp_map_create_parts(const double* const* parts, int32_t on_device, int32_t n
     if ((int64_t)nx * ny * nz > (int64_t)1 << 31) return fail(PP_ERR_INVALID, "map too large");
     for (int c = 0; c < ncomp; ++c)
         if (!parts[c]) return fail(PP_ERR_INVALID, "component %d is null", c);
+    if (!(flags & PP_MAP_NO_COEF) && (flags & PP_MAP_NO_FP64) && (flags & PP_MAP_NO_FP32))
+        return fail(PP_ERR_INVALID, "PP_MAP_NO_FP64 with PP_MAP_NO_FP32 leaves no coefficient table: use PP_MAP_NO_COEF");
 
     pp_map* m = new pp_map();
     memset(m, 0, sizeof(*m));
@@ -589,8 +591,6 @@ int pp_map_create_parts(const double* const* parts, int32_t on_device, int32_t n
     const int64_t ncell = (int64_t)d.nc[0] * d.nc[1] * d.nc[2];
     double* c64 = nullptr;
     float* c32 = nullptr;
-    if (!(flags & PP_MAP_NO_COEF) && (flags & PP_MAP_NO_FP64) && (flags & PP_MAP_NO_FP32))
-        return fail(PP_ERR_INVALID, "PP_MAP_NO_FP64 with PP_MAP_NO_FP32 leaves no coefficient table: use PP_MAP_NO_COEF");
     if (!(flags & PP_MAP_NO_COEF)) {
         if (!(flags & PP_MAP_NO_FP64)) {
             if ((rc = map_alloc(m, sizeof(double) * ncell * ncomp * 8, &p))) { pp_map_destroy(m); return rc; }

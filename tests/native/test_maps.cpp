@@ -114,12 +114,24 @@ static void same_cell() {
     for (pp_map* m : {a, twin, b}) CHECK(pp_map_destroy(m) == PP_OK);
 }
 
+// A map refused for its flags leaves nothing behind.
+static void refused() {
+    const std::vector<double> g = axis(5);
+    std::vector<double> v(125 * 3);
+    const double* parts[3] = {v.data(), v.data() + 125, v.data() + 250};
+    pp_map* m = nullptr;
+    CHECK(pp_map_create_parts(parts, 0, 3, 5, 5, 5, g.data(), g.data(), g.data(), 0.0, PP_MAP_NO_FP64 | PP_MAP_NO_FP32,
+                              &m) == PP_ERR_INVALID);
+    CHECK(m == nullptr && pp_release_staging() == PP_OK && used == 0);
+}
+
 int main(int argc, char** argv) {
     CHECK(argc == 2 && pp_init(0) == PP_OK);
     const std::string w = argv[1];
     if (w == "pieces") pieces();
     else if (w == "same_cell") same_cell();
     else if (w == "layout") layout();
+    else if (w == "refused") refused();
     else CHECK(!"unknown case");
     return 0;
 }

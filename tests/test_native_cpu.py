@@ -66,6 +66,6 @@ def test_routes(native, case):
     run(native("test_routes"), case)
 
 
-@pytest.mark.parametrize("case", ["pieces", "same_cell", "layout"])
+@pytest.mark.parametrize("case", ["pieces", "same_cell", "layout", "refused"])
 def test_maps(native, case):
     run(native("test_maps"), case)
